@@ -42,6 +42,10 @@ constexpr int kCapMax = 1016;   // second-pass capacity limit (FP64 LDS: (4 cap 
 // up to kSmallBlock one wavefront, up to kHugeBlock kMidThreads, above kHugeThreads
 constexpr int64_t kSmallBlock[2] = {384, 384};
 constexpr int64_t kHugeBlock[2] = {(int64_t)1 << 40, 2048};
+// bounds on the m + n above which a block takes the ACA over several
+// workgroups (wide_bound), and the resident 256-thread workgroups it counts
+constexpr int64_t kWideMin = 1024, kWideMax = 4096, kWideShare = 800;
+constexpr int kWideCap = 96;    // their first-pass capacity while memory allows (first_caps)
 constexpr double kTiny = 10.0 * 2.220446049250313e-16;  // global.h:53
 
 struct Tile {
@@ -1126,50 +1130,55 @@ template <int NT, class C> constexpr int kAcaWaves = 1;
 template <> constexpr int kAcaWaves<64, bem_c32> = 4;
 template <> constexpr int kAcaWaves<128, bem_c32> = 4;
 
-// one listed item of a batched launch (nf > 0; the single operator's
-// launches take aca_block directly): block b of frequency f with that
-// frequency's wavenumber, coupling, table and storage
-template <bool EXTRA, int NT, class C, bool PLANE>
-__device__ __forceinline__ void aca_item(const AcaArgs& a, int item, char* dyn, ArgMax* sred)
+// the arguments of one list entry: MODE 0 the block itself, 1 a (frequency,
+// block) item, 3 a (context, block) item
+template <int MODE>
+__device__ __forceinline__ int aca_resolve(AcaArgs& ai, const AcaArgs& a, int item)
 {
-    const int f = (int)(item / a.nbk);
-    const int b = (int)(item - (int64_t)f * a.nbk);
-    AcaArgs ai = a;
-    const double k = a.kf[f];
-    const bem_c64 cc = a.ccf[f];
-    ai.F.k = k;
-    ai.F.cc = cc;
-    ai.F32.k = (float)k;
-    ai.F32.krev = k / (2.0 * BEM_PI);
-    ai.F32.cc = c32((float)cc.re, (float)cc.im);
-    ai.sing = a.singf[f];
-    ai.U = a.Uf[f];
-    ai.V = a.Vf[f];
-    ai.A = a.Af[f];
-    ai.rank_out = a.rank_out + (int64_t)f * a.nbk;
-    ai.flag_out = a.flag_out + (int64_t)f * a.nbk;
-    ai.evals_out = a.evals_out + (int64_t)f * a.nbk;
-    aca_block<EXTRA, NT, C, PLANE>(ai, b, dyn, sred);
+    if constexpr (MODE == 0) {
+        return item;
+    } else if constexpr (MODE == 1) {
+        const int f = (int)(item / a.nbk);
+        const double k = a.kf[f];
+        const bem_c64 cc = a.ccf[f];
+        ai.F.k = k;
+        ai.F.cc = cc;
+        ai.F32.k = (float)k;
+        ai.F32.krev = k / (2.0 * BEM_PI);
+        ai.F32.cc = c32((float)cc.re, (float)cc.im);
+        ai.sing = a.singf[f];
+        ai.U = a.Uf[f];
+        ai.V = a.Vf[f];
+        ai.A = a.Af[f];
+        ai.rank_out = a.rank_out + (int64_t)f * a.nbk;
+        ai.flag_out = a.flag_out + (int64_t)f * a.nbk;
+        ai.evals_out = a.evals_out + (int64_t)f * a.nbk;
+        return (int)(item - (int64_t)f * a.nbk);
+    } else {
+        const MeshJob& J = a.jobs[item >> kJobShift];
+        ai.M = J.M;
+        ai.F = J.F;
+        ai.F32 = J.F32;
+        ai.row0 = J.row0; ai.rows = J.rows; ai.col0 = J.col0; ai.cols = J.cols;
+        ai.uoff = J.uoff; ai.voff = J.voff; ai.aoff = J.aoff; ai.cap = J.cap;
+        ai.U = J.U; ai.V = J.V; ai.A = J.A;
+        ai.rank_out = J.rank_out; ai.flag_out = J.flag_out; ai.evals_out = J.evals_out;
+        ai.piv_off = J.piv_off; ai.piv = J.piv;
+        ai.sing = J.sing; ai.nnz = J.nnz;
+        ai.bnear = J.bnear;
+        ai.nf = 0;
+        return item & kJobMask;
+    }
 }
 
-// one listed (context, block) item of a multi-mesh launch
-template <bool EXTRA, int NT, class C, bool PLANE>
-__device__ __forceinline__ void aca_job(const AcaArgs& a, int item, char* dyn, ArgMax* sred)
+// one list entry of a batched or multi-mesh launch (the single operator's
+// launches take aca_block directly)
+template <bool EXTRA, int NT, class C, bool PLANE, int MODE>
+__device__ __forceinline__ void aca_item(const AcaArgs& a, int item, char* dyn, ArgMax* sred)
 {
-    const MeshJob& J = a.jobs[item >> kJobShift];
     AcaArgs ai = a;
-    ai.M = J.M;
-    ai.F = J.F;
-    ai.F32 = J.F32;
-    ai.row0 = J.row0; ai.rows = J.rows; ai.col0 = J.col0; ai.cols = J.cols;
-    ai.uoff = J.uoff; ai.voff = J.voff; ai.aoff = J.aoff; ai.cap = J.cap;
-    ai.U = J.U; ai.V = J.V; ai.A = J.A;
-    ai.rank_out = J.rank_out; ai.flag_out = J.flag_out; ai.evals_out = J.evals_out;
-    ai.piv_off = J.piv_off; ai.piv = J.piv;
-    ai.sing = J.sing; ai.nnz = J.nnz;
-    ai.bnear = J.bnear;
-    ai.nf = 0;
-    aca_block<EXTRA, NT, C, PLANE>(ai, item & kJobMask, dyn, sred);
+    const int b = aca_resolve<MODE>(ai, a, item);
+    aca_block<EXTRA, NT, C, PLANE>(ai, b, dyn, sred);
 }
 
 // MODE 0: one workgroup per listed block of the single operator; 1: one per
@@ -1187,11 +1196,11 @@ __global__ __launch_bounds__(NT, (PLANE && kAcaWaves<NT, C> > 3 ? 3 : kAcaWaves<
         return;
     }
     if constexpr (MODE == 1) {
-        aca_item<EXTRA, NT, C, PLANE>(a, a.blist[blockIdx.x], dyn, sred);
+        aca_item<EXTRA, NT, C, PLANE, 1>(a, a.blist[blockIdx.x], dyn, sred);
         return;
     }
     if constexpr (MODE == 3) {
-        aca_job<EXTRA, NT, C, PLANE>(a, a.blist[blockIdx.x], dyn, sred);
+        aca_item<EXTRA, NT, C, PLANE, 3>(a, a.blist[blockIdx.x], dyn, sred);
         return;
     }
     __shared__ int s_pos;
@@ -1201,10 +1210,405 @@ __global__ __launch_bounds__(NT, (PLANE && kAcaWaves<NT, C> > 3 ? 3 : kAcaWaves<
         const int pos = s_pos;
         __syncthreads();
         if (pos >= a.nitems) break;
-        if constexpr (MODE == 4) aca_job<EXTRA, NT, C, PLANE>(a, a.blist[pos], dyn, sred);
-        else aca_item<EXTRA, NT, C, PLANE>(a, a.blist[pos], dyn, sred);
+        aca_item<EXTRA, NT, C, PLANE, MODE == 4 ? 3 : 1>(a, a.blist[pos], dyn, sred);
         __syncthreads();
     }
+}
+
+// ---- ACA of large blocks over several workgroups.  One workgroup per block
+// makes a large block's pivot chain the longest path of an assembly: every
+// step evaluates (m + n) / NT entries per thread one after the other while
+// the rest of the chip is idle (the 76440-triangle capsule's ten largest
+// blocks, m + n up to 39000: 287 ms per pass, and a second pass for those
+// above the first rank capacity).  Here a step is two launches over all large
+// blocks at once, a workgroup per kWideChunk entries of a row (k_wide_row)
+// or column (k_wide_col): the entries, the chunk's part of the argmax and of
+// the norm-estimate dot products.  The next launch's workgroups combine the
+// parts, each for itself and in one fixed order, and take the decisions of
+// aca_block (the same pivots, factors, ranks and counts); the kernel
+// boundary is the only barrier.  States are double buffered: a launch reads
+// one copy and its first workgroup of the block writes the other.
+constexpr int kWideChunk = 256;   // entries (and threads) per workgroup
+enum WidePhase : int32_t {
+    kWideStart,      // nothing computed yet
+    kWideProbe,      // EXTRA: the inner loop ended, the next listed pivot comes
+    kWideFirstCol,   // column j to be computed as a first column
+    kWideFirst,      // a first column is in U[r]
+    kWideRow,        // row i is in V[r]
+    kWideStep,       // row and column r are in place, the norm update is due
+    kWideDone
+};
+struct WideState {
+    int64_t i, j, p, ev;   // row and column pivot, position in the pivot list, evaluated entries
+    bem_c64 S;             // norm estimate
+    int32_t r, flag, phase, pad;
+};
+struct WideBlk {
+    int32_t item;          // list entry of the launch mode (block, frequency item or job item)
+    int32_t nmc, nnc;      // chunks of a column and of a row
+    int32_t cap;
+    int64_t am_col, am_row;   // the chunks' argmax parts
+    int64_t d_col, d_row[2];  // the chunks' dot-product parts, cap + 1 each (rows: of even and odd steps)
+};
+struct WideTask { int32_t w, chunk; };
+struct WideArgs {
+    const WideBlk* blk;
+    const WideTask* task;
+    const WideState* in;
+    WideState* out;
+    ArgMax* am;
+    bem_c64* dots;
+    int32_t* active;       // host memory: set when a block still works
+    int odd;               // step parity: a row launch writes d_row[odd] and reads the other
+};
+
+// the best of `cnt` argmax parts (every thread gets it); better() keeps the
+// first index on ties, so the order of combination does not matter
+__device__ __forceinline__ ArgMax wide_best(const ArgMax* part, int cnt, ArgMax* sred)
+{
+    ArgMax a{-1.0, (int64_t)1 << 62};
+    for (int q = threadIdx.x; q < cnt; q += kWideChunk) a = better(a, part[q]);
+    for (int s = 32; s > 0; s >>= 1) {
+        ArgMax o;
+        o.v = __shfl_xor(a.v, s, 64);
+        o.i = __shfl_xor(a.i, s, 64);
+        a = better(a, o);
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = a;
+    __syncthreads();
+    ArgMax r = sred[0];
+    for (int w = 1; w < kWideChunk / 64; w++) r = better(r, sred[w]);
+    return r;
+}
+
+// One chunk of a residual row (ROW: entries (gi, c0 + t), basis V of stride
+// n) or column: the entries minus the cross approximation with the weights
+// sw[0 .. r), into dst, the chunk's argmax (index excl counts as 0) into *am
+// and, with DOTS, |v|^2 and v^H W_l (l < r) into dots[0 .. r].
+template <bool ROW, class C, bool PLANE, bool FIELD>
+__device__ __forceinline__ void wide_line(const AcaArgs& a, int64_t r0, int64_t c0, int64_t len, int r, int64_t fixed,
+                                          const C* W, C* dst, const C* sw, bool nearb, int64_t t0, int64_t excl,
+                                          bool want_dots, C* sv, ArgMax* sred, ArgMax* am, bem_c64* dots)
+{
+    const int tid = threadIdx.x;
+    const int64_t t = t0 + tid;
+    const int cnt = (int)(len - t0 < kWideChunk ? len - t0 : kWideChunk);
+    const int64_t gf = (ROW ? r0 : c0) + fixed;
+    C v = cx_zero<C>();
+    if (tid < cnt) {
+        const int64_t gi = ROW ? gf : r0 + t, gj = ROW ? c0 + t : gf;
+        C e;
+        bool have = true;
+        if constexpr (FIELD) {
+            e = from64<C>(field_entry(a, gi, gj));
+        } else {
+            have = regular_entry<PLANE>(a, gi, gj, &e, nearb);
+            if (!have) e = singular_entry<C>(a, gi, gi == gj ? -1 : near_find(a.M, gi, (int32_t)gj));
+        }
+        v = cx_sub(e, cross_sum<ROW>(sw, W, len, t, r));
+        dst[t] = v;
+    }
+    sv[tid] = v;
+    ArgMax m{-1.0, (int64_t)1 << 62};
+    if (tid < cnt) {
+        const double x = t == excl ? 0.0 : cx_abs2(v);
+        if (x > m.v) { m.v = x; m.i = t; }
+    }
+    for (int s = 32; s > 0; s >>= 1) {
+        ArgMax o;
+        o.v = __shfl_xor(m.v, s, 64);
+        o.i = __shfl_xor(m.i, s, 64);
+        m = better(m, o);
+    }
+    if ((tid & 63) == 0) sred[tid >> 6] = m;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kWideChunk / 64; w++) m = better(m, sred[w]);
+        *am = m;
+    }
+    if (!want_dots) return;
+    const int lane = tid & 63;
+    for (int kb = (tid >> 6) * kDotGroup; kb <= r; kb += (kWideChunk / 64) * kDotGroup) {
+        const C* src[kDotGroup];
+        bem_c64 acc[kDotGroup];
+#pragma unroll
+        for (int g = 0; g < kDotGroup; g++) {
+            const int k = kb + g;
+            src[g] = (k >= 1 && k <= r) ? W + (int64_t)(k - 1) * len + t0 : dst + t0;
+            acc[g] = c64(0, 0);
+        }
+        double nrm = 0.0;
+#pragma unroll
+        for (int q = 0; q < kWideChunk / 64; q++) {
+            const int u = lane + 64 * q;
+            if (u >= cnt) break;
+            const bem_c64 cv = ld64(&sv[u]);
+            C wv[kDotGroup];
+#pragma unroll
+            for (int g = 0; g < kDotGroup; g++) wv[g] = ldg(src[g] + u);
+            nrm = nrm + c64_abs2(cv);
+#pragma unroll
+            for (int g = 0; g < kDotGroup; g++) acc[g] = c64_fma(c64_conj(cv), ld64(&wv[g]), acc[g]);
+        }
+        if (kb == 0) acc[0] = c64(nrm, 0.0);
+        double x[2 * kDotGroup];
+#pragma unroll
+        for (int g = 0; g < kDotGroup; g++) {
+            x[2 * g] = acc[g].re;
+            x[2 * g + 1] = acc[g].im;
+        }
+        const double tot = wave_sum_spread<2 * kDotGroup>(x, lane);
+        constexpr int kStride = 64 / (2 * kDotGroup);
+        if ((lane & (kStride - 1)) == 0) {
+            const int q = lane / kStride, k = kb + (q >> 1);
+            if (k <= r) ((double*)(dots + k))[q & 1] = tot;
+        }
+    }
+}
+
+// totals of the chunks' dot-product parts (nch chunks of stride cap + 1) in
+// chunk order, r + 1 values into out
+__device__ __forceinline__ void wide_totals(const bem_c64* part, int nch, int cap, int r, bem_c64* out)
+{
+    for (int k = threadIdx.x; k < 2 * (r + 1); k += kWideChunk) {
+        const double* p = (const double*)part + k;
+        const int64_t ld = 2 * (int64_t)(cap + 1);
+        double s = 0.0;
+        int q = 0;
+        for (; q + 8 <= nch; q += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = p[(q + u) * ld];
+#pragma unroll
+            for (int u = 0; u < 8; u++) s = s + v[u];
+        }
+        for (; q < nch; q++) s = s + p[q * ld];
+        ((double*)out)[k] = s;
+    }
+}
+
+// The decisions between a step's column and the next row (norm update,
+// stopping rules, the next row pivot or, EXTRA, the next listed pivot), then
+// a chunk of that row.  Dynamic LDS: sw[cap] (C), then 2 (cap + 1) totals.
+template <bool EXTRA, class C, bool PLANE, int MODE, bool FIELD>
+__global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
+{
+    extern __shared__ __attribute__((aligned(16))) char dyn[];
+    __shared__ ArgMax sred[kWideChunk / 64];
+    __shared__ C sv[kWideChunk];
+    const WideTask T = w.task[blockIdx.x];
+    const WideBlk B = w.blk[T.w];
+    WideState s = w.in[T.w];
+    const int tid = threadIdx.x;
+    const bool lead = T.chunk == 0 && tid == 0;
+    if (s.phase == kWideDone) {
+        if (lead) w.out[T.w] = s;
+        return;
+    }
+    AcaArgs a = a0;
+    const int b = aca_resolve<MODE>(a, a0, B.item);
+    const int64_t m = a.rows[b], n = a.cols[b], r0 = a.row0[b], c0 = a.col0[b];
+    const int cap = B.cap;
+    const bool nearb = !FIELD && (!a.bnear || a.bnear[b] != 0);
+    int64_t maxRank = m < n ? m : n;
+    if (a.maxrank > 0 && a.maxrank < maxRank) maxRank = a.maxrank;
+    const C* U = (const C*)a.U + a.uoff[b];
+    C* V = (C*)a.V + a.voff[b];
+    const C* A = (const C*)a.A + a.aoff[b];
+    C* sw = (C*)dyn;
+    bem_c64* tot = (bem_c64*)(dyn + (((size_t)cap * sizeof(C) + 15) & ~(size_t)15));
+    const double tiny2 = kTiny * kTiny, tol2 = a.tol * a.tol;
+    bool probe = false;
+    if (s.phase == kWideStep) {
+        const int r = s.r;
+        bem_c64 *dc = tot, *dr = tot + cap + 1;
+        wide_totals(w.dots + B.d_col, B.nmc, cap, r, dc);
+        wide_totals(w.dots + (w.odd ? B.d_row[0] : B.d_row[1]), B.nnc, cap, r, dr);
+        __syncthreads();
+        // aca_update_norm: the terms in parallel, added in rank order
+        const C alpha = ldg(A + r);
+        const double gain = (cx_abs2(alpha) * dr[0].re) * dc[0].re;
+        const bem_c64 ca2 = c64_scale(c64_conj(ld64(&alpha)), 2.0);
+        for (int l = tid; l < r; l += kWideChunk)
+            dr[1 + l] = c64_mul(c64_mul(c64_mul(ca2, ldg64(A + l)), dc[1 + l]), dr[1 + l]);
+        __syncthreads();
+        const bem_c64 oldS = s.S;
+        s.S.re = s.S.re + gain;
+        for (int l = 0; l < r; l++) s.S = c64_add(s.S, dr[1 + l]);
+        s.r++;
+        if (!isfinite(gain)) {
+            s.flag = 2;
+            s.phase = kWideDone;
+        } else if (a.tol > 0 && gain < tol2 * s.S.re) {
+            if (EXTRA) {
+                if (gain < 0.1 * (tol2 * s.S.re)) { s.r--; s.S = oldS; }
+                probe = true;
+                s.p++;
+            } else {
+                s.phase = kWideDone;
+            }
+        }
+    } else if (s.phase == kWideProbe) {
+        probe = true;
+        s.p++;
+    } else if (s.phase == kWideStart) {
+        if (EXTRA) {
+            probe = true;
+            s.p = a.piv_off[b];
+        } else {
+            s.j = bem_rand_bounded(a.seed, 0, (uint64_t)b, 0, n);
+            s.phase = kWideFirstCol;
+        }
+    }
+    if (s.phase != kWideDone && s.phase != kWideFirstCol && !probe) {
+        // the row pivot: the last column's largest entry (the previous row
+        // pivot was counted as 0 by its chunks)
+        if (s.r >= maxRank) {
+            if (EXTRA) { probe = true; s.p++; }
+            else s.phase = kWideDone;
+        } else if (s.r >= cap) {
+            s.flag = 1;
+            s.phase = kWideDone;
+        } else {
+            const ArgMax am = wide_best(w.am + B.am_col, B.nmc, sred);
+            const C* wcol = U + (int64_t)(s.phase == kWideFirst && EXTRA ? s.r : s.r >= 1 ? s.r - 1 : 0) * m;
+            if (am.i >= m) {   // no finite entry in the column
+                s.flag = 2;
+                s.phase = kWideDone;
+            } else {
+                s.i = am.i;
+                const double x = EXTRA ? cx_abs2(ldg(wcol + am.i)) : am.v;
+                if (x <= tiny2 && s.r >= 1) {
+                    if (EXTRA) { probe = true; s.p++; }
+                    else s.phase = kWideDone;
+                } else {
+                    s.phase = kWideRow;
+                }
+            }
+        }
+    }
+    if (EXTRA && probe) {
+        // the listed pivots from s.p on, 64 at a time (one per lane, every
+        // wavefront the same): the first whose entry the approximation misses
+        const int64_t p1 = a.piv_off[b + 1];
+        const int lane = tid & 63, r = s.r;
+        s.phase = kWideDone;
+        while (s.r < maxRank && s.p < p1) {
+            const int64_t p = s.p + lane;
+            int64_t pj = 0;
+            bool take = false;
+            if (p < p1) {
+                const int64_t pi = a.piv[2 * p];
+                pj = a.piv[2 * p + 1];
+                const C pe = entry_any<PLANE, C, FIELD>(a, r0 + pi, c0 + pj, nearb);
+                if (!(cx_abs2(pe) < tiny2)) {
+                    C approx = cx_zero<C>();
+#pragma unroll 4
+                    for (int l = 0; l < r; l++)
+                        approx = cx_add(approx, cx_mul(cx_mul(ldg(U + (int64_t)l * m + pi), ldg(A + l)),
+                                                       ldg(V + (int64_t)l * n + pj)));
+                    take = !(cx_abs2(cx_sub(pe, approx)) < tol2 * cx_abs2(pe));
+                }
+            }
+            const uint64_t mask = __ballot(take);
+            if (mask) {
+                const int f = __ffsll((unsigned long long)mask) - 1;
+                s.ev += f + 1;
+                s.p += f;
+                s.j = __shfl(pj, f, 64);
+                s.phase = kWideFirstCol;
+                if (s.r >= cap) {
+                    s.flag = 1;
+                    s.phase = kWideDone;
+                }
+                break;
+            }
+            const int64_t left = p1 - s.p < 64 ? p1 - s.p : 64;
+            s.ev += left;
+            s.p += left;
+        }
+    }
+    if (s.phase == kWideRow) s.ev += n;
+    if (lead) {
+        w.out[T.w] = s;
+        if (s.phase == kWideDone) {
+            a.rank_out[b] = s.r;
+            a.flag_out[b] = s.flag;
+            a.evals_out[b] = s.ev;
+        } else {
+            *w.active = 1;
+        }
+    }
+    if (s.phase != kWideRow) return;
+    __syncthreads();
+    for (int l = tid; l < s.r; l += kWideChunk) sw[l] = cx_mul(ldg(U + (int64_t)l * m + s.i), ldg(A + l));
+    __syncthreads();
+    wide_line<true, C, PLANE, FIELD>(a, r0, c0, n, s.r, s.i, V, V + (int64_t)s.r * n, sw, nearb,
+                                     (int64_t)T.chunk * kWideChunk, -1, true, sv, sred, w.am + B.am_row + T.chunk,
+                                     w.dots + (w.odd ? B.d_row[1] : B.d_row[0]) + (int64_t)T.chunk * (cap + 1));
+}
+
+// The column pivot from the row's parts, then a chunk of that column (or of
+// a first column).  Dynamic LDS as k_wide_row.
+template <bool EXTRA, class C, bool PLANE, int MODE, bool FIELD>
+__global__ __launch_bounds__(kWideChunk) void k_wide_col(AcaArgs a0, WideArgs w)
+{
+    extern __shared__ __attribute__((aligned(16))) char dyn[];
+    __shared__ ArgMax sred[kWideChunk / 64];
+    __shared__ C sv[kWideChunk];
+    const WideTask T = w.task[blockIdx.x];
+    const WideBlk B = w.blk[T.w];
+    WideState s = w.in[T.w];
+    const int tid = threadIdx.x;
+    const bool lead = T.chunk == 0 && tid == 0;
+    if (s.phase == kWideDone) {
+        if (lead) w.out[T.w] = s;
+        return;
+    }
+    AcaArgs a = a0;
+    const int b = aca_resolve<MODE>(a, a0, B.item);
+    const int64_t m = a.rows[b], n = a.cols[b], r0 = a.row0[b], c0 = a.col0[b];
+    const int cap = B.cap;
+    const bool nearb = !FIELD && (!a.bnear || a.bnear[b] != 0);
+    C* U = (C*)a.U + a.uoff[b];
+    const C* V = (const C*)a.V + a.voff[b];
+    C* A = (C*)a.A + a.aoff[b];
+    C* sw = (C*)dyn;
+    const double tiny2 = kTiny * kTiny;
+    const int r = s.r;
+    const bool step = s.phase == kWideRow;
+    if (step) {
+        const ArgMax ar = wide_best(w.am + B.am_row, B.nnc, sred);
+        if (ar.i >= n) {   // no finite entry in the row
+            s.flag = 2;
+            s.phase = kWideDone;
+        } else if (ar.v <= tiny2 && r >= 1) {
+            s.phase = EXTRA ? kWideProbe : kWideDone;
+        } else {
+            s.j = ar.i;
+            s.phase = kWideStep;
+            if (lead) A[r] = cx_inv(ldg(V + (int64_t)r * n + s.j));
+        }
+    } else {
+        s.phase = kWideFirst;
+    }
+    const bool work = s.phase == kWideStep || s.phase == kWideFirst;
+    if (work) s.ev += m;
+    if (lead) {
+        w.out[T.w] = s;
+        if (s.phase == kWideDone) {
+            a.rank_out[b] = r;
+            a.flag_out[b] = s.flag;
+            a.evals_out[b] = s.ev;
+        }
+    }
+    if (!work) return;
+    for (int l = tid; l < r; l += kWideChunk) sw[l] = cx_mul(ldg(A + l), ldg(V + (int64_t)l * n + s.j));
+    __syncthreads();
+    wide_line<false, C, PLANE, FIELD>(a, r0, c0, m, r, s.j, U, U + (int64_t)r * m, sw, nearb,
+                                      (int64_t)T.chunk * kWideChunk, step ? s.i : -1, step, sv, sred,
+                                      w.am + B.am_col + T.chunk, w.dots + B.d_col + (int64_t)T.chunk * (cap + 1));
 }
 
 // copy the first rank columns/rows of the ACA scratch into the packed
@@ -2853,6 +3257,10 @@ struct bem_ctx {
     int64_t cls_small[2] = {kSmallBlock[0], kSmallBlock[1]};
     int64_t cls_huge[2] = {kHugeBlock[0], kHugeBlock[1]};
     bool aca_queue = false;
+    // wide ACA: "a block still works" flags of the last two bursts (pinned
+    // host memory; [2] takes the other steps' stores) and their events
+    int32_t* wide_active = nullptr;
+    hipEvent_t wide_ev[2] = {nullptr, nullptr};
     bool capturing = false;   // Timer records no events while a graph is captured
     hipEvent_t gm_ev[2] = {nullptr, nullptr};
 };
@@ -3242,6 +3650,9 @@ int bem_create(bem_ctx_t* out, int device)
         hipEventCreateWithFlags(&c->ev_join[1], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->stage_done, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->gm_ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->wide_ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->wide_ev[1], hipEventDisableTiming) != hipSuccess ||
+        hipHostMalloc((void**)&c->wide_active, 4 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->gm_ev[1], hipEventDisableTiming) != hipSuccess ||
         hipHostMalloc((void**)&c->gm_res, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&c->gm_resq, 2 * kArnMax * sizeof(double), hipHostMallocDefault) != hipSuccess ||
@@ -3276,8 +3687,10 @@ int bem_destroy(bem_ctx_t c)
     (void)hipEventDestroy(c->ev_fork);
     for (hipEvent_t e : c->ev_join) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->gm_ev) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->wide_ev) (void)hipEventDestroy(e);
     (void)hipEventDestroy(c->stage_done);
     if (c->stage) (void)hipHostFree(c->stage);
+    if (c->wide_active) (void)hipHostFree(c->wide_active);
     if (c->gm_res) (void)hipHostFree(c->gm_res);
     if (c->gm_resq) (void)hipHostFree(c->gm_resq);
     (void)hipStreamDestroy(c->stream);
@@ -3769,6 +4182,209 @@ struct PartView {
     int64_t nobs;
 };
 
+// The m + n above which a block of a launch takes the wide ACA.  A block
+// larger than one resident workgroup's share of all the blocks (about 800
+// workgroups of 256 threads are resident) is still at work, alone on its
+// compute unit, when the others have ended; a smaller one is better in one
+// workgroup, which keeps its place while the chip is full (a wide step's
+// workgroups wait for one every time).  Between kWideMin, where a step of two
+// launches takes as long as one workgroup does, and kWideMax.  Solves with
+// the bound at 1024 / 2048 / 4096: 5120-triangle ellipsoid over a plane (share
+// 345) 18.6 / 25.4 / 38.4 ms, 17892-triangle capsule (2491) 31.0 / 31.6 /
+// 53.9 ms, 20480-triangle sphere in FP64 (3126) 23.0 / 22.4 / 20.7 ms.
+int64_t wide_bound(int64_t sum)
+{
+    return std::min(kWideMax, std::max(kWideMin, sum / kWideShare));
+}
+int64_t wide_sum(const std::vector<bemsetup::Block>& blocks, const std::vector<int32_t>& list)
+{
+    int64_t s = 0;
+    for (int32_t b : list) s += blocks[b].rows + blocks[b].cols;
+    return s;
+}
+
+// ACA class of a block: 0, 1, 2 the workgroup classes (largest first), 3 wide
+int aca_class(const bem_ctx* c, const bemsetup::Block& B, int prec, int64_t wide)
+{
+    const int pi = prec == BEM_PREC_FP32 ? 1 : 0;
+    const int64_t s2 = B.rows + B.cols;
+    return s2 > wide ? 3 : s2 > c->cls_huge[pi] ? 0 : s2 > c->cls_small[pi] ? 1 : 2;
+}
+
+// First-pass rank capacities of the listed blocks (largest first): kCapFirst,
+// and kWideCap for wide blocks, whose ranks are the largest and whose second
+// pass costs most (the capsule's ten largest blocks end at ranks up to 67),
+// as long as that adds no more than a quarter to the scratch.
+void first_caps(const std::vector<bemsetup::Block>& blocks, const std::vector<int32_t>& list, int64_t wide,
+                int64_t maxrank, std::vector<int32_t>& cap)
+{
+    auto lim = [&](const bemsetup::Block& B, int64_t k) {
+        int64_t m = std::min(B.rows, B.cols);
+        if (maxrank > 0) m = std::min(m, maxrank);
+        return (int32_t)std::min(m, k);
+    };
+    int64_t total = 0;
+    for (int32_t b : list) {
+        cap[b] = lim(blocks[b], kCapFirst);
+        total += cap[b] * (blocks[b].rows + blocks[b].cols);
+    }
+    int64_t extra = total / 4;
+    for (int32_t b : list) {
+        const auto& B = blocks[b];
+        if (B.rows + B.cols <= wide) continue;
+        const int32_t k = lim(B, kWideCap);
+        extra -= (k - cap[b]) * (B.rows + B.cols);
+        if (extra < 0) break;
+        cap[b] = k;
+    }
+}
+
+// One wide block of a launch: its list entry (block, frequency item or job
+// item) and extents
+struct WideSrc {
+    int32_t item, cap;
+    int64_t rows, cols;
+};
+
+// The wide ACA's task lists, states and parts on the device (owned by
+// `owned`); uploads on c's stream
+struct WideRun {
+    WideArgs w{};
+    const WideTask *rtask = nullptr, *ctask = nullptr;
+    WideState* state[2] = {nullptr, nullptr};
+    unsigned nrt = 0, nct = 0;
+    size_t shm = 0;
+    int64_t max_steps = 0;
+};
+
+int wide_prepare(bem_ctx* c, const std::vector<WideSrc>& src, size_t esz, std::vector<void*>* owned, WideRun& R)
+{
+    if (src.empty()) return BEM_OK;
+    std::vector<WideBlk> blk(src.size());
+    std::vector<WideTask> rt, ct;
+    std::vector<WideState> st(src.size());
+    int64_t am = 0, d = 0;
+    int maxcap = 1;
+    for (size_t q = 0; q < src.size(); q++) {
+        WideBlk& B = blk[q];
+        B.item = src[q].item;
+        B.cap = src[q].cap;
+        B.nmc = (int32_t)((src[q].rows + kWideChunk - 1) / kWideChunk);
+        B.nnc = (int32_t)((src[q].cols + kWideChunk - 1) / kWideChunk);
+        B.am_col = am;
+        B.am_row = am + B.nmc;
+        am += B.nmc + B.nnc;
+        const int64_t ld = B.cap + 1;
+        B.d_col = d;
+        B.d_row[0] = d + B.nmc * ld;
+        B.d_row[1] = B.d_row[0] + B.nnc * ld;
+        d = B.d_row[1] + B.nnc * ld;
+        for (int32_t k = 0; k < B.nnc; k++) rt.push_back(WideTask{(int32_t)q, k});
+        for (int32_t k = 0; k < B.nmc; k++) ct.push_back(WideTask{(int32_t)q, k});
+        st[q] = WideState{};
+        st[q].phase = kWideStart;
+        maxcap = std::max(maxcap, B.cap);
+    }
+    Packer pk;
+    size_t k_blk = pk.add(blk), k_rt = pk.add(rt), k_ct = pk.add(ct), k_st = pk.add(st), k_st2 = pk.add(st);
+    int rc;
+    if ((rc = pk.upload(c, owned))) return rc;
+    R.w.blk = pk.ptr<WideBlk>(k_blk);
+    R.rtask = pk.ptr<WideTask>(k_rt);
+    R.ctask = pk.ptr<WideTask>(k_ct);
+    R.state[0] = pk.ptr<WideState>(k_st);
+    R.state[1] = pk.ptr<WideState>(k_st2);
+    if ((rc = dalloc(c, &R.w.am, (size_t)am, owned))) return rc;
+    if ((rc = dalloc(c, &R.w.dots, (size_t)d, owned))) return rc;
+    R.nrt = (unsigned)rt.size();
+    R.nct = (unsigned)ct.size();
+    R.shm = (((size_t)maxcap * esz + 15) & ~(size_t)15) + 2 * (size_t)(maxcap + 1) * sizeof(bem_c64);
+    // every step adds a rank or moves on in a pivot list (20 groups of pivots
+    // at most); the loop ends long before this bound
+    R.max_steps = 4 * (int64_t)maxcap + 4096;
+    return BEM_OK;
+}
+
+// a row and a column launch of one step
+template <bool EXTRA, class C, bool PLANE, int MODE, bool FIELD>
+void wide_step(const WideRun& R, const AcaArgs& a, int odd, int32_t* active, hipStream_t st)
+{
+    WideArgs w = R.w;
+    w.odd = odd;
+    w.active = active;
+    w.task = R.rtask;
+    w.in = R.state[0];
+    w.out = R.state[1];
+    hipLaunchKernelGGL((k_wide_row<EXTRA, C, PLANE, MODE, FIELD>), dim3(R.nrt), dim3(kWideChunk), R.shm, st, a, w);
+    w.task = R.ctask;
+    w.in = R.state[1];
+    w.out = R.state[0];
+    hipLaunchKernelGGL((k_wide_col<EXTRA, C, PLANE, MODE, FIELD>), dim3(R.nct), dim3(kWideChunk), R.shm, st, a, w);
+}
+
+template <class C>
+void wide_step_any(const WideRun& R, const AcaArgs& a, bool extra, int odd, int32_t* active, hipStream_t st)
+{
+    if constexpr (sizeof(C) == sizeof(bem_c64)) {
+        if (a.obs) {
+            if (extra) wide_step<true, C, false, 0, true>(R, a, odd, active, st);
+            else wide_step<false, C, false, 0, true>(R, a, odd, active, st);
+            return;
+        }
+    }
+    const bool plane = a.M.rvtx != nullptr;
+    if (a.jobs) {
+        if (extra) wide_step<true, C, false, 3, false>(R, a, odd, active, st);
+        else wide_step<false, C, false, 3, false>(R, a, odd, active, st);
+    } else if (a.nf > 0) {
+        if (extra && plane) wide_step<true, C, true, 1, false>(R, a, odd, active, st);
+        else if (extra) wide_step<true, C, false, 1, false>(R, a, odd, active, st);
+        else if (plane) wide_step<false, C, true, 1, false>(R, a, odd, active, st);
+        else wide_step<false, C, false, 1, false>(R, a, odd, active, st);
+    } else {
+        if (extra && plane) wide_step<true, C, true, 0, false>(R, a, odd, active, st);
+        else if (extra) wide_step<true, C, false, 0, false>(R, a, odd, active, st);
+        else if (plane) wide_step<false, C, true, 0, false>(R, a, odd, active, st);
+        else wide_step<false, C, false, 0, false>(R, a, odd, active, st);
+    }
+}
+
+// The wide ACA on stream st, the whole loop: bursts of kWideBurst steps, one
+// burst in flight ahead of the check whether a block still worked at the last
+// step of the one before (launches past the end return at once).
+constexpr int kWideBurst = 4;
+int wide_run(bem_ctx* c, const WideRun& R, const AcaArgs& a, bool extra, bool f32, hipStream_t st)
+{
+    if (!R.nrt) return BEM_OK;
+    Timer t(c, 2, st);
+    auto run = [&]() -> int {
+        auto burst = [&](int64_t q) -> int {
+            c->wide_active[q & 1] = 0;
+            for (int u = 0; u < kWideBurst; u++) {
+                int32_t* act = c->wide_active + (u == kWideBurst - 1 ? q & 1 : 2);
+                if (f32) wide_step_any<bem_c32>(R, a, extra, u & 1, act, st);
+                else wide_step_any<bem_c64>(R, a, extra, u & 1, act, st);
+            }
+            int rc = launch_check(c, "k_wide_row / k_wide_col");
+            if (rc) return rc;
+            HIPC(c, hipEventRecord(c->wide_ev[q & 1], st));
+            return BEM_OK;
+        };
+        static_assert(kWideBurst % 2 == 0, "the step parity runs on across bursts");
+        int rc;
+        if ((rc = burst(0))) return rc;
+        for (int64_t q = 1;; q++) {
+            if ((rc = burst(q))) return rc;
+            HIPC(c, hipEventSynchronize(c->wide_ev[(q - 1) & 1]));
+            if (!((volatile int32_t*)c->wide_active)[(q - 1) & 1]) return BEM_OK;
+            if (q * kWideBurst > R.max_steps) return set_err(c, BEM_ERR_STATE, "wide ACA: no end");
+        }
+    };
+    const int rc = run();
+    if (rc) (void)hipStreamSynchronize(st);   // nothing runs on when the caller gives the buffers back
+    return rc;
+}
+
 // dynamic LDS of aca_block for rank capacity cap and storage size esz
 size_t aca_shm_bytes(int cap, size_t esz)
 {
@@ -3781,8 +4397,8 @@ size_t aca_shm_bytes(int cap, size_t esz)
 // the results array, and the kernel arguments (blist = the ordered list)
 int aca_prepare(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_t seed,
                 const std::vector<int32_t>& list, const std::vector<int32_t>& cap, const int64_t* d_pivoff,
-                const int32_t* d_piv, AcaScratch& S, AcaArgs& a, std::vector<int32_t> (&cls)[3], size_t& shm,
-                const PartView* pv = nullptr)
+                const int32_t* d_piv, int64_t wide, AcaScratch& S, AcaArgs& a, std::vector<int32_t> (&cls)[4],
+                size_t& shm, const PartView* pv = nullptr)
 {
     const std::vector<bemsetup::Block>& blocks = pv ? *pv->blocks : c->blocks;
     int64_t nb = (int64_t)blocks.size();
@@ -3794,7 +4410,7 @@ int aca_prepare(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uin
         const auto& B = blocks[b];
         S.uoff[b] = tu; S.voff[b] = tv; S.aoff[b] = ta;
         tu += B.rows * cap[b]; tv += B.cols * cap[b]; ta += cap[b];
-        maxcap = std::max(maxcap, cap[b]);
+        if (B.rows + B.cols <= wide) maxcap = std::max(maxcap, cap[b]);
     }
     int rc;
     const size_t esz = prec == BEM_PREC_FP32 ? sizeof(bem_c32) : sizeof(bem_c64);
@@ -3808,18 +4424,15 @@ int aca_prepare(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uin
     // size classes: m + n <= kSmallBlock one wavefront, <= kHugeBlock
     // kMidThreads, larger kHugeThreads (measured: with several lanes sharing
     // the chip, smaller workgroups than one block's pivot chain alone would
-    // want give the higher rate).  The huge and large classes run on their
-    // own streams so
-    // that their long tails overlap the small blocks (and the caller's dense
-    // tiles); within each class the largest blocks start first.
+    // want give the higher rate), above `wide` ([3]) several workgroups
+    // per block.  The two multi-wavefront classes and the wide blocks run on
+    // streams of their own so that their pivot chains overlap the small
+    // blocks (and the caller's dense tiles); within each class the largest
+    // blocks start first.
     for (auto& v : cls) v.clear();
-    for (int32_t b : list) {
-        int64_t s2 = blocks[b].rows + blocks[b].cols;
-        const int pi = prec == BEM_PREC_FP32 ? 1 : 0;
-        cls[s2 > c->cls_huge[pi] ? 0 : (s2 > c->cls_small[pi] ? 1 : 2)].push_back(b);
-    }
+    for (int32_t b : list) cls[aca_class(c, blocks[b], prec, wide)].push_back(b);
     std::vector<int32_t> ordered;
-    for (auto& v : cls) ordered.insert(ordered.end(), v.begin(), v.end());
+    for (int q = 0; q < 3; q++) ordered.insert(ordered.end(), cls[q].begin(), cls[q].end());
     // offsets, capacities and the block list in one upload; ranks, flags and
     // evaluation counts in one allocation written by the kernel for every
     // listed block (the host reads listed blocks only)
@@ -3886,12 +4499,22 @@ int run_aca(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_
 {
     const int64_t nb = (int64_t)(pv ? pv->blocks->size() : c->blocks.size());
     AcaArgs a;
-    std::vector<int32_t> cls[3];
+    std::vector<int32_t> cls[4];
     size_t shm = 0;
     int rc;
-    if ((rc = aca_prepare(c, kind, prec, tol, maxrank, seed, list, cap, d_pivoff, d_piv, S, a, cls, shm, pv)))
+    const int64_t wide = wide_bound(wide_sum(pv ? *pv->blocks : c->blocks, list));
+    if ((rc = aca_prepare(c, kind, prec, tol, maxrank, seed, list, cap, d_pivoff, d_piv, wide, S, a, cls, shm, pv)))
         return rc;
+    const bool x = kind == BEM_KIND_DPHI, f32 = prec == BEM_PREC_FP32;
+    std::vector<WideSrc> ws;
+    for (int32_t b : cls[3]) {
+        const auto& B = pv ? (*pv->blocks)[b] : c->blocks[b];
+        ws.push_back(WideSrc{b, cap[b], B.rows, B.cols});
+    }
+    WideRun R;
+    if ((rc = wide_prepare(c, ws, f32 ? sizeof(bem_c32) : sizeof(bem_c64), &S.owned, R))) return rc;
     HIPC(c, hipEventRecord(c->ev_fork, c->stream));
+    for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
     size_t off = 0;
     for (int q = 0; q < 3; q++) {
         AcaArgs aq = a;
@@ -3899,14 +4522,13 @@ int run_aca(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_
         off += cls[q].size();
         if (q == 2 && (rc = main_work())) return rc;   // e.g. the dense tiles, overlapping the large classes
         if (cls[q].empty()) continue;
-        hipStream_t st = q < 2 ? c->side[q] : c->stream;
-        if (q < 2) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
+        hipStream_t st = q < 2 ? c->side[1] : c->stream;
         Timer t(c, 2, st);
-        bool x = kind == BEM_KIND_DPHI;
-        if (prec == BEM_PREC_FP32) launch_aca<bem_c32>(q, x, (unsigned)cls[q].size(), shm, st, aq);
+        if (f32) launch_aca<bem_c32>(q, x, (unsigned)cls[q].size(), shm, st, aq);
         else launch_aca<bem_c64>(q, x, (unsigned)cls[q].size(), shm, st, aq);
         if ((rc = launch_check(c, "k_aca"))) return rc;
     }
+    if ((rc = wide_run(c, R, a, x, f32, c->side[0]))) return rc;
     for (int q = 0; q < 2; q++) {
         HIPC(c, hipEventRecord(c->ev_join[q], c->side[q]));
         HIPC(c, hipStreamWaitEvent(c->stream, c->ev_join[q], 0));
@@ -4079,11 +4701,12 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
     std::vector<int64_t> uoff(nb, 0), voff(nb, 0), aoff(nb, 0);
     int64_t tu = 0, tv = 0, ta = 0;
     int maxcap = 1;
+    const int64_t wide = wide_bound(nf * wide_sum(c->blocks, list));
     for (int32_t b : list) {
         const auto& B = c->blocks[b];
         uoff[b] = tu; voff[b] = tv; aoff[b] = ta;
         tu += B.rows * cap[b]; tv += B.cols * cap[b]; ta += cap[b];
-        maxcap = std::max(maxcap, cap[b]);
+        if (B.rows + B.cols <= wide) maxcap = std::max(maxcap, cap[b]);
     }
     std::vector<uint64_t> Up(nf), Vp(nf), Ap(nf), Sp(nf);
     std::vector<double> kf(nf);
@@ -4107,11 +4730,8 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
         ccf[f] = jobs[f].cc;
     }
     const int pi = prec == BEM_PREC_FP32 ? 1 : 0;
-    std::vector<int32_t> cls[3];
-    for (int32_t b : list) {
-        int64_t s2 = c->blocks[b].rows + c->blocks[b].cols;
-        cls[s2 > c->cls_huge[pi] ? 0 : (s2 > c->cls_small[pi] ? 1 : 2)].push_back(b);
-    }
+    std::vector<int32_t> cls[4];
+    for (int32_t b : list) cls[aca_class(c, c->blocks[b], prec, wide)].push_back(b);
     std::vector<int32_t> items;
     size_t ncls[3];
     for (int q = 0; q < 3; q++) {
@@ -4120,6 +4740,12 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
         ncls[q] = cls[q].size() * nf;
     }
     if ((int64_t)nf * nb >= ((int64_t)1 << 31)) return set_err(c, BEM_ERR_ARG, "bem_assemble_batch: too many items");
+    std::vector<WideSrc> ws;
+    for (int32_t b : cls[3])
+        for (int f = 0; f < nf; f++)
+            ws.push_back(WideSrc{(int32_t)(f * nb + b), cap[b], c->blocks[b].rows, c->blocks[b].cols});
+    WideRun R;
+    if ((rc = wide_prepare(c, ws, esz, &S[0].owned, R))) return rc;
     Packer pk;
     size_t k_uoff = pk.add(uoff), k_voff = pk.add(voff), k_aoff = pk.add(aoff), k_cap = pk.add(cap);
     size_t k_items = pk.add(items), k_kf = pk.add(kf), k_ccf = pk.add(ccf), k_sp = pk.add(Sp);
@@ -4159,6 +4785,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
     a.queue = nullptr; a.nitems = 0;
     size_t shm = aca_shm_bytes(maxcap, esz);
     HIPC(c, hipEventRecord(c->ev_fork, c->stream));
+    for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
     size_t off = 0;
     // resident workgroups of each class on the chip (256 CUs x 4 SIMDs x
     // 4 waves per SIMD, divided by the class's wavefronts per workgroup)
@@ -4170,8 +4797,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
         off += ncls[q];
         if (q == 2 && (rc = main_work())) return rc;
         if (!ncls[q]) continue;
-        hipStream_t st = q < 2 ? c->side[q] : c->stream;
-        if (q < 2) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
+        hipStream_t st = q < 2 ? c->side[1] : c->stream;
         unsigned grid = (unsigned)ncls[q];
         if (useq) {
             aq.queue = d_queue + q;
@@ -4184,6 +4810,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
         else launch_aca<bem_c64>(q, x, grid, shm, st, aq);
         if ((rc = launch_check(c, "k_aca (batch)"))) return rc;
     }
+    if ((rc = wide_run(c, R, a, kind == BEM_KIND_DPHI, pi, c->side[0]))) return rc;
     for (int q = 0; q < 2; q++) {
         HIPC(c, hipEventRecord(c->ev_join[q], c->side[q]));
         HIPC(c, hipStreamWaitEvent(c->stream, c->ev_join[q], 0));
@@ -4360,7 +4987,7 @@ int bem_assemble(bem_ctx_t c, int kind, double tol, int64_t maxrank, int precisi
         if (maxrank > 0) m = std::min(m, maxrank);
         return (int32_t)m;
     };
-    for (int32_t b : c->adm_list) cap[b] = std::min<int32_t>(full_cap(b), kCapFirst);
+    first_caps(c->blocks, c->adm_list, wide_bound(wide_sum(c->blocks, c->adm_list)), maxrank, cap);
     AcaScratch S1, S2;
     std::vector<int32_t> rank, flag, rank2, flag2;
     std::vector<int64_t> evs, evs2;
@@ -4572,7 +5199,7 @@ int bem_assemble_batch(bem_ctx_t c, int kind, int64_t nf, const double* kcc3, do
         return (int32_t)m;
     };
     std::vector<int32_t> cap(nb, 0);
-    for (int32_t b : c->adm_list) cap[b] = std::min<int32_t>(full_cap(b), kCapFirst);
+    first_caps(c->blocks, c->adm_list, wide_bound(nf * wide_sum(c->blocks, c->adm_list)), maxrank, cap);
     std::vector<FreqJob> jobs((size_t)nf);
     for (int64_t f = 0; f < nf; f++) jobs[f] = FreqJob{kcc3[3 * f], c64(kcc3[3 * f + 1], kcc3[3 * f + 2]), sing[f]};
     std::vector<AcaScratch> S1((size_t)nf);
@@ -4673,7 +5300,7 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
     std::vector<AcaScratch> S1((size_t)nctx);
     std::vector<AcaArgs> A((size_t)nctx);
     std::vector<std::vector<int32_t>> caps((size_t)nctx);
-    std::vector<std::array<std::vector<int32_t>, 3>> cls((size_t)nctx);
+    std::vector<std::array<std::vector<int32_t>, 4>> cls((size_t)nctx);
     std::vector<void*> lead_own;
     auto fail = [&](int code) {
         for (auto* h : H)
@@ -4683,6 +5310,9 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
     };
     int rc;
     size_t shm = 0;
+    int64_t wide = 0;
+    for (int64_t q = 0; q < nctx; q++) wide += wide_sum(ctxs[q]->blocks, ctxs[q]->adm_list);
+    wide = wide_bound(wide);
     for (int64_t q = 0; q < nctx; q++) {   // per context: near field, singular table, ACA scratch
         bem_ctx* c = ctxs[q];
         drop_kept(c);
@@ -4737,25 +5367,21 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
         }
         const int64_t nb = (int64_t)c->blocks.size();
         caps[q].assign(nb, 0);
-        for (int32_t b : c->adm_list) {
-            int64_t m = std::min(c->blocks[b].rows, c->blocks[b].cols);
-            if (maxrank > 0) m = std::min(m, maxrank);
-            caps[q][b] = (int32_t)std::min<int64_t>(m, kCapFirst);
-        }
+        first_caps(c->blocks, c->adm_list, wide, maxrank, caps[q]);
         // every context classifies its blocks by the lead's schedule
         const int64_t keep_s = c->cls_small[pi], keep_h = c->cls_huge[pi];
         c->cls_small[pi] = lead->cls_small[pi];
         c->cls_huge[pi] = lead->cls_huge[pi];
         size_t shm_q = 0;
-        std::vector<int32_t> cq[3];
+        std::vector<int32_t> cq[4];
         c->sing_cur = c->d_sing;
-        rc = aca_prepare(c, kind, precision, tol, maxrank, seed, c->adm_list, caps[q], d_pivoff, d_piv, S1[q], A[q], cq,
-                         shm_q);
+        rc = aca_prepare(c, kind, precision, tol, maxrank, seed, c->adm_list, caps[q], d_pivoff, d_piv, wide, S1[q], A[q],
+                         cq, shm_q);
         c->sing_cur = nullptr;
         c->cls_small[pi] = keep_s;
         c->cls_huge[pi] = keep_h;
         if (rc) return fail(rc);
-        for (int k = 0; k < 3; k++) cls[q][k] = std::move(cq[k]);
+        for (int k = 0; k < 4; k++) cls[q][k] = std::move(cq[k]);
         shm = std::max(shm, shm_q);
         // the lead's launches wait for this context's near field, table and uploads
         HIPC(c, hipEventRecord(c->ev_fork, c->stream));
@@ -4797,7 +5423,15 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
     if (lead->aca_queue) HIPC(lead, hipMemsetAsync(d_queue, 0, 3 * sizeof(int), lead->stream));
     AcaArgs a = A[0];
     a.jobs = d_jobs;
+    std::vector<WideSrc> ws;
+    for (int64_t q = 0; q < nctx; q++)
+        for (int32_t b : cls[q][3])
+            ws.push_back(WideSrc{(int32_t)((q << kJobShift) | b), caps[q][b], ctxs[q]->blocks[b].rows,
+                                 ctxs[q]->blocks[b].cols});
+    WideRun R;
+    if ((rc = wide_prepare(lead, ws, esz, &lead_own, R))) return fail(rc);
     HIPC(lead, hipEventRecord(lead->ev_fork, lead->stream));
+    for (hipStream_t st : lead->side) HIPC(lead, hipStreamWaitEvent(st, lead->ev_fork, 0));
     const int nt[3] = {pi ? kHugeThreads<bem_c32> : kHugeThreads<bem_c64>,
                        pi ? kMidThreads<bem_c32> : kMidThreads<bem_c64>, 64};
     size_t off = 0;
@@ -4806,8 +5440,7 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
         aq.blist = d_items + off;
         off += ncls[k];
         if (!ncls[k]) continue;
-        hipStream_t st = k < 2 ? lead->side[k] : lead->stream;
-        if (k < 2) HIPC(lead, hipStreamWaitEvent(st, lead->ev_fork, 0));
+        hipStream_t st = k < 2 ? lead->side[1] : lead->stream;
         unsigned grid = (unsigned)ncls[k];
         if (lead->aca_queue) {
             aq.queue = d_queue + k;
@@ -4820,6 +5453,7 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
         else launch_aca<bem_c64>(k, x, grid, shm, st, aq);
         if ((rc = launch_check(lead, "k_aca (multi)"))) return fail(rc);
     }
+    if ((rc = wide_run(lead, R, a, kind == BEM_KIND_DPHI, f32, lead->side[0]))) return fail(rc);
     for (int k = 0; k < 2; k++) {
         HIPC(lead, hipEventRecord(lead->ev_join[k], lead->side[k]));
         HIPC(lead, hipStreamWaitEvent(lead->stream, lead->ev_join[k], 0));
@@ -6613,7 +7247,7 @@ int bem_field_hmat(bem_ctx_t c, int64_t nobs, const double* obs3, int64_t nblock
     for (int kind = 0; kind < 2; kind++) {
         std::vector<int32_t> cap((size_t)nblocks, 0), flag, rank2, flag2;
         std::vector<int64_t> evs2;
-        for (int32_t b : adm) cap[b] = std::min<int32_t>(full_cap(b), kCapFirst);
+        first_caps(blocks, adm, wide_bound(wide_sum(blocks, adm)), maxrank, cap);
         if (adm.empty()) break;
         if ((rc = run_aca(c, kind, BEM_PREC_FP64, tol, maxrank, seed, adm, cap, kind ? d_pivoff : nullptr,
                           kind ? d_piv : nullptr, [] { return BEM_OK; }, S[kind][0], rank[kind], flag, evs[kind],

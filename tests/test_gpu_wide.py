@@ -1,0 +1,87 @@
+"""Blocks whose ACA runs over several workgroups (m + n above 1024 on these
+meshes): factors, ranks and evaluation counts bit-identical to the CPU
+restatement in FP64, and the batched, multi-mesh and single launches
+bit-identical to each other in both precisions."""
+import numpy as np
+import pytest
+
+from helpers import upload_problem
+
+pytestmark = pytest.mark.gpu
+WIDE = 1024
+
+
+def same(x, y):
+    return np.array_equal(np.ascontiguousarray(x).view(np.uint64), np.ascontiguousarray(y).view(np.uint64))
+
+
+def capsule_problem(O, meshes, edge, freq, impedance=0.3, plane=None):
+    """capsule with a lined patchwork (columns of both boundary-condition
+    forms in one block), ragged block sizes"""
+    tri = meshes.capsule(2.0, 0.25, edge)
+    bc = meshes.impedance_bc(len(tri), 2 * np.pi * freq / 343.0, impedance, 4)
+    P = O.Problem(tri, bc, leaf=32, eta=2.0)
+    P.set_frequency(freq, 343.0, 1)
+    if plane is not None:
+        P.set_plane(*plane)
+    wide = [b for b in range(len(P.blocks)) if P.blocks[b][4] and P.blocks[b][1] + P.blocks[b][3] > WIDE]
+    assert wide, "no block is large enough"
+    return P, wide
+
+
+@pytest.mark.parametrize("edge,tol,maxrank,plane", [
+    (0.055, 1e-4, 0, None),
+    (0.055, 1e-9, 0, None),       # ranks beyond the first capacity: run again with the full one
+    (0.055, 1e-9, 7, None),       # stopped by the rank limit
+    (0.061, 1e-5, 0, (np.array([0.0, 0.0, -1.5]), np.array([0.0, 0.0, 1.0]))),
+])
+def test_wide_blocks_bit_exact(bem, O, meshes, edge, tol, maxrank, plane):
+    P, wide = capsule_problem(O, meshes, edge, 800.0, plane=plane)
+    ctx = upload_problem(bem, P)
+    if plane is not None:
+        ctx.set_plane(*plane)
+        prm = P.params()
+        ctx.set_frequency(prm["k"], prm["cc"])
+    for kind in (0, 1):
+        H = P.assemble(kind, tol, maxrank, 5)
+        G = ctx.assemble(kind, tol, maxrank, seed=5)
+        ranks = [H.rank(b) for b in wide]
+        print("wide blocks", len(wide), "kind", kind, "tol", tol, "ranks", min(ranks), max(ranks), flush=True)
+        for b in wide:
+            assert G.rank(b) == H.rank(b), (kind, b)
+            for x, y in zip(G.block(b), H.block(b)):
+                assert same(x, y), (kind, b)
+        assert G.stats()["evaluated"] == H.evaluated
+        G.close()
+    ctx.close()
+
+
+def test_wide_launch_forms_agree(bem, O, meshes):
+    freqs = [600.0, 800.0]
+    P, wide = capsule_problem(O, meshes, 0.055, freqs[0], impedance=0.0)
+    Q, wide2 = capsule_problem(O, meshes, 0.061, 700.0)
+    ctx, ctx2 = upload_problem(bem, P), upload_problem(bem, Q)
+    kcc = []
+    for f in freqs:
+        P.set_frequency(f, 343.0, 1)
+        prm = P.params()
+        kcc.append([prm["k"], prm["cc"].real, prm["cc"].imag])
+    for prec in (bem.FP64, bem.FP32):
+        for kind in (0, 1):
+            batch = ctx.assemble_batch(kind, kcc, 1e-4, precision=prec, seed=3)
+            for f in range(len(freqs)):
+                ctx.set_frequency(kcc[f][0], complex(kcc[f][1], kcc[f][2]))
+                single = ctx.assemble(kind, 1e-4, precision=prec, seed=3)
+                assert batch[f].stats()["evaluated"] == single.stats()["evaluated"]
+                assert all(same(x, y) for b in wide for x, y in zip(batch[f].block(b), single.block(b)))
+                batch[f].close()
+                if f == len(freqs) - 1:
+                    multi = bem.assemble_multi([ctx, ctx2], kind, 1e-4, precision=prec, seed=3)
+                    other = ctx2.assemble(kind, 1e-4, precision=prec, seed=3)
+                    assert all(same(x, y) for b in wide for x, y in zip(multi[0].block(b), single.block(b)))
+                    assert all(same(x, y) for b in wide2 for x, y in zip(multi[1].block(b), other.block(b)))
+                    for h in (*multi, other):
+                        h.close()
+                single.close()
+    ctx.close()
+    ctx2.close()
