@@ -571,6 +571,79 @@ template <class C> __device__ __forceinline__ C from64(bem_c64 z);
 template <> __device__ __forceinline__ bem_c64 from64<bem_c64>(bem_c64 z) { return z; }
 template <> __device__ __forceinline__ bem_c32 from64<bem_c32>(bem_c64 z) { return c32((float)z.re, (float)z.im); }
 
+// Lane exchanges on the vector unit: through LDS (ds_bpermute, what
+// __shfl_xor compiles to) each step of a reduction waits some 100 cycles,
+// with data-parallel moves and the half / row swaps of gfx950 a few.
+struct D2 { double a, b; };
+union DWords { double d; uint32_t w[2]; };
+// a's upper half of the wavefront trades with b's lower half: lanes below 32
+// then hold a of both halves (in a and b), the others b of both
+__device__ __forceinline__ D2 lane_swap32(double a, double b)
+{
+    DWords x, y;
+    x.d = a;
+    y.d = b;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const auto t = __builtin_amdgcn_permlane32_swap(x.w[q], y.w[q], false, false);
+        x.w[q] = t[0];
+        y.w[q] = t[1];
+    }
+    return D2{x.d, y.d};
+}
+// the same between the odd rows (16 lanes) of a and the even rows of b
+__device__ __forceinline__ D2 lane_swap16(double a, double b)
+{
+    DWords x, y;
+    x.d = a;
+    y.d = b;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const auto t = __builtin_amdgcn_permlane16_swap(x.w[q], y.w[q], false, false);
+        x.w[q] = t[0];
+        y.w[q] = t[1];
+    }
+    return D2{x.d, y.d};
+}
+// word of lane ^ S
+template <int S>
+__device__ __forceinline__ uint32_t word_xor(uint32_t x)
+{
+    if constexpr (S == 1) return __builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, true);        // quad_perm 1 0 3 2
+    else if constexpr (S == 2) return __builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xF, 0xF, true);   // quad_perm 2 3 0 1
+    else if constexpr (S == 4) {   // from lane + 4 in the even banks of a row, lane - 4 in the odd ones
+        const int t = __builtin_amdgcn_update_dpp((int)x, (int)x, 0x104, 0xF, 0x5, false);
+        return __builtin_amdgcn_update_dpp(t, (int)x, 0x114, 0xF, 0xA, false);
+    } else if constexpr (S == 8) return __builtin_amdgcn_mov_dpp((int)x, 0x128, 0xF, 0xF, true);   // row_ror 8
+    else if constexpr (S == 16) {
+        const auto t = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return (threadIdx.x & 16) ? t[0] : t[1];
+    } else {
+        const auto t = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return (threadIdx.x & 32) ? t[0] : t[1];
+    }
+}
+// value of lane ^ s (s a constant after unrolling)
+__device__ __forceinline__ double lane_xor(double x, int s)
+{
+    DWords u;
+    u.d = x;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        uint32_t w = u.w[q];
+        switch (s) {
+        case 1: w = word_xor<1>(w); break;
+        case 2: w = word_xor<2>(w); break;
+        case 4: w = word_xor<4>(w); break;
+        case 8: w = word_xor<8>(w); break;
+        case 16: w = word_xor<16>(w); break;
+        default: w = word_xor<32>(w); break;
+        }
+        u.w[q] = w;
+    }
+    return u.d;
+}
+
 struct ArgMax { double v; int64_t i; };
 
 __device__ __forceinline__ ArgMax better(ArgMax a, ArgMax b)
@@ -579,50 +652,50 @@ __device__ __forceinline__ ArgMax better(ArgMax a, ArgMax b)
     return a;
 }
 
-// first index of the largest |v_i|^2 over [0, len); index `excl` counts as 0.
-// NT threads (NT / 64 wavefronts); every thread gets the result.  GLOBAL: v
-// lies in device global memory (the ACA's factors) and is read through the
-// global address space; otherwise (e.g. LDS) through generic loads.
-template <bool GLOBAL, class C> __device__ __forceinline__ C ld_any(const C* p)
+// the best of the wavefront's candidates in every lane: the largest value,
+// then the first of the indexes (below 2^31) that have it; none (every v at
+// its initial -1) leaves an index beyond every block
+constexpr int kNoIndex = 0x7fffffff;
+__device__ __forceinline__ ArgMax wave_best(double v, int i)
 {
-    if constexpr (GLOBAL) return ldg(p);
-    else return *p;
+    double m = v;
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) m = fmax(m, lane_xor(m, s));
+    uint32_t k = v == m ? (uint32_t)i : (uint32_t)kNoIndex;
+    k = min(k, word_xor<32>(k));
+    k = min(k, word_xor<16>(k));
+    k = min(k, word_xor<8>(k));
+    k = min(k, word_xor<4>(k));
+    k = min(k, word_xor<2>(k));
+    k = min(k, word_xor<1>(k));
+    return ArgMax{m, (int64_t)k};
 }
-template <int NT, class C, bool GLOBAL = false>
-__device__ ArgMax block_argmax(const C* __restrict__ v, int64_t len, int64_t excl, ArgMax* sred)
+// the same over a workgroup of NT threads (sred: one entry per wavefront)
+template <int NT>
+__device__ __forceinline__ ArgMax group_best(double v, int i, ArgMax* sred)
 {
-    const int tid = threadIdx.x;
-    ArgMax a{-1.0, (int64_t)1 << 62};
-    int64_t t = tid;
-    // four elements per thread loaded together, then compared in index order
-    for (; t + 3 * NT < len; t += 4 * NT) {
-        C e[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) e[u] = ld_any<GLOBAL>(v + t + u * NT);
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int64_t tu = t + u * NT;
-            double x = tu == excl ? 0.0 : cx_abs2(e[u]);
-            if (x > a.v) { a.v = x; a.i = tu; }
-        }
-    }
-    for (; t < len; t += NT) {
-        double x = t == excl ? 0.0 : cx_abs2(ld_any<GLOBAL>(v + t));
-        if (x > a.v) { a.v = x; a.i = t; }
-    }
-    for (int s = 32; s > 0; s >>= 1) {
-        ArgMax o;
-        o.v = __shfl_xor(a.v, s, 64);
-        o.i = __shfl_xor(a.i, s, 64);
-        a = better(a, o);
-    }
+    const ArgMax a = wave_best(v, i);
     if (NT == 64) return a;
     __syncthreads();
-    if ((tid & 63) == 0) sred[tid >> 6] = a;
+    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = a;
     __syncthreads();
     ArgMax r = sred[0];
     for (int w = 1; w < NT / 64; w++) r = better(r, sred[w]);
     return r;
+}
+
+// first index of the largest |v_i|^2 over [0, len); index `excl` counts as 0.
+// NT threads (NT / 64 wavefronts); every thread gets the result.
+template <int NT, class C>
+__device__ ArgMax block_argmax(const C* __restrict__ v, int64_t len, int64_t excl, ArgMax* sred)
+{
+    double best = -1.0;
+    int at = kNoIndex;
+    for (int64_t t = threadIdx.x; t < len; t += NT) {
+        const double x = t == excl ? 0.0 : cx_abs2(v[t]);
+        if (x > best) { best = x; at = (int)t; }
+    }
+    return group_best<NT>(best, at, sred);
 }
 
 struct MeshJob;
@@ -708,7 +781,7 @@ constexpr int32_t kJobMask = (1 << kJobShift) - 1;
 // and the group's totals are reduced together (wave_sum_spread); each task
 // keeps the canonical lane-strided / pairwise order.  Accumulation is FP64
 // for both types.
-constexpr int kDotGroup = 4;
+constexpr int kDotGroup = 8;
 
 // Totals over the 64 lanes of NV values per lane (NV a power of two up to
 // 64), each by the pairwise tree of the device reduction order (partial p
@@ -730,16 +803,21 @@ __device__ __forceinline__ double wave_sum_spread(const double (&x)[NV], int lan
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) {
         if (nv > 1) {
-            const bool hi = lane & s;
             const int h = nv / 2;
 #pragma unroll
             for (int j = 0; j < h; j++) {
-                const double send = hi ? cur[j] : cur[h + j], keep = hi ? cur[h + j] : cur[j];
-                cur[j] = keep + __shfl_xor(send, s, 64);
+                if (s >= 16) {   // one swap per word trades the halves
+                    const D2 t = s == 32 ? lane_swap32(cur[j], cur[h + j]) : lane_swap16(cur[j], cur[h + j]);
+                    cur[j] = t.a + t.b;
+                } else {
+                    const bool hi = lane & s;
+                    const double send = hi ? cur[j] : cur[h + j], keep = hi ? cur[h + j] : cur[j];
+                    cur[j] = keep + lane_xor(send, s);
+                }
             }
             nv = h;
         } else {
-            cur[0] = cur[0] + __shfl_xor(cur[0], s, 64);
+            cur[0] = cur[0] + lane_xor(cur[0], s);
         }
     }
     return cur[0];
@@ -808,17 +886,19 @@ __device__ __forceinline__ void aca_dots(const C* col, const C* row, const C* U,
 
 // Frobenius-norm estimate update of partialPivotACA (hmatrix.cpp:568-572);
 // every thread computes it identically from the LDS dot products
-template <class C>
-__device__ __forceinline__ double aca_update_norm(C alpha, const C* A, int r, const bem_c64* sdots, bem_c64& S)
+// (the terms formed in parallel into the dot products' places, then added in
+// rank order by every thread)
+template <int NT, class C>
+__device__ __forceinline__ double aca_update_norm(C alpha, const C* A, int r, bem_c64* sdots, bem_c64& S)
 {
-    double gain = (cx_abs2(alpha) * sdots[0].re) * sdots[1].re;
+    const double gain = (cx_abs2(alpha) * sdots[0].re) * sdots[1].re;
     bem_c64 s = S;
     s.re = s.re + gain;
-    bem_c64 ca2 = c64_scale(c64_conj(ld64(&alpha)), 2.0);
-    for (int l = 0; l < r; l++) {
-        bem_c64 t = c64_mul(c64_mul(c64_mul(ca2, ld64(A + l)), sdots[3 + 2 * l]), sdots[2 + 2 * l]);
-        s = c64_add(s, t);
-    }
+    const bem_c64 ca2 = c64_scale(c64_conj(ld64(&alpha)), 2.0);
+    for (int l = threadIdx.x; l < r; l += NT)
+        sdots[2 + 2 * l] = c64_mul(c64_mul(c64_mul(ca2, ld64(A + l)), sdots[3 + 2 * l]), sdots[2 + 2 * l]);
+    __syncthreads();
+    for (int l = 0; l < r; l++) s = c64_add(s, sdots[2 + 2 * l]);
     S = s;
     return gain;
 }
@@ -861,16 +941,54 @@ __device__ __forceinline__ bool near_or_self(const DevMesh& M, int64_t i, int64_
 
 // regular entry of (i, j), or false for a self / near-singular pair; PLANE:
 // plus the mirror image's entry (a template argument so that the plain
-// kernels keep their register budget)
+// kernels keep their register budget).  Only the operators the active lanes'
+// entries use are accumulated (bc_needs); two quadrature points at a time, so
+// that one point's chain of dependent operations fills the other's waits.
+constexpr int kQuadUnroll = 2;
+__device__ __forceinline__ bem_ops4 ops_of(int need, double k, double px, double py, double pz, double npx,
+                                           double npy, double npz, double nqx, double nqy, double nqz, double area,
+                                           const ElemVtx& e)
+{
+    if (need == 1) return regular_ops_need<1, kQuadUnroll>(k, px, py, pz, npx, npy, npz, nqx, nqy, nqz, area, e);
+    if (need == 2) return regular_ops_need<2, kQuadUnroll>(k, px, py, pz, npx, npy, npz, nqx, nqy, nqz, area, e);
+    return regular_ops_need<3, kQuadUnroll>(k, px, py, pz, npx, npy, npz, nqx, nqy, nqz, area, e);
+}
+__device__ __forceinline__ bem_c32f4 ops_of_f32(int need, const DevFreq32& F, const DevMesh& M, int64_t i, int64_t j,
+                                                const double* edg, const double* qnx, const double* qny,
+                                                const double* qnz)
+{
+    const int64_t n = M.n;
+    const double* g = edg + j;
+    const double dx = M.px[i] - g[0], dy = M.py[i] - g[n], dz = M.pz[i] - g[2 * n];
+    const double ax = g[3 * n], ay = g[4 * n], az = g[5 * n], bx = g[6 * n], by = g[7 * n], bz = g[8 * n];
+    const float npx = (float)M.nx[i], npy = (float)M.ny[i], npz = (float)M.nz[i];
+    const float nqx = (float)qnx[j], nqy = (float)qny[j], nqz = (float)qnz[j];
+    const float area = (float)M.area[j];
+    if (need == 1)
+        return regular_ops_f32_need<1, kQuadUnroll>(F, dx, dy, dz, ax, ay, az, bx, by, bz, npx, npy, npz, nqx, nqy, nqz, area);
+    if (need == 2)
+        return regular_ops_f32_need<2, kQuadUnroll>(F, dx, dy, dz, ax, ay, az, bx, by, bz, npx, npy, npz, nqx, nqy, nqz, area);
+    return regular_ops_f32_need<3, kQuadUnroll>(F, dx, dy, dz, ax, ay, az, bx, by, bz, npx, npy, npz, nqx, nqy, nqz, area);
+}
 template <bool PLANE>
 __device__ __forceinline__ bool regular_entry(const AcaArgs& a, int64_t i, int64_t j, bem_c64* e, bool nearb = true)
 {
     const DevMesh& M = a.M;
     if (nearb && near_or_self(M, i, j)) return false;
-    bem_ops4 o = regular_ops_vtx<1>(a.F.k, M.px[i], M.py[i], M.pz[i], M.nx[i], M.ny[i], M.nz[i], M.nx[j], M.ny[j],
-                                    M.nz[j], M.area[j], load_vtx(M, j));
+    const int need = bc_needs(a.F.subst, a.F.cd, a.kind, j);
+    const double px = M.px[i], py = M.py[i], pz = M.pz[i], npx = M.nx[i], npy = M.ny[i], npz = M.nz[i];
+    bem_ops4 o = ops_of(need, a.F.k, px, py, pz, npx, npy, npz, M.nx[j], M.ny[j], M.nz[j], M.area[j], load_vtx(M, j));
     *e = bc_entry(a.F, a.kind, o, i, j);
-    if (PLANE) *e = c64_add(*e, refl_entry(M, a.F, a.kind, i, j));
+    if (PLANE) {   // refl_entry
+        const double* v = M.rvtx + j;
+        const int64_t n = M.n;
+        const ElemVtx r{v[0], v[n], v[2 * n], v[3 * n], v[4 * n], v[5 * n], v[6 * n], v[7 * n], v[8 * n]};
+        o = ops_of(need, a.F.k, px, py, pz, npx, npy, npz, M.rnx[j], M.rny[j], M.rnz[j], M.area[j], r);
+        bem_c64 X, Y;
+        bem_xy(&o, a.F.cc, 0, &X, &Y);
+        *e = c64_add(*e, a.kind == 0 ? bem_phi_entry(X, Y, a.F.subst[j], a.F.cphi[j])
+                                     : bem_dphi_entry(X, Y, a.F.subst[j], a.F.cd[j]));
+    }
     return true;
 }
 template <bool PLANE>
@@ -878,13 +996,11 @@ __device__ __forceinline__ bool regular_entry(const AcaArgs& a, int64_t i, int64
 {
     const DevMesh& M = a.M;
     if (nearb && near_or_self(M, i, j)) return false;
-    // only the operators the entry uses (the others stay zero, and the
-    // entry formula then gives the same value)
-    const int need = bc_needs_f32(a.F32, a.F.subst, a.kind, j);
-    bem_c32f4 o = regular_ops_f32_edge<1>(a.F32, M, i, j, need & 1, need & 2);
-    *e = bc_entry_f32(a.F32, a.F.subst, a.kind, o, j);
+    const int need = bc_needs(a.F.subst, a.F32.cd, a.kind, j);
+    *e = bc_entry_f32(a.F32, a.F.subst, a.kind, ops_of_f32(need, a.F32, M, i, j, M.edg, M.nx, M.ny, M.nz), j);
     if (PLANE) {
-        bem_c32 r = bc_entry_f32(a.F32, a.F.subst, a.kind, refl_ops_f32(a.F32, M, i, j), j);
+        const bem_c32 r = bc_entry_f32(a.F32, a.F.subst, a.kind,
+                                       ops_of_f32(need, a.F32, M, i, j, M.redg, M.rnx, M.rny, M.rnz), j);
         *e = c32(e->re + r.re, e->im + r.im);
     }
     return true;
@@ -930,70 +1046,34 @@ __device__ __forceinline__ C entry_any(const AcaArgs& a, int64_t i, int64_t j, b
     return singular_entry<C>(a, i, i == j ? -1 : near_find(a.M, i, (int32_t)j));
 }
 
-// Row i of the block minus the current cross approximation, into dst.
-// Regular entries first; the few self / near-singular entries of the row
-// (CSR row r0 + i) in a second pass, so that the main loop has no divergent
-// branch.
+// Row `fixed` (row) or column `fixed` of the block minus the current cross
+// approximation, into dst; every thread gets the largest |v|^2 and its first
+// index, index `excl` counting as 0.  One body for rows and columns (a
+// scalar decides), so that the quadrature is in the kernel once.
 template <int NT, class C, bool PLANE, bool FIELD = false>
-__device__ void aca_row(const AcaArgs& a, int64_t r0, int64_t c0, int64_t m, int64_t n, int r, int64_t i,
-                        const C* U, const C* V, const C* A, C* dst, C* sw, bool nearb)
+__device__ __forceinline__ ArgMax aca_line(const AcaArgs& a, bool row, int64_t r0, int64_t c0, int64_t m, int64_t n,
+                                           int r, int64_t fixed, const C* U, const C* V, const C* A, C* dst, C* sw,
+                                           bool nearb, int64_t excl, ArgMax* sred)
 {
-    for (int l = threadIdx.x; l < r; l += NT) sw[l] = cx_mul(ldg(U + (int64_t)l * m + i), ldg(A + l));
+    if (row)
+        for (int l = threadIdx.x; l < r; l += NT) sw[l] = cx_mul(ldg(U + (int64_t)l * m + fixed), ldg(A + l));
+    else
+        for (int l = threadIdx.x; l < r; l += NT) sw[l] = cx_mul(ldg(A + l), ldg(V + (int64_t)l * n + fixed));
     __syncthreads();
-    const int64_t gi = r0 + i;
-    for (int64_t j = threadIdx.x; j < n; j += NT) {
-        C e;
-        if constexpr (FIELD) e = from64<C>(field_entry(a, gi, c0 + j));
-        else if (!regular_entry<PLANE>(a, gi, c0 + j, &e, nearb)) continue;
-        dst[j] = cx_sub(e, cross_sum<true>(sw, V, n, j, r));
+    const int64_t len = row ? n : m, gi0 = row ? r0 + fixed : r0, gj0 = row ? c0 : c0 + fixed;
+    double best = -1.0;
+    int at = kNoIndex;
+    for (int64_t t = threadIdx.x; t < len; t += NT) {
+        const int64_t gi = row ? gi0 : gi0 + t, gj = row ? gj0 + t : gj0;
+        const C e = entry_any<PLANE, C, FIELD>(a, gi, gj, nearb);
+        const C v = cx_sub(e, row ? cross_sum<true>(sw, V, n, t, r) : cross_sum<false>(sw, U, m, t, r));
+        dst[t] = v;
+        const double x = t == excl ? 0.0 : cx_abs2(v);
+        if (x > best) { best = x; at = (int)t; }
     }
-    // no self or near-singular entries between observation points and
-    // elements, nor in a block whose collocation boxes lie apart
-    if (FIELD || !nearb) {
-        __syncthreads();
-        return;
-    }
-    const int64_t p0 = a.M.nr_ptr[gi], p1 = a.M.nr_ptr[gi + 1];
-    for (int64_t t = p0 + threadIdx.x; t <= p1; t += NT) {
-        int64_t gj = t < p1 ? a.M.nr_col[t] : gi;
-        if (gj < c0 || gj >= c0 + n) continue;
-        int64_t j = gj - c0;
-        C e = singular_entry<C>(a, gi, t < p1 ? t : -1);
-        dst[j] = cx_sub(e, cross_sum<true>(sw, V, n, j, r));
-    }
+    const ArgMax q = group_best<NT>(best, at, sred);
     __syncthreads();
-}
-
-// column j of the block minus the current cross approximation, into dst;
-// the near-singular rows of column c0 + j are the near list of row c0 + j
-// (the distance criterion is symmetric)
-template <int NT, class C, bool PLANE, bool FIELD = false>
-__device__ void aca_col(const AcaArgs& a, int64_t r0, int64_t c0, int64_t m, int64_t n, int r, int64_t j,
-                        const C* U, const C* V, const C* A, C* dst, C* sw, bool nearb)
-{
-    for (int l = threadIdx.x; l < r; l += NT) sw[l] = cx_mul(ldg(A + l), ldg(V + (int64_t)l * n + j));
-    __syncthreads();
-    const int64_t gj = c0 + j;
-    for (int64_t i = threadIdx.x; i < m; i += NT) {
-        C e;
-        if constexpr (FIELD) e = from64<C>(field_entry(a, r0 + i, gj));
-        else if (!regular_entry<PLANE>(a, r0 + i, gj, &e, nearb)) continue;
-        dst[i] = cx_sub(e, cross_sum<false>(sw, U, m, i, r));
-    }
-    if (FIELD || !nearb) {
-        __syncthreads();
-        return;
-    }
-    const int64_t p0 = a.M.nr_ptr[gj], p1 = a.M.nr_ptr[gj + 1];
-    for (int64_t t = p0 + threadIdx.x; t <= p1; t += NT) {
-        int64_t gi = t < p1 ? a.M.nr_col[t] : gj;
-        if (gi < r0 || gi >= r0 + m) continue;
-        int64_t i = gi - r0;
-        int64_t pair = t < p1 ? near_find(a.M, gi, (int32_t)gj) : -1;
-        C e = singular_entry<C>(a, gi, pair);
-        dst[i] = cx_sub(e, cross_sum<false>(sw, U, m, i, r));
-    }
-    __syncthreads();
+    return q;
 }
 
 // The entry counter of an ACA is the same in every lane; it is kept in scalar
@@ -1006,6 +1086,50 @@ __device__ __forceinline__ int64_t uni64(int64_t x)
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)x >> 32));
     return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// a condition that is the same in every lane, as a scalar
+__device__ __forceinline__ bool uni_true(bool x) { return __builtin_amdgcn_readfirstlane((int)x) != 0; }
+
+// The first listed pivot from position p on (p1 the end) whose entry is
+// nonzero and not met by the approximation: 64 positions at a time, one per
+// lane, every wavefront the same.  Its column, and p its position; -1 when
+// none is left.  ev counts the entries evaluated up to it.
+template <bool PLANE, class C, bool FIELD>
+__device__ __forceinline__ int64_t next_pivot(const AcaArgs& a, int64_t r0, int64_t c0, int64_t m, int64_t n, int r,
+                                              const C* U, const C* V, const C* A, int64_t& p, int64_t p1, double tol2,
+                                              double tiny2, bool nearb, int64_t& ev)
+{
+    const int lane = threadIdx.x & 63;
+    while (p < p1) {
+        int64_t pj = 0;
+        bool take = false;
+        if (p + lane < p1) {
+            const int64_t pi = a.piv[2 * (p + lane)];
+            pj = a.piv[2 * (p + lane) + 1];
+            const C pe = entry_any<PLANE, C, FIELD>(a, r0 + pi, c0 + pj, nearb);
+            if (!(cx_abs2(pe) < tiny2)) {
+                // the approximation there, its rank terms in rank order
+                C approx = cx_zero<C>();
+#pragma unroll 4
+                for (int l = 0; l < r; l++)
+                    approx = cx_add(approx, cx_mul(cx_mul(ldg(U + (int64_t)l * m + pi), ldg(A + l)),
+                                                   ldg(V + (int64_t)l * n + pj)));
+                take = !(cx_abs2(cx_sub(pe, approx)) < tol2 * cx_abs2(pe));
+            }
+        }
+        const uint64_t mask = __ballot(take);
+        if (mask) {
+            const int f = __ffsll((unsigned long long)mask) - 1;
+            ev = uni64(ev + f + 1);
+            p = uni64(p + f);
+            return __shfl(pj, f, 64);
+        }
+        const int64_t left = p1 - p < 64 ? p1 - p : 64;
+        ev = uni64(ev + left);
+        p = uni64(p + left);
+    }
+    return -1;
 }
 
 // ACA of one admissible block b by a workgroup of NT threads.  Plain
@@ -1033,87 +1157,76 @@ __device__ void aca_block(const AcaArgs& a, const int b, char* dyn, ArgMax* sred
     int r = 0, flag = 0;
     int64_t ev = 0;
     bem_c64 S = c64(0, 0);
-    if (!EXTRA) {
-        int64_t j = bem_rand_bounded(a.seed, 0, (uint64_t)b, 0, n);
-        aca_col<NT, C, PLANE, FIELD>(a, r0, c0, m, n, 0, j, U, V, A, U, sw, nearb);
-        ev = uni64(ev + m);
-        int64_t i = -1;
-        while (r < maxRank) {
-            if (r >= cap) { flag = 1; break; }
-            const C* wcol = r >= 1 ? U + (int64_t)(r - 1) * m : U;
-            ArgMax am = block_argmax<NT, C, true>(wcol, m, r >= 1 ? i : -1, sred);
-            i = am.i;
-            if (am.v <= tiny2 && r >= 1) break;
-            C* row = V + (int64_t)r * n;
-            aca_row<NT, C, PLANE, FIELD>(a, r0, c0, m, n, r, i, U, V, A, row, sw, nearb);
-            ev = uni64(ev + n);
-            ArgMax ar = block_argmax<NT, C, true>(row, n, -1, sred);
-            if (ar.v <= tiny2 && r >= 1) break;
-            C* col = U + (int64_t)r * m;
-            aca_col<NT, C, PLANE, FIELD>(a, r0, c0, m, n, r, ar.i, U, V, A, col, sw, nearb);
-            ev = uni64(ev + m);
-            C alpha = cx_inv(row[ar.i]);
-            if (threadIdx.x == 0) A[r] = sA[r] = alpha;
-            aca_dots<NT>(col, row, U, V, m, n, r, sdots);
-            __syncthreads();
-            double gain = aca_update_norm(alpha, sA, r, sdots, S);
-            r++;
-            __syncthreads();
-            if (!(isfinite(gain))) { flag = 2; break; }
-            if (a.tol > 0 && gain < tol2 * S.re) break;
-        }
+    int64_t p = EXTRA ? a.piv_off[b] : 0;
+    const int64_t p1 = EXTRA ? a.piv_off[b + 1] : 0;
+    // the line to compute next: column `fixed` (a first column, or with
+    // `step` the column of the row pivot i) or row `fixed`
+    bool row = false, step = false;
+    int64_t fixed = 0, excl = -1, i = -1;
+    if (EXTRA) {
+        fixed = uni64(next_pivot<PLANE, C, FIELD>(a, r0, c0, m, n, r, U, V, A, p, p1, tol2, tiny2, nearb, ev));
+        if (fixed >= 0 && cap < 1) { flag = 1; fixed = -1; }
     } else {
-        const int64_t p0 = a.piv_off[b], p1 = a.piv_off[b + 1];
-        bool done = false;
-        for (int64_t p = p0; p < p1 && r < maxRank && !done; p++) {
-            int64_t i = a.piv[2 * p], j = a.piv[2 * p + 1];
-            C pe = entry_any<PLANE, C, FIELD>(a, r0 + i, c0 + j, nearb);
-            ev = uni64(ev + 1);
-            if (cx_abs2(pe) < tiny2) continue;
-            // the approximation at (i, j): its rank terms formed in parallel,
-            // then summed in rank order by every thread
-            for (int l = threadIdx.x; l < r; l += NT)
-                sw[l] = cx_mul(cx_mul(ldg(U + (int64_t)l * m + i), sA[l]), ldg(V + (int64_t)l * n + j));
-            __syncthreads();
-            C approx = cx_zero<C>();
-            for (int l = 0; l < r; l++) approx = cx_add(approx, sw[l]);
-            __syncthreads();
-            if (cx_abs2(cx_sub(pe, approx)) < tol2 * cx_abs2(pe)) continue;
-            if (r >= cap) { flag = 1; break; }
-            aca_col<NT, C, PLANE, FIELD>(a, r0, c0, m, n, r, j, U, V, A, U + (int64_t)r * m, sw, nearb);
-            ev = uni64(ev + m);
-            bool first = true;
-            while (r < maxRank) {
-                if (r >= cap) { flag = 1; done = true; break; }
-                const C* wcol = first ? U + (int64_t)r * m : U + (int64_t)(r - 1) * m;
-                ArgMax am = block_argmax<NT, C, true>(wcol, m, first ? -1 : i, sred);
-                i = am.i;
-                first = false;
-                if (cx_abs2(wcol[i]) <= tiny2 && r >= 1) break;
-                C* row = V + (int64_t)r * n;
-                aca_row<NT, C, PLANE, FIELD>(a, r0, c0, m, n, r, i, U, V, A, row, sw, nearb);
-                ev = uni64(ev + n);
-                ArgMax ar = block_argmax<NT, C, true>(row, n, -1, sred);
-                if (ar.v <= tiny2 && r >= 1) break;
-                C* col = U + (int64_t)r * m;
-                aca_col<NT, C, PLANE, FIELD>(a, r0, c0, m, n, r, ar.i, U, V, A, col, sw, nearb);
-                ev = uni64(ev + m);
-                C alpha = cx_inv(row[ar.i]);
+        fixed = bem_rand_bounded(a.seed, 0, (uint64_t)b, 0, n);
+    }
+    while (fixed >= 0) {
+        C* dst = row ? V + (int64_t)r * n : U + (int64_t)r * m;
+        const ArgMax q = aca_line<NT, C, PLANE, FIELD>(a, row, r0, c0, m, n, r, fixed, U, V, A, dst, sw, nearb, excl,
+                                                       sred);
+        const int64_t qi = uni64(q.i);
+        ev = uni64(ev + (row ? n : m));
+        if (qi == kNoIndex) {   // no finite entry
+            flag = 2;
+            break;
+        }
+        if (row) {
+            if (uni_true(!(q.v <= tiny2 && r >= 1))) {   // its column comes next
+                row = false;
+                step = true;
+                fixed = qi;
+                excl = i;
+                continue;
+            }
+        } else {
+            bool more = true;
+            if (step) {   // row and column r are in place
+                const C* vrow = V + (int64_t)r * n;
+                const C alpha = cx_inv(ldg(vrow + fixed));
                 if (threadIdx.x == 0) A[r] = sA[r] = alpha;
-                aca_dots<NT>(col, row, U, V, m, n, r, sdots);
+                aca_dots<NT>(dst, vrow, U, V, m, n, r, sdots);
                 __syncthreads();
-                bem_c64 oldS = S;
-                double gain = aca_update_norm(alpha, sA, r, sdots, S);
+                const bem_c64 oldS = S;
+                const double gain = aca_update_norm<NT>(alpha, sA, r, sdots, S);
                 r++;
                 __syncthreads();
-                if (!(isfinite(gain))) { flag = 2; done = true; break; }
-                double target = tol2 * S.re;
-                if (a.tol > 0 && gain < target) {
-                    if (gain < 0.1 * target) { r--; S = oldS; }
-                    break;
+                if (uni_true(!isfinite(gain))) { flag = 2; break; }
+                const double target = tol2 * S.re;
+                if (uni_true(a.tol > 0 && gain < target)) {
+                    if (!EXTRA) break;
+                    if (uni_true(gain < 0.1 * target)) { r--; S = oldS; }
+                    more = false;
+                }
+            }
+            if (more && r < maxRank) {
+                if (r >= cap) { flag = 1; break; }
+                // the row pivot: the largest entry of the last column
+                i = qi;
+                const double x = EXTRA && qi == excl ? cx_abs2(ldg(dst + qi)) : q.v;
+                if (uni_true(!(x <= tiny2 && r >= 1))) {
+                    row = true;
+                    fixed = i;
+                    excl = -1;
+                    continue;
                 }
             }
         }
+        // the pivot chain ended: the next listed pivot, if any
+        if (!EXTRA || r >= maxRank) break;
+        p++;
+        fixed = uni64(next_pivot<PLANE, C, FIELD>(a, r0, c0, m, n, r, U, V, A, p, p1, tol2, tiny2, nearb, ev));
+        if (fixed >= 0 && r >= cap) { flag = 1; break; }
+        row = step = false;
+        excl = -1;
     }
     if (threadIdx.x == 0) {
         a.rank_out[b] = r;
@@ -1229,6 +1342,7 @@ __global__ __launch_bounds__(NT, (PLANE && kAcaWaves<NT, C> > 3 ? 3 : kAcaWaves<
 // boundary is the only barrier.  States are double buffered: a launch reads
 // one copy and its first workgroup of the block writes the other.
 constexpr int kWideChunk = 256;   // entries (and threads) per workgroup
+constexpr int kWideDots = 4;      // dot products per wavefront at a time
 enum WidePhase : int32_t {
     kWideStart,      // nothing computed yet
     kWideProbe,      // EXTRA: the inner loop ended, the next listed pivot comes
@@ -1266,20 +1380,9 @@ struct WideArgs {
 // first index on ties, so the order of combination does not matter
 __device__ __forceinline__ ArgMax wide_best(const ArgMax* part, int cnt, ArgMax* sred)
 {
-    ArgMax a{-1.0, (int64_t)1 << 62};
+    ArgMax a{-1.0, kNoIndex};
     for (int q = threadIdx.x; q < cnt; q += kWideChunk) a = better(a, part[q]);
-    for (int s = 32; s > 0; s >>= 1) {
-        ArgMax o;
-        o.v = __shfl_xor(a.v, s, 64);
-        o.i = __shfl_xor(a.i, s, 64);
-        a = better(a, o);
-    }
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = a;
-    __syncthreads();
-    ArgMax r = sred[0];
-    for (int w = 1; w < kWideChunk / 64; w++) r = better(r, sred[w]);
-    return r;
+    return group_best<kWideChunk>(a.v, (int)a.i, sred);
 }
 
 // One chunk of a residual row (ROW: entries (gi, c0 + t), basis V of stride
@@ -1298,42 +1401,26 @@ __device__ __forceinline__ void wide_line(const AcaArgs& a, int64_t r0, int64_t 
     C v = cx_zero<C>();
     if (tid < cnt) {
         const int64_t gi = ROW ? gf : r0 + t, gj = ROW ? c0 + t : gf;
-        C e;
-        bool have = true;
-        if constexpr (FIELD) {
-            e = from64<C>(field_entry(a, gi, gj));
-        } else {
-            have = regular_entry<PLANE>(a, gi, gj, &e, nearb);
-            if (!have) e = singular_entry<C>(a, gi, gi == gj ? -1 : near_find(a.M, gi, (int32_t)gj));
-        }
+        const C e = entry_any<PLANE, C, FIELD>(a, gi, gj, nearb);
         v = cx_sub(e, cross_sum<ROW>(sw, W, len, t, r));
         dst[t] = v;
     }
     sv[tid] = v;
-    ArgMax m{-1.0, (int64_t)1 << 62};
+    double best = -1.0;
+    int at = kNoIndex;
     if (tid < cnt) {
         const double x = t == excl ? 0.0 : cx_abs2(v);
-        if (x > m.v) { m.v = x; m.i = t; }
+        if (x > best) { best = x; at = (int)t; }
     }
-    for (int s = 32; s > 0; s >>= 1) {
-        ArgMax o;
-        o.v = __shfl_xor(m.v, s, 64);
-        o.i = __shfl_xor(m.i, s, 64);
-        m = better(m, o);
-    }
-    if ((tid & 63) == 0) sred[tid >> 6] = m;
-    __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < kWideChunk / 64; w++) m = better(m, sred[w]);
-        *am = m;
-    }
+    const ArgMax q = group_best<kWideChunk>(best, at, sred);   // (its barriers also publish sv)
+    if (tid == 0) *am = q;
     if (!want_dots) return;
     const int lane = tid & 63;
-    for (int kb = (tid >> 6) * kDotGroup; kb <= r; kb += (kWideChunk / 64) * kDotGroup) {
-        const C* src[kDotGroup];
-        bem_c64 acc[kDotGroup];
+    for (int kb = (tid >> 6) * kWideDots; kb <= r; kb += (kWideChunk / 64) * kWideDots) {
+        const C* src[kWideDots];
+        bem_c64 acc[kWideDots];
 #pragma unroll
-        for (int g = 0; g < kDotGroup; g++) {
+        for (int g = 0; g < kWideDots; g++) {
             const int k = kb + g;
             src[g] = (k >= 1 && k <= r) ? W + (int64_t)(k - 1) * len + t0 : dst + t0;
             acc[g] = c64(0, 0);
@@ -1344,22 +1431,22 @@ __device__ __forceinline__ void wide_line(const AcaArgs& a, int64_t r0, int64_t 
             const int u = lane + 64 * q;
             if (u >= cnt) break;
             const bem_c64 cv = ld64(&sv[u]);
-            C wv[kDotGroup];
+            C wv[kWideDots];
 #pragma unroll
-            for (int g = 0; g < kDotGroup; g++) wv[g] = ldg(src[g] + u);
+            for (int g = 0; g < kWideDots; g++) wv[g] = ldg(src[g] + u);
             nrm = nrm + c64_abs2(cv);
 #pragma unroll
-            for (int g = 0; g < kDotGroup; g++) acc[g] = c64_fma(c64_conj(cv), ld64(&wv[g]), acc[g]);
+            for (int g = 0; g < kWideDots; g++) acc[g] = c64_fma(c64_conj(cv), ld64(&wv[g]), acc[g]);
         }
         if (kb == 0) acc[0] = c64(nrm, 0.0);
-        double x[2 * kDotGroup];
+        double x[2 * kWideDots];
 #pragma unroll
-        for (int g = 0; g < kDotGroup; g++) {
+        for (int g = 0; g < kWideDots; g++) {
             x[2 * g] = acc[g].re;
             x[2 * g + 1] = acc[g].im;
         }
-        const double tot = wave_sum_spread<2 * kDotGroup>(x, lane);
-        constexpr int kStride = 64 / (2 * kDotGroup);
+        const double tot = wave_sum_spread<2 * kWideDots>(x, lane);
+        constexpr int kStride = 64 / (2 * kWideDots);
         if ((lane & (kStride - 1)) == 0) {
             const int q = lane / kStride, k = kb + (q >> 1);
             if (k <= r) ((double*)(dots + k))[q & 1] = tot;
@@ -1491,42 +1578,14 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
     if (EXTRA && probe) {
         // the listed pivots from s.p on, 64 at a time (one per lane, every
         // wavefront the same): the first whose entry the approximation misses
-        const int64_t p1 = a.piv_off[b + 1];
-        const int lane = tid & 63, r = s.r;
         s.phase = kWideDone;
-        while (s.r < maxRank && s.p < p1) {
-            const int64_t p = s.p + lane;
-            int64_t pj = 0;
-            bool take = false;
-            if (p < p1) {
-                const int64_t pi = a.piv[2 * p];
-                pj = a.piv[2 * p + 1];
-                const C pe = entry_any<PLANE, C, FIELD>(a, r0 + pi, c0 + pj, nearb);
-                if (!(cx_abs2(pe) < tiny2)) {
-                    C approx = cx_zero<C>();
-#pragma unroll 4
-                    for (int l = 0; l < r; l++)
-                        approx = cx_add(approx, cx_mul(cx_mul(ldg(U + (int64_t)l * m + pi), ldg(A + l)),
-                                                       ldg(V + (int64_t)l * n + pj)));
-                    take = !(cx_abs2(cx_sub(pe, approx)) < tol2 * cx_abs2(pe));
-                }
+        if (s.r < maxRank) {
+            s.j = next_pivot<PLANE, C, FIELD>(a, r0, c0, m, n, s.r, U, V, A, s.p, a.piv_off[b + 1], tol2, tiny2, nearb,
+                                              s.ev);
+            if (s.j >= 0) {
+                if (s.r >= cap) s.flag = 1;
+                else s.phase = kWideFirstCol;
             }
-            const uint64_t mask = __ballot(take);
-            if (mask) {
-                const int f = __ffsll((unsigned long long)mask) - 1;
-                s.ev += f + 1;
-                s.p += f;
-                s.j = __shfl(pj, f, 64);
-                s.phase = kWideFirstCol;
-                if (s.r >= cap) {
-                    s.flag = 1;
-                    s.phase = kWideDone;
-                }
-                break;
-            }
-            const int64_t left = p1 - s.p < 64 ? p1 - s.p : 64;
-            s.ev += left;
-            s.p += left;
         }
     }
     if (s.phase == kWideRow) s.ev += n;

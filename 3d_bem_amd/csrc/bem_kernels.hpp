@@ -24,6 +24,30 @@ __constant__ static const double kTriX[16][2] = {
     {0.89890554336594, 0.05054722831703}, {0.26311282963464, 0.72849239295540}, {0.72849239295540, 0.00839477740996},
     {0.00839477740996, 0.26311282963464}, {0.72849239295540, 0.26311282963464}, {0.26311282963464, 0.00839477740996},
     {0.00839477740996, 0.72849239295540}};
+// (xi1, xi2, xi3, w) with xi3 = (1 - xi2) - xi1 as the points are formed, and
+// the weight in FP32
+struct TriPoint { double x1, x2, x3, w; float wf, pad; };
+constexpr TriPoint tri_point(double x1, double x2, double w)
+{
+    return TriPoint{x1, x2, (1.0 - x2) - x1, w, (float)w, 0.0f};
+}
+__constant__ static const TriPoint kTri16[16] = {
+    tri_point(0.33333333333333, 0.33333333333333, 0.14431560767779),
+    tri_point(0.45929258829272, 0.45929258829272, 0.09509163426728),
+    tri_point(0.45929258829272, 0.08141482341455, 0.09509163426728),
+    tri_point(0.08141482341455, 0.45929258829272, 0.09509163426728),
+    tri_point(0.17056930775176, 0.17056930775176, 0.10321737053472),
+    tri_point(0.17056930775176, 0.65886138449648, 0.10321737053472),
+    tri_point(0.65886138449648, 0.17056930775176, 0.10321737053472),
+    tri_point(0.05054722831703, 0.05054722831703, 0.03245849762320),
+    tri_point(0.05054722831703, 0.89890554336594, 0.03245849762320),
+    tri_point(0.89890554336594, 0.05054722831703, 0.03245849762320),
+    tri_point(0.26311282963464, 0.72849239295540, 0.02723031417443),
+    tri_point(0.72849239295540, 0.00839477740996, 0.02723031417443),
+    tri_point(0.00839477740996, 0.26311282963464, 0.02723031417443),
+    tri_point(0.72849239295540, 0.26311282963464, 0.02723031417443),
+    tri_point(0.26311282963464, 0.00839477740996, 0.02723031417443),
+    tri_point(0.00839477740996, 0.72849239295540, 0.02723031417443)};
 // 5-point Gauss-Legendre (linequadraturerules.cpp:63-86)
 __constant__ static const double kGL5X[5] = {-0.906179845938664, -0.5384693101056831, 0.0, 0.5384693101056831,
                                              0.906179845938664};
@@ -72,6 +96,125 @@ struct DevFreq {
     const bem_c64* cphi;
     const bem_c64* cd;
 };
+
+// r = sqrt(rr) and 1 / r, both correctly rounded, from one reciprocal square
+// root: the square root by the Goldschmidt steps the compiler's own FP64
+// square root takes (without its scaling of arguments below 2^-767, squared
+// distances of elements are far above), then two Newton steps of the
+// reciprocal from the by-product h = 1 / (2 r).  The second starts within one
+// unit in the last place, and its exact residual makes the result correctly
+// rounded unless all significand bits of r are ones (Markstein, IBM J. Res.
+// Dev. 34, 1990): then the steps end on the power of two one unit below, and
+// the unit is set at the end (meshes with straight sides do give distances
+// one unit below 1).  20 operations instead of the 27, one of them a second
+// quarter-rate one, of a scaled square root and a division, in the same bits.
+__device__ __forceinline__ void sqrt_rcp(double rr, double* r_out, double* inv_out)
+{
+    const double y = __builtin_amdgcn_rsq(rr);
+    double h = 0.5 * y, g = rr * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, rr), h, g);
+    g = fma(fma(-g, g, rr), h, g);
+    union { double d; uint32_t w[2]; } v, u;
+    v.d = h + h;
+    v.d = fma(v.d, fma(-g, v.d, 1.0), v.d);
+    v.d = fma(v.d, fma(-g, v.d, 1.0), v.d);
+    u.d = g;
+    v.w[0] = ((u.w[1] | 0xFFF00000u) & u.w[0]) == 0xFFFFFFFFu ? 1u : v.w[0];
+    *r_out = g;
+    *inv_out = v.d;
+}
+
+// the coefficients of det_sincos (bem_detmath.h) as memory, so that they are
+// scalar operands of the polynomial steps instead of copies into the
+// accumulating register before each
+__constant__ static const double kSinCos[16] = {
+    2.8114572543455206e-15, -7.647163731819816e-13, 1.6059043836821613e-10, -2.505210838544172e-08,
+    2.7557319223985893e-06, -0.0001984126984126984, 0.008333333333333333, -0.16666666666666666,
+    -1.5619206968586225e-16, 4.779477332387385e-14, -1.1470745597729725e-11, 2.08767569878681e-09,
+    -2.755731922398589e-07, 2.48015873015873e-05, -0.001388888888888889, 0.041666666666666664};
+
+// x * y + c with the addend c in scalar registers (one instruction)
+__device__ __forceinline__ double fma_s(double x, double y, double c)
+{
+    double d;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(x), "v"(y), "s"(c));
+    return d;
+}
+
+// det_sincos, the same operations
+__device__ __forceinline__ void dev_sincos(const double* t, double x, double* s_out, double* c_out)
+{
+    const double n = rint(x * BEM_2_OVER_PI);
+    double y = fma(-n, BEM_PIO2_1, x);
+    y = fma(-n, BEM_PIO2_2, y);
+    y = fma(-n, BEM_PIO2_3, y);
+    const double z = y * y;
+    double ps = t[0], pc = t[8];
+#pragma unroll
+    for (int i = 1; i < 8; i++) {
+        ps = fma_s(ps, z, t[i]);
+        pc = fma_s(pc, z, t[8 + i]);
+    }
+    const double s = fma(y * z, ps, y);
+    const double hz = 0.5 * z;
+    const double w = 1.0 - hz;
+    const double c = w + (((1.0 - w) - hz) + (z * z) * pc);
+    const int q = (int)n;
+    union { double d; uint64_t u; } so, co;
+    so.d = (q & 1) ? c : s;
+    co.d = (q & 1) ? -s : c;
+    const uint64_t flip = (uint64_t)(q & 2) << 62;
+    so.u ^= flip;
+    co.u ^= flip;
+    *s_out = so.d;
+    *c_out = co.d;
+}
+
+// bem_point_accumulate with R = p - q given and only the operators of X
+// (L, Mt; NEED & 1) and Y (M, N; NEED & 2): each operator gets the same
+// operations, the others keep their value
+template <int NEED>
+__device__ __forceinline__ void point_ops(bem_ops4* acc, const double* t, double k, double Rx, double Ry, double Rz,
+                                          double npx, double npy, double npz, double nqx, double nqy, double nqz,
+                                          double upnq, double w)
+{
+    const double rr = fma(Rz, Rz, fma(Ry, Ry, Rx * Rx));
+    double r, inv_r, s, c;
+    sqrt_rcp(rr, &r, &inv_r);
+    const double rnp = fma(Rz, npz, fma(Ry, npy, Rx * npx)) * inv_r;
+    const double kr = k * r;
+    dev_sincos(t, kr, &s, &c);
+    const double g = inv_r * BEM_INV_4PI;
+    const double Gre = c * g, Gim = s * g;
+    const double Grre = Gre * inv_r, Grim = Gim * inv_r;
+    const double dGre = fma(-Grim, kr, -Grre);
+    const double dGim = fma(Grre, kr, -Grim);
+    if (NEED & 1) {
+        acc->L.re = fma(w, Gre, acc->L.re);
+        acc->L.im = fma(w, Gim, acc->L.im);
+        acc->Mt.re = fma(w, dGre * rnp, acc->Mt.re);
+        acc->Mt.im = fma(w, dGim * rnp, acc->Mt.im);
+    }
+    if (NEED & 2) {
+        const double rnq = -fma(Rz, nqz, fma(Ry, nqy, Rx * nqx)) * inv_r;
+        const double Grrre = Grre * inv_r, Grrim = Grim * inv_r;
+        const double a = fma(-kr, kr, 2.0);
+        const double b = -2.0 * kr;
+        const double d2Gre = fma(Grrre, a, -(Grrim * b));
+        const double d2Gim = fma(Grrre, b, Grrim * a);
+        const double pp = rnp * rnq;
+        const double tt = -(upnq + pp) * inv_r;
+        const double Nre = fma(dGre, tt, d2Gre * pp);
+        const double Nim = fma(dGim, tt, d2Gim * pp);
+        acc->M.re = fma(w, dGre * rnq, acc->M.re);
+        acc->M.im = fma(w, dGim * rnq, acc->M.im);
+        acc->N.re = fma(w, Nre, acc->N.re);
+        acc->N.im = fma(w, Nim, acc->N.im);
+    }
+}
 
 // regular branch of BemOperatorsConst (boundaryelementsolver.cpp:856-893);
 // quadrature points read with stride qs from qx/qy/qz
@@ -133,6 +276,36 @@ __device__ __forceinline__ bem_ops4 regular_ops_vtx(double k, double px, double 
     o.M = c64_scale(o.M, area);
     o.Mt = c64_scale(o.Mt, area);
     o.N = c64_scale(o.N, area);
+    return o;
+}
+
+// regular_ops_vtx with only the operators that NEED names
+template <int NEED, int UNROLL>
+__device__ __forceinline__ bem_ops4 regular_ops_need(double k, double px, double py, double pz, double npx,
+                                                     double npy, double npz, double nqx, double nqy, double nqz,
+                                                     double area, const ElemVtx& e)
+{
+    const double upnq = fma(npz, nqz, fma(npy, nqy, npx * nqx));
+    bem_ops4 o = bem_ops4_zero();
+    double t[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) t[i] = kSinCos[i];
+#pragma unroll UNROLL
+    for (int q = 0; q < 16; q++) {
+        const TriPoint T = kTri16[q];
+        const double qx = (T.x1 * e.ax + T.x2 * e.bx) + T.x3 * e.cx;
+        const double qy = (T.x1 * e.ay + T.x2 * e.by) + T.x3 * e.cy;
+        const double qz = (T.x1 * e.az + T.x2 * e.bz) + T.x3 * e.cz;
+        point_ops<NEED>(&o, t, k, px - qx, py - qy, pz - qz, npx, npy, npz, nqx, nqy, nqz, upnq, T.w);
+    }
+    if (NEED & 1) {
+        o.L = c64_scale(o.L, area);
+        o.Mt = c64_scale(o.Mt, area);
+    }
+    if (NEED & 2) {
+        o.M = c64_scale(o.M, area);
+        o.N = c64_scale(o.N, area);
+    }
     return o;
 }
 
@@ -451,22 +624,45 @@ __device__ __forceinline__ bem_c32f4 regular_ops_f32_edge_of(const DevFreq32& F,
     return o;
 }
 
-template <int UNROLL = 1>
-__device__ __forceinline__ bem_c32f4 regular_ops_f32_edge(const DevFreq32& F, const DevMesh& M, int64_t i, int64_t j,
-                                                          bool needX = true, bool needY = true)
+// which of X and Y an off-diagonal entry of column j uses (bc_entry,
+// bc_entry_f32): Phi takes X (subst) or Y; DPhi takes both, except cd = 0,
+// where the other one is multiplied by zero.  The X bit 1 and the Y bit 2,
+// for all active lanes together: the quadrature then branches on a scalar,
+// and a lane that got both has the same entry.
+template <class C>
+__device__ __forceinline__ int bc_needs(const int32_t* subst, const C* cd, int kind, int64_t j)
 {
-    return regular_ops_f32_edge_of<UNROLL>(F, M, i, j, M.edg, M.nx, M.ny, M.nz, needX, needY);
+    int need = subst[j] ? 1 : 2;
+    if (kind != 0) {
+        const C v = cd[j];
+        need = v.re == 0 && v.im == 0 ? 3 - need : 3;
+    }
+    return (__any(need & 1) ? 1 : 0) | (__any(need & 2) ? 2 : 0);
 }
 
-// which of X and Y an off-diagonal entry of column j uses (bc_entry_f32):
-// Phi takes X (subst) or Y; DPhi takes both, except cd = 0, where the
-// other one is multiplied by zero.  Returns the X bit 1 and the Y bit 2.
-__device__ __forceinline__ int bc_needs_f32(const DevFreq32& F, const int32_t* subst, int kind, int64_t j)
+// regular_ops_f32_edge_of with the operators that NEED names, for a row point
+// p (normal np) and the column's edge form
+template <int NEED, int UNROLL>
+__device__ __forceinline__ bem_c32f4 regular_ops_f32_need(const DevFreq32& F, double dx, double dy, double dz,
+                                                          double ax, double ay, double az, double bx, double by,
+                                                          double bz, float npx, float npy, float npz, float nqx,
+                                                          float nqy, float nqz, float area)
 {
-    if (kind == 0) return subst[j] ? 1 : 2;
-    const bem_c32 cd = F.cd[j];
-    if (cd.re == 0.0f && cd.im == 0.0f) return subst[j] ? 2 : 1;
-    return 3;
+    const float upnq = fmaf(npz, nqz, fmaf(npy, nqy, npx * nqx));
+    bem_c32f4 o;
+    o.L = o.M = o.Mt = o.N = c32(0.0f, 0.0f);
+#pragma unroll UNROLL
+    for (int q = 0; q < 16; q++) {
+        const double x1 = kTri16[q].x1, x2 = kTri16[q].x2;
+        point_accumulate_f32_r(&o, F, fma(-x1, ax, fma(-x2, bx, dx)), fma(-x1, ay, fma(-x2, by, dy)),
+                               fma(-x1, az, fma(-x2, bz, dz)), npx, npy, npz, nqx, nqy, nqz, upnq, kTri16[q].wf,
+                               NEED & 1, NEED & 2);
+    }
+    o.L = c32(o.L.re * area, o.L.im * area);
+    o.M = c32(o.M.re * area, o.M.im * area);
+    o.Mt = c32(o.Mt.re * area, o.Mt.im * area);
+    o.N = c32(o.N.re * area, o.N.im * area);
+    return o;
 }
 
 // the FP32 form of refl_ops (mirror image of element j, edge form)

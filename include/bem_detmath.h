@@ -30,7 +30,8 @@
  * sqrt and division are IEEE correctly rounded on both x86-64 (SSE2) and
  * gfx950 (HIP's default f64 lowering), and fma is exact-then-round on both.
  * The functions below contain nothing else, so the host and the device
- * produce bit-identical results.
+ * produce bit-identical results.  Device code that forms the same values with
+ * fewer instructions (point_ops in bem_kernels.hpp) keeps every rounding.
  */
 #ifndef BEM_DETMATH_H
 #define BEM_DETMATH_H

@@ -157,7 +157,9 @@ int bem_hmat_destroy(bem_hmat_t h);
    unchanged.
    bem_set_aca_schedule: the ACA size-class bounds on m + n for one
    precision (one wavefront up to small_bound, the middle workgroup shape
-   up to huge_bound, the largest above) and, for queue >= 0, whether batched
+   up to huge_bound, the largest above; the few blocks, above 1024 to 4096
+   depending on the launch's total, that would outlast all others run over
+   several workgroups whatever the bounds) and, for queue >= 0, whether batched
    ACA launches run as persistent workgroups that take items from a device
    counter (1) or one workgroup per item (0).  Results do not depend on it. */
 int bem_assemble_batch(bem_ctx_t ctx, int kind, int64_t nf, const double* kcc3, double aca_tol, int64_t max_rank,
@@ -200,7 +202,7 @@ int bem_block_download(bem_hmat_t h, int64_t b, double* full_or_U, double* alpha
    wall clock), [5] blocks re-run after rank-capacity overflow, [6] device ms
    of the singular, dense and first ACA pass, [7] device ms of the re-run and
    the packing, [8] device bytes the H-matrix holds (when no block
-   overflowed, the first ACA pass's storage at its capacity of 48 per block
+   overflowed, the first ACA pass's storage at its capacity of 48 (up to 96) per block
    is kept as is, so this exceeds [3]) */
 int bem_hmat_stats(bem_hmat_t h, double* stats9);
 
