@@ -104,6 +104,7 @@ struct TilePairs {
     }
 };
 
+constexpr int kDenseUnroll = 2;   // quadrature points whose dependent chains overlap
 // Dense near-field tiles (K1): regular quadrature of every (row, col) pair of
 // a 64 x 64 tile with the row and column data staged in LDS.  Self and
 // near-singular pairs are skipped here and written by k_fixup.  The
@@ -153,8 +154,17 @@ __global__ __launch_bounds__(kWG, PLANE ? 1 : 4) void k_dense(DevMesh M, DevFreq
         const double npx = srow[3][r], npy = srow[4][r], npz = srow[5][r];
         double dx = px - sp[0][c], dy = py - sp[1][c], dz = pz - sp[2][c];
         if (i == j || sqrt(fma(dz, dz, fma(dy, dy, dx * dx))) < M.near_lim) continue;
-        bem_ops4 o = regular_ops(F.k, px, py, pz, npx, npy, npz, sn[0][c], sn[1][c], sn[2][c], sa[c], &sq[0][0][c],
-                                 &sq[1][0][c], &sq[2][0][c], kTile);
+        const int need = (outPhi ? bc_needs(F.subst, F.cd, BEM_KIND_PHI, j) : 0) |
+                         (outDPhi ? bc_needs(F.subst, F.cd, BEM_KIND_DPHI, j) : 0);
+        bem_ops4 o;
+        auto ops = [&](auto N) {
+            o = regular_ops_pts<decltype(N)::value, kDenseUnroll>(F.k, px, py, pz, npx, npy, npz, sn[0][c], sn[1][c],
+                                                                  sn[2][c], sa[c], &sq[0][0][c], &sq[1][0][c],
+                                                                  &sq[2][0][c], kTile);
+        };
+        if (need == 1) ops(std::integral_constant<int, 1>());
+        else if (need == 2) ops(std::integral_constant<int, 2>());
+        else ops(std::integral_constant<int, 3>());
         bem_c64 X, Y;
         bem_xy(&o, F.cc, 0, &X, &Y);
         int64_t d = T.dest + r + (int64_t)c * T.ld;
@@ -162,7 +172,8 @@ __global__ __launch_bounds__(kWG, PLANE ? 1 : 4) void k_dense(DevMesh M, DevFreq
         bem_c64 ed = bem_dphi_entry(X, Y, F.subst[j], F.cd[j]);
         if (PLANE) {   // impedance plane: + the mirror image's entry (refl_xy on the staged image)
             const ElemVtx e{rv[0][c], rv[1][c], rv[2][c], rv[3][c], rv[4][c], rv[5][c], rv[6][c], rv[7][c], rv[8][c]};
-            bem_ops4 ro = regular_ops_vtx<1>(F.k, px, py, pz, npx, npy, npz, rn[0][c], rn[1][c], rn[2][c], sa[c], e);
+            const bem_ops4 ro = regular_ops_need<3, 1>(F.k, px, py, pz, npx, npy, npz, rn[0][c], rn[1][c], rn[2][c],
+                                                       sa[c], e);
             bem_xy(&ro, F.cc, 0, &X, &Y);
             ep = c64_add(ep, bem_phi_entry(X, Y, F.subst[j], F.cphi[j]));
             ed = c64_add(ed, bem_dphi_entry(X, Y, F.subst[j], F.cd[j]));
@@ -312,33 +323,47 @@ __global__ void k_entries(DevMesh M, DevFreq F, int mode, int64_t np, const int6
 __constant__ static const double kTri7[7][3] = BEM_TRI7;
 constexpr int64_t kFieldChunk = 1024;   // boundary elements per partial sum of the field
 
+// The 7 points of kTile elements from column j0 on (cnt of them, vertices vtx),
+// coordinate d of point q in sq[3 q + d], formed as the element rule forms
+// them.  A wavefront evaluates one element at a time for 64 observation
+// points, so the points are the same in every lane: formed here once per
+// tile, not by every lane for every pair (15 of some 90 operations).
+__device__ __forceinline__ void stage_field_points(const double* __restrict__ vtx, int64_t n, int64_t j0, int cnt,
+                                                   double (*sq)[kTile])
+{
+    for (int idx = threadIdx.x; idx < 21 * kTile; idx += kWG) {
+        const int c = idx % kTile, d = (idx / kTile) % 3, q = idx / (3 * kTile);
+        if (c >= cnt) continue;
+        const double* v = vtx + d * n + j0 + c;
+        const double x1 = kTri7[q][0], x2 = kTri7[q][1];
+        const double x3 = (1.0 - x2) - x1;
+        sq[3 * q + d][c] = (x1 * v[0] + x2 * v[3 * n]) + x3 * v[6 * n];
+    }
+}
+
 // L and M of one element for the observation point p (BemOperatorField,
-// boundaryelementsolver.cpp:2319-2353; vertices and normal from LDS column c)
-__device__ __forceinline__ void field_ops(double k, double px, double py, double pz, const double (*sv)[kTile],
-                                          const double (*sn)[kTile], int c, double area, bem_c64* L, bem_c64* Mk)
+// boundaryelementsolver.cpp:2319-2353; points and normal from LDS column c)
+__device__ __forceinline__ void field_ops(const SinCosCoef& t, double k, double px, double py, double pz,
+                                          const double (*sq)[kTile], const double (*sn)[kTile], int c, double area,
+                                          bem_c64* L, bem_c64* Mk)
 {
     *L = c64(0, 0);
     *Mk = c64(0, 0);
 #pragma unroll
-    for (int q = 0; q < 7; q++) {
-        double x1 = kTri7[q][0], x2 = kTri7[q][1];
-        double x3 = (1.0 - x2) - x1;
-        double qx = (x1 * sv[0][c] + x2 * sv[3][c]) + x3 * sv[6][c];
-        double qy = (x1 * sv[1][c] + x2 * sv[4][c]) + x3 * sv[7][c];
-        double qz = (x1 * sv[2][c] + x2 * sv[5][c]) + x3 * sv[8][c];
-        bem_field_point_accumulate(L, Mk, k, px, py, pz, sn[0][c], sn[1][c], sn[2][c], qx, qy, qz, kTri7[q][2]);
-    }
+    for (int q = 0; q < 7; q++)
+        field_point<3>(L, Mk, t, k, px - sq[3 * q][c], py - sq[3 * q + 1][c], pz - sq[3 * q + 2][c], sn[0][c], sn[1][c],
+                       sn[2][c], kTri7[q][2]);
     *L = c64_scale(*L, area);
     *Mk = c64_scale(*Mk, area);
 }
 
 // M phi - L dphi of one element
-__device__ __forceinline__ bem_c64 field_term(double k, double px, double py, double pz, const double (*sv)[kTile],
-                                              const double (*sn)[kTile], int c, double area, bem_c64 phi,
-                                              bem_c64 dphi)
+__device__ __forceinline__ bem_c64 field_term(const SinCosCoef& t, double k, double px, double py, double pz,
+                                              const double (*sq)[kTile], const double (*sn)[kTile], int c, double area,
+                                              bem_c64 phi, bem_c64 dphi)
 {
     bem_c64 L, Mk;
-    field_ops(k, px, py, pz, sv, sn, c, area, &L, &Mk);
+    field_ops(t, k, px, py, pz, sq, sn, c, area, &L, &Mk);
     return bem_field_term(L, Mk, phi, dphi);
 }
 
@@ -349,15 +374,20 @@ __device__ __forceinline__ bem_c64 field_term(double k, double px, double py, do
 // term is followed by its mirror image's (:2305-2311) and the two are added
 // first.  Canonical order: inside a chunk four partial sums over element index
 // mod 4 (ascending), combined (s0 + s1) + (s2 + s3); k_field_reduce adds the
-// chunks in order.
+// chunks in order.  VALU-bound: 433 cycles per wavefront and quadrature point
+// against about 375 of its instructions alone (20011 points x 6300 elements
+// 2.43 ms, 52e9 pairs/s; 3.03 ms with every lane forming the points and a
+// scaled square root and division per point).
+template <bool PLANE>
 __global__ __launch_bounds__(kWG) void k_field(DevMesh M, double k, int64_t nobs, const double* __restrict__ obs,
                                                const bem_c64* __restrict__ phi, const bem_c64* __restrict__ dphi,
                                                int nchunk, bem_c64* __restrict__ part)
 {
-    __shared__ double sv[9][kTile], rv[9][kTile];
-    __shared__ double sn[3][kTile], rn[3][kTile], sa[kTile];
+    __shared__ double sq[21][kTile], rq[PLANE ? 21 : 1][kTile];
+    __shared__ double sn[3][kTile], rn[PLANE ? 3 : 1][kTile], sa[kTile];
     __shared__ bem_c64 sphi[kTile], sdphi[kTile];
     __shared__ bem_c64 red[4][kTile];
+    const SinCosCoef sc = sincos_coef();
     const int tid = threadIdx.x, r = tid & (kTile - 1), cg = tid >> 6;
     const int64_t n = M.n;
     const int64_t i = (int64_t)blockIdx.x * kTile + r;
@@ -369,16 +399,11 @@ __global__ __launch_bounds__(kWG) void k_field(DevMesh M, double k, int64_t nobs
     for (int64_t t0 = j0; t0 < j1; t0 += kTile) {
         const int cnt = (int)(j1 - t0 < kTile ? j1 - t0 : kTile);
         __syncthreads();
-        for (int idx = tid; idx < 9 * kTile; idx += kWG) {
-            int d = idx / kTile, c = idx % kTile;
-            if (c < cnt) {
-                sv[d][c] = M.vtx[(int64_t)d * n + t0 + c];
-                if (M.rvtx) rv[d][c] = M.rvtx[(int64_t)d * n + t0 + c];
-            }
-        }
+        stage_field_points(M.vtx, n, t0, cnt, sq);
+        if constexpr (PLANE) stage_field_points(M.rvtx, n, t0, cnt, rq);
         for (int c = tid; c < cnt; c += kWG) {
             sn[0][c] = M.nx[t0 + c]; sn[1][c] = M.ny[t0 + c]; sn[2][c] = M.nz[t0 + c];
-            if (M.rvtx) { rn[0][c] = M.rnx[t0 + c]; rn[1][c] = M.rny[t0 + c]; rn[2][c] = M.rnz[t0 + c]; }
+            if constexpr (PLANE) { rn[0][c] = M.rnx[t0 + c]; rn[1][c] = M.rny[t0 + c]; rn[2][c] = M.rnz[t0 + c]; }
             sa[c] = M.area[t0 + c];
             sphi[c] = phi[t0 + c];
             sdphi[c] = dphi[t0 + c];
@@ -386,8 +411,8 @@ __global__ __launch_bounds__(kWG) void k_field(DevMesh M, double k, int64_t nobs
         __syncthreads();
         if (!live) continue;
         for (int c = cg; c < cnt; c += 4) {
-            bem_c64 v = field_term(k, px, py, pz, sv, sn, c, sa[c], sphi[c], sdphi[c]);
-            if (M.rvtx) v = c64_add(v, field_term(k, px, py, pz, rv, rn, c, sa[c], sphi[c], sdphi[c]));
+            bem_c64 v = field_term(sc, k, px, py, pz, sq, sn, c, sa[c], sphi[c], sdphi[c]);
+            if constexpr (PLANE) v = c64_add(v, field_term(sc, k, px, py, pz, rq, rn, c, sa[c], sphi[c], sdphi[c]));
             acc = c64_add(acc, v);
         }
     }
@@ -412,17 +437,15 @@ __global__ __launch_bounds__(kWG) void k_field_dense(DevMesh M, double k, int64_
                                                      const bem_c64* __restrict__ phi, const bem_c64* __restrict__ dphi,
                                                      bem_c64* __restrict__ part)
 {
-    __shared__ double sv[9][kTile];
+    __shared__ double sq[21][kTile];
     __shared__ double sn[3][kTile], sa[kTile];
     __shared__ bem_c64 sphi[kTile], sdphi[kTile];
     __shared__ bem_c64 redM[4][kTile], redL[4][kTile];
     const FieldTile T = tiles[blockIdx.x];
     const int tid = threadIdx.x, r = tid & (kTile - 1), cg = tid >> 6;
     const int64_t n = M.n;
-    for (int idx = tid; idx < 9 * kTile; idx += kWG) {
-        int d = idx / kTile, c = idx % kTile;
-        if (c < T.cols) sv[d][c] = M.vtx[(int64_t)d * n + T.col0 + c];
-    }
+    const SinCosCoef sc = sincos_coef();
+    stage_field_points(M.vtx, n, T.col0, T.cols, sq);
     for (int c = tid; c < T.cols; c += kWG) {
         sn[0][c] = M.nx[T.col0 + c]; sn[1][c] = M.ny[T.col0 + c]; sn[2][c] = M.nz[T.col0 + c];
         sa[c] = M.area[T.col0 + c];
@@ -436,7 +459,7 @@ __global__ __launch_bounds__(kWG) void k_field_dense(DevMesh M, double k, int64_
         const double px = obs[i], py = obs[nobs + i], pz = obs[2 * nobs + i];
         for (int c = cg; c < T.cols; c += 4) {
             bem_c64 L, Mk;
-            field_ops(k, px, py, pz, sv, sn, c, sa[c], &L, &Mk);
+            field_ops(sc, k, px, py, pz, sq, sn, c, sa[c], &L, &Mk);
             sM = c64_fma(Mk, sphi[c], sM);
             sL = c64_fma(L, sdphi[c], sL);
         }
@@ -1013,18 +1036,24 @@ __device__ __forceinline__ bool regular_entry(const AcaArgs& a, int64_t i, int64
 __device__ __forceinline__ bem_c64 field_entry(const AcaArgs& a, int64_t i, int64_t j)
 {
     const DevMesh& M = a.M;
-    const int64_t n = M.n;
     const double px = a.obs[i], py = a.obs[a.nobs + i], pz = a.obs[2 * a.nobs + i];
     const double nqx = M.nx[j], nqy = M.ny[j], nqz = M.nz[j];
+    const ElemVtx v = load_vtx(M, j);
+    const SinCosCoef t = sincos_coef();
     bem_c64 L = c64(0, 0), Mk = c64(0, 0);
-    for (int q = 0; q < 7; q++) {
-        double x1 = kTri7[q][0], x2 = kTri7[q][1];
-        double x3 = (1.0 - x2) - x1;
-        double qx = (x1 * M.vtx[j] + x2 * M.vtx[3 * n + j]) + x3 * M.vtx[6 * n + j];
-        double qy = (x1 * M.vtx[n + j] + x2 * M.vtx[4 * n + j]) + x3 * M.vtx[7 * n + j];
-        double qz = (x1 * M.vtx[2 * n + j] + x2 * M.vtx[5 * n + j]) + x3 * M.vtx[8 * n + j];
-        bem_field_point_accumulate(&L, &Mk, a.F.k, px, py, pz, nqx, nqy, nqz, qx, qy, qz, kTri7[q][2]);
-    }
+    auto sum = [&](auto N) {
+#pragma unroll kQuadUnroll
+        for (int q = 0; q < 7; q++) {
+            const double x1 = kTri7[q][0], x2 = kTri7[q][1];
+            const double x3 = (1.0 - x2) - x1;
+            const double qx = (x1 * v.ax + x2 * v.bx) + x3 * v.cx;
+            const double qy = (x1 * v.ay + x2 * v.by) + x3 * v.cy;
+            const double qz = (x1 * v.az + x2 * v.bz) + x3 * v.cz;
+            field_point<decltype(N)::value>(&L, &Mk, t, a.F.k, px - qx, py - qy, pz - qz, nqx, nqy, nqz, kTri7[q][2]);
+        }
+    };
+    if (a.kind == 0) sum(std::integral_constant<int, 1>());
+    else sum(std::integral_constant<int, 2>());
     return c64_scale(a.kind == 0 ? Mk : L, M.area[j]);
 }
 
@@ -7183,7 +7212,7 @@ int bem_field(bem_ctx_t c, int64_t nobs, const double* obs3, const void* phi, co
     if ((rc = dalloc(c, &d_out, (size_t)nobs, &own))) { free_list(c, own); return rc; }
     {
         Timer t(c, 6);
-        hipLaunchKernelGGL(k_field, dim3(nblk(nobs, kTile), nchunk), dim3(kWG), 0, c->stream, c->mesh, c->k, nobs,
+        hipLaunchKernelGGL(c->mesh.rvtx ? k_field<true> : k_field<false>, dim3(nblk(nobs, kTile), nchunk), dim3(kWG), 0, c->stream, c->mesh, c->k, nobs,
                            d_obs, (const bem_c64*)phi, (const bem_c64*)dphi, nchunk, d_part);
     }
     hipLaunchKernelGGL(k_field_reduce, dim3(nblk(nobs, 256)), dim3(256), 0, c->stream, nobs, nchunk, d_part, d_out);
@@ -7211,7 +7240,7 @@ int bem_field_noalloc(bem_ctx_t c, int64_t nobs, const double* obs_dev, const vo
                                            std::to_string(cap) + " (32 MiB)");
     HIPC(c, hipSetDevice(c->device));
     bem_c64* part = (bem_c64*)c->scratch_dev;
-    hipLaunchKernelGGL(k_field, dim3(nblk(nobs, kTile), (unsigned)nchunk), dim3(kWG), 0, c->stream, c->mesh, c->k,
+    hipLaunchKernelGGL(c->mesh.rvtx ? k_field<true> : k_field<false>, dim3(nblk(nobs, kTile), (unsigned)nchunk), dim3(kWG), 0, c->stream, c->mesh, c->k,
                        nobs, obs_dev, (const bem_c64*)phi, (const bem_c64*)dphi, (int)nchunk, part);
     hipLaunchKernelGGL(k_field_reduce, dim3(nblk(nobs, 256)), dim3(256), 0, c->stream, nobs, (int)nchunk, part,
                        (bem_c64*)out_dev);

@@ -136,6 +136,15 @@ __constant__ static const double kSinCos[16] = {
     -1.5619206968586225e-16, 4.779477332387385e-14, -1.1470745597729725e-11, 2.08767569878681e-09,
     -2.755731922398589e-07, 2.48015873015873e-05, -0.001388888888888889, 0.041666666666666664};
 
+struct SinCosCoef { double t[16]; };
+__device__ __forceinline__ SinCosCoef sincos_coef()
+{
+    SinCosCoef c;
+#pragma unroll
+    for (int i = 0; i < 16; i++) c.t[i] = kSinCos[i];
+    return c;
+}
+
 // x * y + c with the addend c in scalar registers (one instruction)
 __device__ __forceinline__ double fma_s(double x, double y, double c)
 {
@@ -145,8 +154,9 @@ __device__ __forceinline__ double fma_s(double x, double y, double c)
 }
 
 // det_sincos, the same operations
-__device__ __forceinline__ void dev_sincos(const double* t, double x, double* s_out, double* c_out)
+__device__ __forceinline__ void dev_sincos(const SinCosCoef& C, double x, double* s_out, double* c_out)
 {
+    const double* t = C.t;
     const double n = rint(x * BEM_2_OVER_PI);
     double y = fma(-n, BEM_PIO2_1, x);
     y = fma(-n, BEM_PIO2_2, y);
@@ -177,7 +187,7 @@ __device__ __forceinline__ void dev_sincos(const double* t, double x, double* s_
 // (L, Mt; NEED & 1) and Y (M, N; NEED & 2): each operator gets the same
 // operations, the others keep their value
 template <int NEED>
-__device__ __forceinline__ void point_ops(bem_ops4* acc, const double* t, double k, double Rx, double Ry, double Rz,
+__device__ __forceinline__ void point_ops(bem_ops4* acc, const SinCosCoef& t, double k, double Rx, double Ry, double Rz,
                                           double npx, double npy, double npz, double nqx, double nqy, double nqz,
                                           double upnq, double w)
 {
@@ -216,23 +226,56 @@ __device__ __forceinline__ void point_ops(bem_ops4* acc, const double* t, double
     }
 }
 
-// regular branch of BemOperatorsConst (boundaryelementsolver.cpp:856-893);
-// quadrature points read with stride qs from qx/qy/qz
-template <int UNROLL = 2>
-__device__ __forceinline__ bem_ops4 regular_ops(double k, double px, double py, double pz, double npx, double npy,
-                                                double npz, double nqx, double nqy, double nqz, double area,
-                                                const double* qx, const double* qy, const double* qz, int64_t qs)
+// bem_field_point_accumulate with the point given; NEED & 1 the M kernel,
+// NEED & 2 the L kernel, each with the same operations
+template <int NEED>
+__device__ __forceinline__ void field_point(bem_c64* L, bem_c64* M, const SinCosCoef& t, double k, double Rx, double Ry,
+                                            double Rz, double nqx, double nqy, double nqz, double w)
 {
-    double upnq = fma(npz, nqz, fma(npy, nqy, npx * nqx));
+    const double rr = fma(Rz, Rz, fma(Ry, Ry, Rx * Rx));
+    double r, inv_r, s, c;
+    sqrt_rcp(rr, &r, &inv_r);
+    const double kr = k * r;
+    dev_sincos(t, kr, &s, &c);
+    const double g = inv_r * BEM_INV_4PI;
+    const double Gre = c * g, Gim = s * g;
+    if (NEED & 2) {
+        L->re = fma(w, Gre, L->re);
+        L->im = fma(w, Gim, L->im);
+    }
+    if (NEED & 1) {
+        const double rnq = -fma(Rz, nqz, fma(Ry, nqy, Rx * nqx)) * inv_r;
+        const double Grre = Gre * inv_r, Grim = Gim * inv_r;
+        const double dGre = fma(-Grim, kr, -Grre);
+        const double dGim = fma(Grre, kr, -Grim);
+        M->re = fma(w, dGre * rnq, M->re);
+        M->im = fma(w, dGim * rnq, M->im);
+    }
+}
+
+// regular branch of BemOperatorsConst (boundaryelementsolver.cpp:856-893)
+// with only the operators that NEED names; quadrature points read with
+// stride qs from qx/qy/qz
+template <int NEED, int UNROLL>
+__device__ __forceinline__ bem_ops4 regular_ops_pts(double k, double px, double py, double pz, double npx, double npy,
+                                                    double npz, double nqx, double nqy, double nqz, double area,
+                                                    const double* qx, const double* qy, const double* qz, int64_t qs)
+{
+    const double upnq = fma(npz, nqz, fma(npy, nqy, npx * nqx));
     bem_ops4 o = bem_ops4_zero();
+    const SinCosCoef t = sincos_coef();
 #pragma unroll UNROLL
     for (int q = 0; q < 16; q++)
-        bem_point_accumulate(&o, k, px, py, pz, npx, npy, npz, nqx, nqy, nqz, upnq, qx[q * qs], qy[q * qs],
-                             qz[q * qs], kTriW[q]);
-    o.L = c64_scale(o.L, area);
-    o.M = c64_scale(o.M, area);
-    o.Mt = c64_scale(o.Mt, area);
-    o.N = c64_scale(o.N, area);
+        point_ops<NEED>(&o, t, k, px - qx[q * qs], py - qy[q * qs], pz - qz[q * qs], npx, npy, npz, nqx, nqy, nqz, upnq,
+                        kTri16[q].w);
+    if (NEED & 1) {
+        o.L = c64_scale(o.L, area);
+        o.Mt = c64_scale(o.Mt, area);
+    }
+    if (NEED & 2) {
+        o.M = c64_scale(o.M, area);
+        o.N = c64_scale(o.N, area);
+    }
     return o;
 }
 
@@ -249,37 +292,7 @@ __device__ __forceinline__ ElemVtx load_vtx(const DevMesh& M, int64_t j)
     return ElemVtx{v[0], v[n], v[2 * n], v[3 * n], v[4 * n], v[5 * n], v[6 * n], v[7 * n], v[8 * n]};
 }
 
-__device__ __forceinline__ void quad_point(const ElemVtx& e, int q, double* qx, double* qy, double* qz)
-{
-    double x1 = kTriX[q][0], x2 = kTriX[q][1];
-    double x3 = (1.0 - x2) - x1;
-    *qx = (x1 * e.ax + x2 * e.bx) + x3 * e.cx;
-    *qy = (x1 * e.ay + x2 * e.by) + x3 * e.cy;
-    *qz = (x1 * e.az + x2 * e.bz) + x3 * e.cz;
-}
-
-// regular_ops with the points of element j formed from its vertices
-template <int UNROLL = 1>
-__device__ __forceinline__ bem_ops4 regular_ops_vtx(double k, double px, double py, double pz, double npx,
-                                                    double npy, double npz, double nqx, double nqy, double nqz,
-                                                    double area, const ElemVtx& e)
-{
-    double upnq = fma(npz, nqz, fma(npy, nqy, npx * nqx));
-    bem_ops4 o = bem_ops4_zero();
-#pragma unroll UNROLL
-    for (int q = 0; q < 16; q++) {
-        double qx, qy, qz;
-        quad_point(e, q, &qx, &qy, &qz);
-        bem_point_accumulate(&o, k, px, py, pz, npx, npy, npz, nqx, nqy, nqz, upnq, qx, qy, qz, kTriW[q]);
-    }
-    o.L = c64_scale(o.L, area);
-    o.M = c64_scale(o.M, area);
-    o.Mt = c64_scale(o.Mt, area);
-    o.N = c64_scale(o.N, area);
-    return o;
-}
-
-// regular_ops_vtx with only the operators that NEED names
+// regular_ops_pts with the points of element j formed from its vertices
 template <int NEED, int UNROLL>
 __device__ __forceinline__ bem_ops4 regular_ops_need(double k, double px, double py, double pz, double npx,
                                                      double npy, double npz, double nqx, double nqy, double nqz,
@@ -287,9 +300,7 @@ __device__ __forceinline__ bem_ops4 regular_ops_need(double k, double px, double
 {
     const double upnq = fma(npz, nqz, fma(npy, nqy, npx * nqx));
     bem_ops4 o = bem_ops4_zero();
-    double t[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) t[i] = kSinCos[i];
+    const SinCosCoef t = sincos_coef();
 #pragma unroll UNROLL
     for (int q = 0; q < 16; q++) {
         const TriPoint T = kTri16[q];
@@ -317,6 +328,7 @@ __device__ __noinline__ bem_ops4 near_ops(double k, double px, double py, double
 {
     double upnq = fma(npz, nqz, fma(npy, nqy, npx * nqx));
     bem_ops4 o = bem_ops4_zero();
+    const SinCosCoef sc = sincos_coef();
     for (int s = 0; s < nsub; s++) {
         const double* g = geo + s * kNearSub;
         bem_ops4 t = bem_ops4_zero();
@@ -329,7 +341,7 @@ __device__ __noinline__ bem_ops4 near_ops(double k, double px, double py, double
                 double qy = (g[1] + x * g[4]) + y * g[7];
                 double qz = (g[2] + x * g[5]) + y * g[8];
                 double fw = ((maxR / 2.0 * rs) * kGL5W[ia]) * kGL5W[ib];
-                bem_point_accumulate(&t, k, px, py, pz, npx, npy, npz, nqx, nqy, nqz, upnq, qx, qy, qz, fw);
+                point_ops<3>(&t, sc, k, px - qx, py - qy, pz - qz, npx, npy, npz, nqx, nqy, nqz, upnq, fw);
             }
         }
         double h = g[9];
@@ -396,8 +408,8 @@ __device__ bem_ops4 ops_general(const DevMesh& M, double k, int64_t i, int64_t j
             return near_ops(k, M.px[i], M.py[i], M.pz[i], M.nx[i], M.ny[i], M.nz[i], M.nx[j], M.ny[j], M.nz[j],
                             M.nr_geo + M.nr_off[t], M.nr_nsub[t]);
     }
-    return regular_ops(k, M.px[i], M.py[i], M.pz[i], M.nx[i], M.ny[i], M.nz[i], M.nx[j], M.ny[j], M.nz[j],
-                       M.area[j], M.qx + j, M.qy + j, M.qz + j, M.n);
+    return regular_ops_pts<3, 2>(k, M.px[i], M.py[i], M.pz[i], M.nx[i], M.ny[i], M.nz[i], M.nx[j], M.ny[j], M.nz[j],
+                                 M.area[j], M.qx + j, M.qy + j, M.qz + j, M.n);
 }
 
 // implicitPhiMatrix2 / implicitDPhiMatrix2 (boundaryelementsolver.cpp:2004-2040)
@@ -416,8 +428,8 @@ __device__ __forceinline__ bem_ops4 refl_ops(const DevMesh& M, double k, int64_t
     const double* v = M.rvtx + j;
     const int64_t n = M.n;
     const ElemVtx e{v[0], v[n], v[2 * n], v[3 * n], v[4 * n], v[5 * n], v[6 * n], v[7 * n], v[8 * n]};
-    return regular_ops_vtx<1>(k, M.px[i], M.py[i], M.pz[i], M.nx[i], M.ny[i], M.nz[i], M.rnx[j], M.rny[j], M.rnz[j],
-                              M.area[j], e);
+    return regular_ops_need<3, 1>(k, M.px[i], M.py[i], M.pz[i], M.nx[i], M.ny[i], M.nz[i], M.rnx[j], M.rny[j],
+                                  M.rnz[j], M.area[j], e);
 }
 
 // implicitPhiMatrixReflected / implicitDPhiMatrixReflected
@@ -563,27 +575,6 @@ __device__ __forceinline__ bem_c32f4 regular_ops_f32(const DevFreq32& F, double 
     for (int q = 0; q < 16; q++)
         point_accumulate_f32(&o, F, px, py, pz, npx, npy, npz, nqx, nqy, nqz, upnq, qx[q * qs], qy[q * qs],
                              qz[q * qs], kTriWf[q]);
-    o.L = c32(o.L.re * area, o.L.im * area);
-    o.M = c32(o.M.re * area, o.M.im * area);
-    o.Mt = c32(o.Mt.re * area, o.Mt.im * area);
-    o.N = c32(o.N.re * area, o.N.im * area);
-    return o;
-}
-
-template <int UNROLL = 1>
-__device__ __forceinline__ bem_c32f4 regular_ops_f32_vtx(const DevFreq32& F, double px, double py, double pz,
-                                                         float npx, float npy, float npz, float nqx, float nqy,
-                                                         float nqz, float area, const ElemVtx& e)
-{
-    float upnq = fmaf(npz, nqz, fmaf(npy, nqy, npx * nqx));
-    bem_c32f4 o;
-    o.L = o.M = o.Mt = o.N = c32(0.0f, 0.0f);
-#pragma unroll UNROLL
-    for (int q = 0; q < 16; q++) {
-        double qx, qy, qz;
-        quad_point(e, q, &qx, &qy, &qz);
-        point_accumulate_f32(&o, F, px, py, pz, npx, npy, npz, nqx, nqy, nqz, upnq, qx, qy, qz, kTriWf[q]);
-    }
     o.L = c32(o.L.re * area, o.L.im * area);
     o.M = c32(o.M.re * area, o.M.im * area);
     o.Mt = c32(o.Mt.re * area, o.Mt.im * area);
