@@ -1390,6 +1390,8 @@ struct WideBlk {
     int32_t item;          // list entry of the launch mode (block, frequency item or job item)
     int32_t nmc, nnc;      // chunks of a column and of a row
     int32_t cap;
+    int64_t row0, rows, col0, cols, uoff, voff, aoff;   // the block's, so that one load has them
+    int64_t nearb;         // 0: no self or near-singular pair in the block
     int64_t am_col, am_row;   // the chunks' argmax parts
     int64_t d_col, d_row[2];  // the chunks' dot-product parts, cap + 1 each (rows: of even and odd steps)
 };
@@ -1483,24 +1485,44 @@ __device__ __forceinline__ void wide_line(const AcaArgs& a, int64_t r0, int64_t 
     }
 }
 
-// totals of the chunks' dot-product parts (nch chunks of stride cap + 1) in
-// chunk order, r + 1 values into out
-__device__ __forceinline__ void wide_totals(const bem_c64* part, int nch, int cap, int r, bem_c64* out)
+// Totals of the chunks' dot-product parts (chunks of stride cap + 1), r + 1
+// values of the column's and the row's into `col` and `row` (LDS).  The
+// chunks are dealt to groups of threads, a thread per value in each, so that
+// the loads run side by side (one thread per value took 8 us of a step at 35
+// chunks); the groups' sums are added in group order.  `red`: two doubles per
+// thread.  A barrier is left to the caller.
+__device__ __forceinline__ void wide_totals(const bem_c64* pc, int nc, const bem_c64* pr, int nr, int cap, int r,
+                                            double* red, bem_c64* col, bem_c64* row)
 {
-    for (int k = threadIdx.x; k < 2 * (r + 1); k += kWideChunk) {
-        const double* p = (const double*)part + k;
-        const int64_t ld = 2 * (int64_t)(cap + 1);
-        double s = 0.0;
-        int q = 0;
-        for (; q + 8 <= nch; q += 8) {
-            double v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = p[(q + u) * ld];
-#pragma unroll
-            for (int u = 0; u < 8; u++) s = s + v[u];
+    const int nv = 2 * (r + 1), tid = threadIdx.x;
+    const int64_t ld = 2 * (int64_t)(cap + 1);
+    if (nv > kWideChunk) {
+        for (int k = tid; k < nv; k += kWideChunk) {
+            double x = 0.0, y = 0.0;
+            for (int q = 0; q < nc; q++) x = x + ((const double*)pc)[q * ld + k];
+            for (int q = 0; q < nr; q++) y = y + ((const double*)pr)[q * ld + k];
+            ((double*)col)[k] = x;
+            ((double*)row)[k] = y;
         }
-        for (; q < nch; q++) s = s + p[q * ld];
-        ((double*)out)[k] = s;
+        return;
+    }
+    const int lg = 32 - __builtin_clz(nv - 1);   // values rounded up to a power of two
+    const int k = tid & ((1 << lg) - 1), g = tid >> lg, ng = kWideChunk >> lg;
+    double x = 0.0, y = 0.0;
+    if (k < nv) {
+#pragma unroll 4
+        for (int q = g; q < nc; q += ng) x = x + ((const double*)pc)[q * ld + k];
+#pragma unroll 4
+        for (int q = g; q < nr; q += ng) y = y + ((const double*)pr)[q * ld + k];
+    }
+    red[tid] = x;
+    red[kWideChunk + tid] = y;
+    __syncthreads();
+    for (int t = tid; t < 2 * nv; t += kWideChunk) {
+        const int side = t >= nv, v = side ? t - nv : t;
+        double z = red[side * kWideChunk + v];
+        for (int q = 1; q < ng; q++) z = z + red[side * kWideChunk + (q << lg) + v];
+        ((double*)(side ? row : col))[v] = z;
     }
 }
 
@@ -1513,6 +1535,7 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
     extern __shared__ __attribute__((aligned(16))) char dyn[];
     __shared__ ArgMax sred[kWideChunk / 64];
     __shared__ C sv[kWideChunk];
+    __shared__ double red[2 * kWideChunk];
     const WideTask T = w.task[blockIdx.x];
     const WideBlk B = w.blk[T.w];
     WideState s = w.in[T.w];
@@ -1524,14 +1547,14 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
     }
     AcaArgs a = a0;
     const int b = aca_resolve<MODE>(a, a0, B.item);
-    const int64_t m = a.rows[b], n = a.cols[b], r0 = a.row0[b], c0 = a.col0[b];
+    const int64_t m = B.rows, n = B.cols, r0 = B.row0, c0 = B.col0;
     const int cap = B.cap;
-    const bool nearb = !FIELD && (!a.bnear || a.bnear[b] != 0);
+    const bool nearb = !FIELD && B.nearb != 0;
     int64_t maxRank = m < n ? m : n;
     if (a.maxrank > 0 && a.maxrank < maxRank) maxRank = a.maxrank;
-    const C* U = (const C*)a.U + a.uoff[b];
-    C* V = (C*)a.V + a.voff[b];
-    const C* A = (const C*)a.A + a.aoff[b];
+    const C* U = (const C*)a.U + B.uoff;
+    C* V = (C*)a.V + B.voff;
+    const C* A = (const C*)a.A + B.aoff;
     C* sw = (C*)dyn;
     bem_c64* tot = (bem_c64*)(dyn + (((size_t)cap * sizeof(C) + 15) & ~(size_t)15));
     const double tiny2 = kTiny * kTiny, tol2 = a.tol * a.tol;
@@ -1539,11 +1562,10 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
     if (s.phase == kWideStep) {
         const int r = s.r;
         bem_c64 *dc = tot, *dr = tot + cap + 1;
-        wide_totals(w.dots + B.d_col, B.nmc, cap, r, dc);
-        wide_totals(w.dots + (w.odd ? B.d_row[0] : B.d_row[1]), B.nnc, cap, r, dr);
+        const C alpha = ldg(A + r);
+        wide_totals(w.dots + B.d_col, B.nmc, w.dots + (w.odd ? B.d_row[0] : B.d_row[1]), B.nnc, cap, r, red, dc, dr);
         __syncthreads();
         // aca_update_norm: the terms in parallel, added in rank order
-        const C alpha = ldg(A + r);
         const double gain = (cx_abs2(alpha) * dr[0].re) * dc[0].re;
         const bem_c64 ca2 = c64_scale(c64_conj(ld64(&alpha)), 2.0);
         for (int l = tid; l < r; l += kWideChunk)
@@ -1656,12 +1678,12 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_col(AcaArgs a0, WideArgs w)
     }
     AcaArgs a = a0;
     const int b = aca_resolve<MODE>(a, a0, B.item);
-    const int64_t m = a.rows[b], n = a.cols[b], r0 = a.row0[b], c0 = a.col0[b];
+    const int64_t m = B.rows, n = B.cols, r0 = B.row0, c0 = B.col0;
     const int cap = B.cap;
-    const bool nearb = !FIELD && (!a.bnear || a.bnear[b] != 0);
-    C* U = (C*)a.U + a.uoff[b];
-    const C* V = (const C*)a.V + a.voff[b];
-    C* A = (C*)a.A + a.aoff[b];
+    const bool nearb = !FIELD && B.nearb != 0;
+    C* U = (C*)a.U + B.uoff;
+    const C* V = (const C*)a.V + B.voff;
+    C* A = (C*)a.A + B.aoff;
     C* sw = (C*)dyn;
     const double tiny2 = kTiny * kTiny;
     const int r = s.r;
@@ -3296,6 +3318,7 @@ struct bem_ctx {
     // partition
     std::vector<bemsetup::Block> blocks;
     int64_t *d_row0 = nullptr, *d_rows = nullptr, *d_col0 = nullptr, *d_cols = nullptr;
+    std::vector<int8_t> h_bnear;
     int8_t* d_bnear = nullptr;   // per block: may hold self / near-singular pairs (aca_block)
     std::vector<int64_t> dense_off;          // per block (-1 if admissible)
     int64_t dense_total = 0;
@@ -4176,6 +4199,7 @@ int bem_upload_partition(bem_ctx_t c, int64_t nb, const int64_t* row0, const int
     if ((rc = dupload(c, &c->d_rows, rs.data(), nb, ap))) return rc;
     if ((rc = dupload(c, &c->d_col0, c0.data(), nb, ap))) return rc;
     if ((rc = dupload(c, &c->d_cols, cs.data(), nb, ap))) return rc;
+    c->h_bnear = bnear;
     if ((rc = dupload(c, &c->d_bnear, bnear.data(), nb, ap))) return rc;
     if ((rc = dupload(c, &c->d_tiles, c->tiles.data(), c->tiles.size(), ap))) return rc;
     if ((rc = dupload(c, &c->d_fixes, c->fixes.data(), c->fixes.size(), ap))) return rc;
@@ -4375,7 +4399,9 @@ void first_caps(const std::vector<bemsetup::Block>& blocks, const std::vector<in
 // item) and extents
 struct WideSrc {
     int32_t item, cap;
-    int64_t rows, cols;
+    bemsetup::Block B;
+    int64_t uoff, voff, aoff;
+    bool nearb;
 };
 
 // The wide ACA's task lists, states and parts on the device (owned by
@@ -4401,8 +4427,12 @@ int wide_prepare(bem_ctx* c, const std::vector<WideSrc>& src, size_t esz, std::v
         WideBlk& B = blk[q];
         B.item = src[q].item;
         B.cap = src[q].cap;
-        B.nmc = (int32_t)((src[q].rows + kWideChunk - 1) / kWideChunk);
-        B.nnc = (int32_t)((src[q].cols + kWideChunk - 1) / kWideChunk);
+        const auto& X = src[q].B;
+        B.nmc = (int32_t)((X.rows + kWideChunk - 1) / kWideChunk);
+        B.nnc = (int32_t)((X.cols + kWideChunk - 1) / kWideChunk);
+        B.row0 = X.row0; B.rows = X.rows; B.col0 = X.col0; B.cols = X.cols;
+        B.uoff = src[q].uoff; B.voff = src[q].voff; B.aoff = src[q].aoff;
+        B.nearb = src[q].nearb;
         B.am_col = am;
         B.am_row = am + B.nmc;
         am += B.nmc + B.nnc;
@@ -4641,7 +4671,7 @@ int run_aca(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_
     std::vector<WideSrc> ws;
     for (int32_t b : cls[3]) {
         const auto& B = pv ? (*pv->blocks)[b] : c->blocks[b];
-        ws.push_back(WideSrc{b, cap[b], B.rows, B.cols});
+        ws.push_back(WideSrc{b, cap[b], B, S.uoff[b], S.voff[b], S.aoff[b], !pv && c->h_bnear[b] != 0});
     }
     WideRun R;
     if ((rc = wide_prepare(c, ws, f32 ? sizeof(bem_c32) : sizeof(bem_c64), &S.owned, R))) return rc;
@@ -4875,7 +4905,8 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
     std::vector<WideSrc> ws;
     for (int32_t b : cls[3])
         for (int f = 0; f < nf; f++)
-            ws.push_back(WideSrc{(int32_t)(f * nb + b), cap[b], c->blocks[b].rows, c->blocks[b].cols});
+            ws.push_back(WideSrc{(int32_t)(f * nb + b), cap[b], c->blocks[b], uoff[b], voff[b], aoff[b],
+                                 c->h_bnear[b] != 0});
     WideRun R;
     if ((rc = wide_prepare(c, ws, esz, &S[0].owned, R))) return rc;
     Packer pk;
@@ -5558,8 +5589,8 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
     std::vector<WideSrc> ws;
     for (int64_t q = 0; q < nctx; q++)
         for (int32_t b : cls[q][3])
-            ws.push_back(WideSrc{(int32_t)((q << kJobShift) | b), caps[q][b], ctxs[q]->blocks[b].rows,
-                                 ctxs[q]->blocks[b].cols});
+            ws.push_back(WideSrc{(int32_t)((q << kJobShift) | b), caps[q][b], ctxs[q]->blocks[b], S1[q].uoff[b],
+                                 S1[q].voff[b], S1[q].aoff[b], ctxs[q]->h_bnear[b] != 0});
     WideRun R;
     if ((rc = wide_prepare(lead, ws, esz, &lead_own, R))) return fail(rc);
     HIPC(lead, hipEventRecord(lead->ev_fork, lead->stream));
