@@ -1744,155 +1744,254 @@ __global__ __launch_bounds__(kWG) void k_compact(const int32_t* blist, const int
 // Block storage is complex FP64 (bem_c64) or FP32 (bem_c32); products
 // accumulate in FP64 and vectors are FP64 in both cases.
 
-// near-field tiles (K4): partial[tile][row] = sum_c F[row, c] x[c]; the
-// body takes x and the partial vectors with element stride XS (one column
-// of XS interleaved ones)
-template <class S, int XS>
+// The operators' matrices are read once per product, so every kernel here is a
+// stream whose speed is the number of bytes in flight: each load's address
+// comes from one record (LrT, LrU, Tile), several loads of a lane are issued
+// before the first product, and vectors that a whole wavefront shares are
+// read through the scalar cache.  Product with the 20480-triangle operator
+// (FP32 storage, 470 MB) 132 -> 113 us, 4.2 TB/s, with the five extents, offsets
+// and ranks of a task looked up one after the other before its first load.
+
+// the four wavefronts of a workgroup as a scalar
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// values that no workgroup of the running kernel writes, at an address all
+// lanes share: scalar loads
+__device__ __forceinline__ bem_c64 ld_shared(const bem_c64* p)
+{
+    const bem_v2d x = *(const __attribute__((address_space(4))) bem_v2d*)p;
+    return c64(x.x, x.y);
+}
+
+// near-field tiles (K4): partial[tile][row][q] = sum_c F[row, c] x[c][q] for R
+// interleaved columns; wavefront w takes the columns w, w + 4, ..., four
+// loaded together
+template <class S, int R>
 __device__ __forceinline__ void mvm_dense_tile(const Tile& T, const S* __restrict__ F, const bem_c64* __restrict__ x,
                                                bem_c64* __restrict__ part)
 {
-    __shared__ bem_c64 red[4][kTile];
-    const int tid = threadIdx.x, r = tid & (kTile - 1), cg = tid >> 6;
-    bem_c64 acc = c64(0, 0);
+    __shared__ bem_c64 red[4][kTile * R];
+    constexpr int UN = 4;
+    const int tid = threadIdx.x, r = tid & (kTile - 1), cg = wave_id();
+    bem_c64 acc[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) acc[q] = c64(0, 0);
     if (r < T.rows) {
         const S* f = F + T.dest + r;
-        for (int c = cg; c < T.cols; c += 4)
-            acc = c64_fma(ld64(f + (int64_t)c * T.ld), x[(int64_t)(T.col0 + c) * XS], acc);
+        const bem_c64* xs = x + (int64_t)T.col0 * R;
+        int c = cg;
+        for (; c + 4 * (UN - 1) < T.cols; c += 4 * UN) {
+            S v[UN];
+#pragma unroll
+            for (int e = 0; e < UN; e++) v[e] = f[(int64_t)(c + 4 * e) * T.ld];
+#pragma unroll
+            for (int e = 0; e < UN; e++)
+#pragma unroll
+                for (int q = 0; q < R; q++)
+                    acc[q] = c64_fma(ld64(&v[e]), ld_shared(xs + (c + 4 * e) * R + q), acc[q]);
+        }
+        for (; c < T.cols; c += 4) {
+            const bem_c64 v = ld64(f + (int64_t)c * T.ld);
+#pragma unroll
+            for (int q = 0; q < R; q++) acc[q] = c64_fma(v, ld_shared(xs + c * R + q), acc[q]);
+        }
     }
-    red[cg][r] = acc;
+#pragma unroll
+    for (int q = 0; q < R; q++) red[cg][r * R + q] = acc[q];
     __syncthreads();
-    if (cg == 0 && r < T.rows)
-        part[(T.part + r) * XS] = c64_add(c64_add(c64_add(red[0][r], red[1][r]), red[2][r]), red[3][r]);
+    for (int o = tid; o < T.rows * R; o += kWG)
+        part[T.part * R + o] = c64_add(c64_add(c64_add(red[0][o], red[1][o]), red[2][o]), red[3][o]);
 }
 
-template <class S>
+template <class S, int Q>
 __global__ __launch_bounds__(kWG) void k_mvm_dense(const Tile* __restrict__ tiles, const S* __restrict__ F,
                                                    const bem_c64* __restrict__ x, bem_c64* __restrict__ part)
 {
-    mvm_dense_tile<S, 1>(tiles[blockIdx.x], F, x, part);
+    mvm_dense_tile<S, Q>(tiles[blockIdx.x], F, x, part);
 }
 
-// low-rank blocks, phase 1 (K5a): t_b[l] = alpha_l (V_b[l, :] . x_J), one
-// wavefront per (block, l0) task covering rows l0 .. l0 + kLrRows - 1 of V_b.
-// FP64 storage: every row over all 64 lanes (lane-strided sums and the
-// wavefront tree, the order the restatement follows), each x element loaded
-// once for the group.  FP32 storage: 16 lanes per row with four loads in
-// flight per lane and a 16-lane tree (a sixth of the shuffles).
+// One low-rank task of each phase: rows l0 .. of a block's V (phase 1, at
+// most kLrRows; `left` rows from l0 to the rank), 64 rows of a block's U
+// (phase 2)
 constexpr int kLrRows = 4;
-static_assert(kLrRows * 16 == 64, "FP32 k_lr_t: 16 lanes per row");
-// (body with x of element stride XS)
-template <class S, int XS>
-__device__ __forceinline__ void lr_t_task(int64_t task, const int32_t* __restrict__ tasks,
-                                          const int64_t* __restrict__ col0, const int64_t* __restrict__ cols,
-                                          const int32_t* __restrict__ rank, const int64_t* __restrict__ voff,
-                                          const int64_t* __restrict__ aoff, const int64_t* __restrict__ toff,
-                                          const S* __restrict__ V, const S* __restrict__ A,
+constexpr int kLrURows = 64;
+struct LrT {
+    int64_t v, a;          // offsets of row l0 in V and of its alpha
+    int32_t x, n, t;       // first element of x, columns, first t
+    int16_t left, l0;
+};
+struct LrU {
+    int64_t u, p;          // offset of the first row in U and in the partial vectors
+    int32_t ld, k, t, rows;
+};
+static_assert(sizeof(LrT) == 32 && sizeof(LrU) == 32, "one cache line holds four tasks");
+
+// the tasks from their (block, l0) and (block, row chunk) lists
+__global__ void k_lr_tasks(const int32_t* __restrict__ tt, int64_t ntt, const int32_t* __restrict__ ut, int64_t nut,
+                           const int64_t* __restrict__ rows, const int64_t* __restrict__ col0,
+                           const int64_t* __restrict__ cols, const int32_t* __restrict__ rank,
+                           const int64_t* __restrict__ uoff, const int64_t* __restrict__ voff,
+                           const int64_t* __restrict__ aoff, const int64_t* __restrict__ toff,
+                           const int64_t* __restrict__ poff, LrT* T, LrU* U)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < ntt) {
+        const int b = tt[2 * i], l0 = tt[2 * i + 1];
+        LrT t;
+        t.v = voff[b] + l0 * cols[b];
+        t.a = aoff[b] + l0;
+        t.x = (int32_t)col0[b];
+        t.n = (int32_t)cols[b];
+        t.t = (int32_t)(toff[b] + l0);
+        t.left = (int16_t)(rank[b] - l0);
+        t.l0 = (int16_t)l0;
+        T[i] = t;
+    }
+    if (i < nut) {
+        const int b = ut[2 * i];
+        const int64_t r0 = (int64_t)ut[2 * i + 1] * kLrURows;
+        LrU u;
+        u.u = uoff[b] + r0;
+        u.p = poff[b] + r0;
+        u.ld = (int32_t)rows[b];
+        u.k = rank[b];
+        u.t = (int32_t)toff[b];
+        u.rows = (int32_t)(rows[b] - r0 < kLrURows ? rows[b] - r0 : kLrURows);
+        U[i] = u;
+    }
+}
+
+// E adjacent columns of a row, 16 bytes
+template <class S> struct RowLoad;
+template <> struct RowLoad<bem_c32> {
+    static constexpr int E = 2;
+    struct __attribute__((aligned(8))) V { bem_c32 v[2]; };
+};
+template <> struct RowLoad<bem_c64> {
+    static constexpr int E = 1;
+    struct V { bem_c64 v[1]; };
+};
+
+// low-rank blocks, phase 1 (K5a): t[l][q] = alpha_l (V[l, :] . x[:, q]) for R
+// interleaved columns, one wavefront per task, 16 lanes per row; each lane
+// takes 16 bytes of the row at a time, UN of them loaded together, with
+// accumulators of their own
+template <class S, int R>
+__device__ __forceinline__ void lr_t_task(const LrT& T, const S* __restrict__ V, const S* __restrict__ A,
                                           const bem_c64* __restrict__ x, bem_c64* __restrict__ t)
 {
-    const int lane = threadIdx.x & 63;
-    const int b = tasks[2 * task], l0 = tasks[2 * task + 1];
-    const int64_t n = cols[b];
-    const int nl = min(kLrRows, rank[b] - l0);
-    const S* v = V + voff[b] + (int64_t)l0 * n;
-    const bem_c64* xs = x + col0[b] * XS;
-    if constexpr (sizeof(S) == sizeof(bem_c32)) {
-        const int u = lane >> 4, q = lane & 15;   // row l0 + u, columns q, q + 16, ...
-        bem_c64 p = c64(0, 0);
-        if (u < nl) {
-            // four independent accumulators (columns q + 16 e + 64 i in pe[e]),
-            // so that consecutive multiply-adds do not wait on each other
-            const S* vr = v + (int64_t)u * n;
-            bem_c64 pe[4];
+    using L = RowLoad<S>;
+    constexpr int E = L::E, UN = R == 1 ? 4 / E : R == 2 ? 4 / E : R == 4 ? 2 / E : 1;
+    const int lane = threadIdx.x & 63, u = lane >> 4, q = lane & 15;
+    bem_c64 p[R];
 #pragma unroll
-            for (int e = 0; e < 4; e++) pe[e] = c64(0, 0);
-            int64_t j = q;
-            for (; j + 48 < n; j += 64) {
-                S vv[4];
-                bem_c64 xv[4];
+    for (int c = 0; c < R; c++) p[c] = c64(0, 0);
+    bem_c64 al = c64(0, 0);
+    if (u < T.left) {
+        al = ld64(A + T.a + u);
+        const S* vr = V + T.v + (int64_t)u * T.n;
+        const bem_c64* xs = x + (int64_t)T.x * R;
+        const int n = T.n;
+        bem_c64 pe[E * UN][R];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    vv[e] = vr[j + 16 * e];
-                    xv[e] = xs[(j + 16 * e) * XS];
+        for (int e = 0; e < E * UN; e++)
+#pragma unroll
+            for (int c = 0; c < R; c++) pe[e][c] = c64(0, 0);
+        int j = E * q;
+        for (; j + 16 * E * (UN - 1) + E - 1 < n; j += 16 * E * UN) {
+            typename L::V vv[UN];
+#pragma unroll
+            for (int e = 0; e < UN; e++) vv[e] = *(const typename L::V*)(vr + j + 16 * E * e);
+#pragma unroll
+            for (int e = 0; e < UN; e++)
+#pragma unroll
+                for (int d = 0; d < E; d++)
+#pragma unroll
+                    for (int c = 0; c < R; c++)
+                        pe[e * E + d][c] = c64_fma(ld64(&vv[e].v[d]), xs[(int64_t)(j + 16 * E * e + d) * R + c],
+                                                   pe[e * E + d][c]);
+        }
+#pragma unroll
+        for (int e = 0; e < UN; e++)
+#pragma unroll
+            for (int d = 0; d < E; d++) {
+                const int jj = j + 16 * E * e + d;
+                if (jj < n) {
+                    const bem_c64 v = ld64(vr + jj);
+#pragma unroll
+                    for (int c = 0; c < R; c++) pe[e * E + d][c] = c64_fma(v, xs[(int64_t)jj * R + c], pe[e * E + d][c]);
                 }
-#pragma unroll
-                for (int e = 0; e < 4; e++) pe[e] = c64_fma(ld64(&vv[e]), xv[e], pe[e]);
             }
-            // at most three columns are left (j + 48 >= n)
-            if (j < n) pe[0] = c64_fma(ld64(vr + j), xs[j * XS], pe[0]);
-            if (j + 16 < n) pe[1] = c64_fma(ld64(vr + j + 16), xs[(j + 16) * XS], pe[1]);
-            if (j + 32 < n) pe[2] = c64_fma(ld64(vr + j + 32), xs[(j + 32) * XS], pe[2]);
-            p = c64_add(c64_add(pe[0], pe[1]), c64_add(pe[2], pe[3]));
+#pragma unroll
+        for (int c = 0; c < R; c++) {
+            p[c] = pe[0][c];
+#pragma unroll
+            for (int e = 1; e < E * UN; e++) p[c] = c64_add(p[c], pe[e][c]);
         }
+    }
+#pragma unroll
+    for (int c = 0; c < R; c++)
+#pragma unroll
         for (int s = 8; s > 0; s >>= 1) {
-            p.re = p.re + __shfl_xor(p.re, s, 16);
-            p.im = p.im + __shfl_xor(p.im, s, 16);
+            p[c].re = p[c].re + lane_xor(p[c].re, s);
+            p[c].im = p[c].im + lane_xor(p[c].im, s);
         }
-        if (q == 0 && u < nl) t[toff[b] + l0 + u] = c64_mul(ld64(A + aoff[b] + l0 + u), p);
-        return;
-    }
-    bem_c64 p[kLrRows];
+    if (q == 0 && u < T.left) {
 #pragma unroll
-    for (int u = 0; u < kLrRows; u++) p[u] = c64(0, 0);
-    for (int64_t j = lane; j < n; j += 64) {
-        const bem_c64 xv = xs[j * XS];
-#pragma unroll
-        for (int u = 0; u < kLrRows; u++)
-            if (u < nl) p[u] = c64_fma(ld64(v + (int64_t)u * n + j), xv, p[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kLrRows; u++) p[u] = wave_sum(p[u]);
-    if (lane == 0) {   // wave_sum leaves the full sums in lane 0
-#pragma unroll
-        for (int u = 0; u < kLrRows; u++)
-            if (u < nl) t[toff[b] + l0 + u] = c64_mul(ld64(A + aoff[b] + l0 + u), p[u]);
+        for (int c = 0; c < R; c++) t[(int64_t)(T.t + u) * R + c] = c64_mul(al, p[c]);
     }
 }
 
-template <class S>
-__global__ __launch_bounds__(kWG) void k_lr_t(const int32_t* __restrict__ tasks, int64_t ntask,
-                                              const int64_t* __restrict__ col0, const int64_t* __restrict__ cols,
-                                              const int32_t* __restrict__ rank, const int64_t* __restrict__ voff,
-                                              const int64_t* __restrict__ aoff, const int64_t* __restrict__ toff,
-                                              const S* __restrict__ V, const S* __restrict__ A,
-                                              const bem_c64* __restrict__ x, bem_c64* __restrict__ t)
+template <class S, int Q>
+__global__ __launch_bounds__(kWG) void k_lr_t(const LrT* __restrict__ tasks, int64_t ntask, const S* __restrict__ V,
+                                              const S* __restrict__ A, const bem_c64* __restrict__ x,
+                                              bem_c64* __restrict__ t)
 {
-    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + (threadIdx.x >> 6);
+    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + wave_id();
     if (task >= ntask) return;
-    lr_t_task<S, 1>(task, tasks, col0, cols, rank, voff, aoff, toff, V, A, x, t);
+    lr_t_task<S, Q>(tasks[task], V, A, x, t);
 }
 
-// low-rank blocks, phase 2 (K5b): partial_b[i] = sum_l U_b[i, l] t_b[l] over a
-// chunk of kWG rows of one block
-// (body: task `task`, t staged in st, partial vectors of element stride XS)
-template <class S, int XS>
-__device__ __forceinline__ void lr_u_task(int64_t task, const int32_t* __restrict__ tasks,
-                                          const int64_t* __restrict__ rows, const int32_t* __restrict__ rank,
-                                          const int64_t* __restrict__ uoff, const int64_t* __restrict__ toff,
-                                          const int64_t* __restrict__ poff, const S* __restrict__ U,
-                                          const bem_c64* __restrict__ t, bem_c64* st, bem_c64* __restrict__ part)
+// low-rank blocks, phase 2 (K5b): partial[i][q] = sum_l U[i, l] t[l][q] over
+// 64 rows of one block, one wavefront per task, a row per lane
+template <class S, int R>
+__device__ __forceinline__ void lr_u_task(const LrU& T, const S* __restrict__ U, const bem_c64* __restrict__ t,
+                                          bem_c64* __restrict__ part)
 {
-    const int b = tasks[2 * task], chunk = tasks[2 * task + 1];
-    const int64_t m = rows[b];
-    const int k = rank[b];
-    for (int l = threadIdx.x; l < k; l += kWG) st[l] = t[toff[b] + l];
-    __syncthreads();
-    const int64_t i = (int64_t)chunk * kWG + threadIdx.x;
-    if (i >= m) return;
-    const S* u = U + uoff[b] + i;
-    bem_c64 acc = c64(0, 0);
-    for (int l = 0; l < k; l++) acc = c64_fma(ld64(u + (int64_t)l * m), st[l], acc);
-    part[(poff[b] + i) * XS] = acc;
+    constexpr int UN = 4;
+    const int i = threadIdx.x & 63;
+    if (i >= T.rows) return;
+    const S* u = U + T.u + i;
+    const bem_c64* tb = t + (int64_t)T.t * R;
+    bem_c64 acc[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) acc[q] = c64(0, 0);
+    int l = 0;
+    for (; l + UN <= T.k; l += UN) {
+        S v[UN];
+#pragma unroll
+        for (int e = 0; e < UN; e++) v[e] = u[(int64_t)(l + e) * T.ld];
+#pragma unroll
+        for (int e = 0; e < UN; e++)
+#pragma unroll
+            for (int q = 0; q < R; q++) acc[q] = c64_fma(ld64(&v[e]), ld_shared(tb + (l + e) * R + q), acc[q]);
+    }
+    for (; l < T.k; l++) {
+        const bem_c64 v = ld64(u + (int64_t)l * T.ld);
+#pragma unroll
+        for (int q = 0; q < R; q++) acc[q] = c64_fma(v, ld_shared(tb + l * R + q), acc[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < R; q++) part[(T.p + i) * R + q] = acc[q];
 }
 
-template <class S>
-__global__ __launch_bounds__(kWG) void k_lr_u(const int32_t* __restrict__ tasks, const int64_t* __restrict__ rows,
-                                              const int32_t* __restrict__ rank, const int64_t* __restrict__ uoff,
-                                              const int64_t* __restrict__ toff, const int64_t* __restrict__ poff,
-                                              const S* __restrict__ U, const bem_c64* __restrict__ t,
-                                              bem_c64* __restrict__ part)
+template <class S, int Q>
+__global__ __launch_bounds__(kWG) void k_lr_u(const LrU* __restrict__ tasks, int64_t ntask, const S* __restrict__ U,
+                                              const bem_c64* __restrict__ t, bem_c64* __restrict__ part)
 {
-    extern __shared__ bem_c64 st[];
-    lr_u_task<S, 1>(blockIdx.x, tasks, rows, rank, uoff, toff, poff, U, t, st, part);
+    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + wave_id();
+    if (task >= ntask) return;
+    lr_u_task<S, Q>(tasks[task], U, t, part);
 }
 
 // y_i (+)= sum of the partial vectors covering row i in partition order:
@@ -1904,8 +2003,18 @@ __global__ void k_mvm_gather(int64_t n, const int64_t* __restrict__ gptr, const 
     const int64_t i = g >> 4;
     const int q = (int)(g & 15);
     bem_c64 acc = c64(0, 0);
-    if (i < n)
-        for (int64_t p = gptr[i] + q; p < gptr[i + 1]; p += 16) acc = c64_add(acc, part[gidx[p]]);
+    if (i < n) {
+        const int64_t p1 = gptr[i + 1];
+        int64_t p = gptr[i] + q;
+        for (; p + 48 < p1; p += 64) {   // four partials loaded together
+            bem_c64 v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = part[gidx[p + 16 * e]];
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = c64_add(acc, v[e]);
+        }
+        for (; p < p1; p += 16) acc = c64_add(acc, part[gidx[p]]);
+    }
     for (int s = 8; s > 0; s >>= 1) {
         acc.re = acc.re + __shfl_down(acc.re, s, 16);
         acc.im = acc.im + __shfl_down(acc.im, s, 16);
@@ -2649,40 +2758,6 @@ __device__ __forceinline__ void mfma_cstep(bem_c64 a, bem_c64 b, v4d& cr, v4d& c
     ci = mfma_f64(a.im, b.re, ci);
 }
 
-// near-field tiles, Q right-hand sides on the VALU (body: R columns of
-// vectors with XS interleaved ones)
-template <class S, int R, int XS>
-__device__ __forceinline__ void mvm_dense_tile_q(const Tile& T, const S* __restrict__ F,
-                                                 const bem_c64* __restrict__ x, bem_c64* __restrict__ part)
-{
-    __shared__ bem_c64 red[4][kTile * R];
-    const int tid = threadIdx.x, r = tid & (kTile - 1), cg = tid >> 6;
-    bem_c64 acc[R];
-#pragma unroll
-    for (int q = 0; q < R; q++) acc[q] = c64(0, 0);
-    if (r < T.rows) {
-        const S* f = F + T.dest + r;
-        for (int c = cg; c < T.cols; c += 4) {
-            const bem_c64 fv = ld64(f + (int64_t)c * T.ld);
-            const bem_c64* xc = x + (int64_t)(T.col0 + c) * XS;
-#pragma unroll
-            for (int q = 0; q < R; q++) acc[q] = c64_fma(fv, xc[q], acc[q]);
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < R; q++) red[cg][r * R + q] = acc[q];
-    __syncthreads();
-    for (int o = tid; o < T.rows * R; o += kWG)
-        part[(T.part + o / R) * XS + o % R] = c64_add(c64_add(c64_add(red[0][o], red[1][o]), red[2][o]), red[3][o]);
-}
-
-template <class S, int Q>
-__global__ __launch_bounds__(kWG) void k_mvm_dense_q(const Tile* __restrict__ tiles, const S* __restrict__ F,
-                                                     const bem_c64* __restrict__ x, bem_c64* __restrict__ part)
-{
-    mvm_dense_tile_q<S, Q, Q>(tiles[blockIdx.x], F, x, part);
-}
-
 // near-field tiles on the matrix cores: wavefront w takes rows 16 w ..
 // 16 w + 15 of the tile over its columns in K steps of four
 template <class S, int Q>
@@ -2696,6 +2771,7 @@ __global__ __launch_bounds__(kWG) void k_mvm_dense_mfma(const Tile* __restrict__
     const bool rowok = rb + lo < T.rows;
     const S* f = F + T.dest + rb + lo;
     v4d cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+#pragma unroll 4
     for (int kk = 0; kk < T.cols; kk += 4) {
         const int c = kk + kq;
         const bool cok = c < T.cols;
@@ -2712,145 +2788,103 @@ __global__ __launch_bounds__(kWG) void k_mvm_dense_mfma(const Tile* __restrict__
     }
 }
 
-// low-rank phase 1, Q right-hand sides: t_b[l][q] = alpha_l (V_b[l, :] . x_J[:, q]),
-// one wavefront per (block, l0) task of kLrRows rows of V (rows l0 .. l0 + NR - 1
-// per pass, NR = kLrRows / Q rounded up to one).  Body: R columns of x with
-// XS interleaved ones, t with R.
-template <class S, int R, int XS>
-__device__ __forceinline__ void lr_t_task_q(int64_t task, const int32_t* __restrict__ tasks,
-                                            const int64_t* __restrict__ col0, const int64_t* __restrict__ cols,
-                                            const int32_t* __restrict__ rank, const int64_t* __restrict__ voff,
-                                            const int64_t* __restrict__ aoff, const int64_t* __restrict__ toff,
-                                            const S* __restrict__ V, const S* __restrict__ A,
-                                            const bem_c64* __restrict__ x, bem_c64* __restrict__ t)
+// low-rank phase 1 on the matrix cores: 16 rows of a block's V by Q columns,
+// one workgroup per 16 rows (of the 4-row task list the tasks at multiples of
+// 16), its wavefronts taking every fourth 16 columns.  Within those a lane
+// (row lo, group kq) holds the four adjacent columns 4 kq .. 4 kq + 3, the
+// K steps being any order of the columns, so that a row's 16 are read in one
+// piece; x is read once per 16 rows.  (On the VALU every row read all Q
+// columns of x again: 85 us for the 5120-triangle ellipsoid's 51 MB with
+// eight columns, FP64, 22 us here.)
+template <class S, int Q>
+__global__ __launch_bounds__(kWG) void k_lr_t_mfma(const LrT* __restrict__ tasks, const S* __restrict__ V,
+                                                   const S* __restrict__ A, const bem_c64* __restrict__ x,
+                                                   bem_c64* __restrict__ t)
 {
-    constexpr int NR = kLrRows / R > 0 ? kLrRows / R : 1;
-    const int lane = threadIdx.x & 63;
-    const int b = tasks[2 * task], lt = tasks[2 * task + 1];
-    const int64_t n = cols[b];
-    const bem_c64* xs = x + col0[b] * XS;
-    for (int l0 = lt; l0 < lt + kLrRows && l0 < rank[b]; l0 += NR) {
-        const int nl = min(NR, rank[b] - l0);
-        const S* v = V + voff[b] + (int64_t)l0 * n;
-        bem_c64 p[NR][R];
+    const LrT T = tasks[blockIdx.x];
+    if (T.l0 & 15) return;
+    __shared__ double sr[kWG / 64 - 1][64][8];
+    const int lane = threadIdx.x & 63, w = wave_id(), lo = lane & 15, kq = lane >> 4;
+    const int n = T.n;
+    const bool rowok = lo < T.left;
+    const S* vr = V + T.v + (int64_t)(rowok ? lo : 0) * n;
+    const bem_c64* xs = x + (int64_t)T.x * Q;
+    v4d cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+#pragma unroll 2
+    for (int k0 = 16 * w; k0 < n; k0 += 64) {
+        const int c0 = k0 + 4 * kq;
+        S a[4];
+        bem_c64 b[4];
 #pragma unroll
-        for (int u = 0; u < NR; u++)
+        for (int e = 0; e < 4; e++) a[e] = vr[min(c0 + e, n - 1)];
 #pragma unroll
-            for (int q = 0; q < R; q++) p[u][q] = c64(0, 0);
-        for (int64_t j = lane; j < n; j += 64) {
-            bem_c64 xv[R];
+        for (int e = 0; e < 4; e++) b[e] = xs[(int64_t)min(c0 + e, n - 1) * Q + (lo < Q ? lo : 0)];
 #pragma unroll
-            for (int q = 0; q < R; q++) xv[q] = xs[j * XS + q];
-#pragma unroll
-            for (int u = 0; u < NR; u++)
-                if (u < nl) {
-                    const bem_c64 vv = ld64(v + (int64_t)u * n + j);
-#pragma unroll
-                    for (int q = 0; q < R; q++) p[u][q] = c64_fma(vv, xv[q], p[u][q]);
-                }
+        for (int e = 0; e < 4; e++) {
+            const bem_c64 av = rowok && c0 + e < n ? ld64(&a[e]) : c64(0, 0);
+            const bem_c64 bv = lo < Q && c0 + e < n ? b[e] : c64(0, 0);
+            mfma_cstep(av, bv, cr, ci);
         }
+    }
+    if (w > 0) {
 #pragma unroll
-        for (int u = 0; u < NR; u++)
-#pragma unroll
-            for (int q = 0; q < R; q++) p[u][q] = wave_sum(p[u][q]);
-        if (lane == 0) {
-#pragma unroll
-            for (int u = 0; u < NR; u++)
-                if (u < nl) {
-                    const bem_c64 al = ld64(A + aoff[b] + l0 + u);
-#pragma unroll
-                    for (int q = 0; q < R; q++) t[(toff[b] + l0 + u) * R + q] = c64_mul(al, p[u][q]);
-                }
+        for (int e = 0; e < 4; e++) {
+            sr[w - 1][lane][e] = cr[e];
+            sr[w - 1][lane][4 + e] = ci[e];
         }
+    }
+    __syncthreads();
+    if (w > 0 || lo >= Q) return;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        double re = cr[e], im = ci[e];
+        for (int g = 0; g < kWG / 64 - 1; g++) {
+            re = re + sr[g][lane][e];
+            im = im + sr[g][lane][4 + e];
+        }
+        const int row = kq + 4 * e;
+        if (row < T.left) t[(int64_t)(T.t + row) * Q + lo] = c64_mul(ld64(A + T.a + row), c64(re, im));
     }
 }
 
+// low-rank phase 2 on the matrix cores: 64 rows of one block per wavefront as
+// four row tiles that share the columns of t; K = the block's rank in steps
+// of four
 template <class S, int Q>
-__global__ __launch_bounds__(kWG) void k_lr_t_q(const int32_t* __restrict__ tasks, int64_t ntask,
-                                                const int64_t* __restrict__ col0, const int64_t* __restrict__ cols,
-                                                const int32_t* __restrict__ rank, const int64_t* __restrict__ voff,
-                                                const int64_t* __restrict__ aoff, const int64_t* __restrict__ toff,
-                                                const S* __restrict__ V, const S* __restrict__ A,
-                                                const bem_c64* __restrict__ x, bem_c64* __restrict__ t)
-{
-    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + (threadIdx.x >> 6);
-    if (task >= ntask) return;
-    lr_t_task_q<S, Q, Q>(task, tasks, col0, cols, rank, voff, aoff, toff, V, A, x, t);
-}
-
-// low-rank phase 2, Q right-hand sides on the VALU: partial_b[i][q] =
-// sum_l U_b[i, l] t_b[l][q] over a chunk of kWG rows (body: t of R columns,
-// partial vectors with XS interleaved ones)
-template <class S, int R, int XS>
-__device__ __forceinline__ void lr_u_task_q(int64_t task, const int32_t* __restrict__ tasks,
-                                            const int64_t* __restrict__ rows, const int32_t* __restrict__ rank,
-                                            const int64_t* __restrict__ uoff, const int64_t* __restrict__ toff,
-                                            const int64_t* __restrict__ poff, const S* __restrict__ U,
-                                            const bem_c64* __restrict__ t, bem_c64* __restrict__ part)
-{
-    const int b = tasks[2 * task], chunk = tasks[2 * task + 1];
-    const int64_t m = rows[b];
-    const int k = rank[b];
-    const int64_t i = (int64_t)chunk * kWG + threadIdx.x;
-    if (i >= m) return;
-    const S* u = U + uoff[b] + i;
-    const bem_c64* tb = t + toff[b] * R;   // the same k R values for every thread (cached)
-    bem_c64 acc[R];
-#pragma unroll
-    for (int q = 0; q < R; q++) acc[q] = c64(0, 0);
-    for (int l = 0; l < k; l++) {
-        const bem_c64 uv = ld64(u + (int64_t)l * m);
-#pragma unroll
-        for (int q = 0; q < R; q++) acc[q] = c64_fma(uv, tb[l * R + q], acc[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < R; q++) part[(poff[b] + i) * XS + q] = acc[q];
-}
-
-template <class S, int Q>
-__global__ __launch_bounds__(kWG) void k_lr_u_q(const int32_t* __restrict__ tasks, const int64_t* __restrict__ rows,
-                                                const int32_t* __restrict__ rank, const int64_t* __restrict__ uoff,
-                                                const int64_t* __restrict__ toff, const int64_t* __restrict__ poff,
-                                                const S* __restrict__ U, const bem_c64* __restrict__ t,
-                                                bem_c64* __restrict__ part)
-{
-    lr_u_task_q<S, Q, Q>(blockIdx.x, tasks, rows, rank, uoff, toff, poff, U, t, part);
-}
-
-// low-rank phase 2 on the matrix cores: the chunk's kWG rows as 16 row tiles,
-// wavefront w taking tiles w, w + 4, ...; K = the block's rank in steps of four
-template <class S, int Q>
-__global__ __launch_bounds__(kWG) void k_lr_u_mfma(const int32_t* __restrict__ tasks, const int64_t* __restrict__ rows,
-                                                   const int32_t* __restrict__ rank, const int64_t* __restrict__ uoff,
-                                                   const int64_t* __restrict__ toff, const int64_t* __restrict__ poff,
+__global__ __launch_bounds__(kWG) void k_lr_u_mfma(const LrU* __restrict__ tasks, int64_t ntask,
                                                    const S* __restrict__ U, const bem_c64* __restrict__ t,
                                                    bem_c64* __restrict__ part)
 {
-    const int b = tasks[2 * blockIdx.x], chunk = tasks[2 * blockIdx.x + 1];
-    const int64_t m = rows[b];
-    const int k = rank[b];
+    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + wave_id();
+    if (task >= ntask) return;
+    const LrU T = tasks[task];
     const int lane = threadIdx.x & 63, lo = lane & 15, kq = lane >> 4;
-    const S* u = U + uoff[b];
-    const bem_c64* tb = t + toff[b] * Q;
-    for (int tile = threadIdx.x >> 6; tile < kWG / 16; tile += kWG / 64) {
-        const int64_t r0 = (int64_t)chunk * kWG + 16 * tile;
-        if (r0 >= m) break;
-        const bool rowok = r0 + lo < m;
-        v4d cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
-        for (int kk = 0; kk < k; kk += 4) {
-            const int l = kk + kq;
-            const bool lok = l < k;
-            const bem_c64 a = rowok && lok ? ld64(u + (r0 + lo) + (int64_t)l * m) : c64(0, 0);
-            const bem_c64 bb = lo < Q && lok ? tb[l * Q + lo] : c64(0, 0);
-            mfma_cstep(a, bb, cr, ci);
-        }
-        if (lo < Q) {
+    const S* u = U + T.u;
+    const bem_c64* tb = t + (int64_t)T.t * Q;
+    v4d cr[4], ci[4];
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int64_t row = r0 + kq + 4 * v;
-                if (row < m) part[(poff[b] + row) * Q + lo] = c64(cr[v], ci[v]);
+    for (int g = 0; g < 4; g++) {
+        cr[g] = v4d{0, 0, 0, 0};
+        ci[g] = v4d{0, 0, 0, 0};
+    }
+    for (int kk = 0; kk < T.k; kk += 4) {
+        const int l = min(kk + kq, T.k - 1);
+        const bool lok = kk + kq < T.k;
+        S a[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) a[g] = u[(int64_t)l * T.ld + min(16 * g + lo, T.rows - 1)];
+        const bem_c64 b = lok && lo < Q ? tb[l * Q + lo] : c64(0, 0);
+#pragma unroll
+        for (int g = 0; g < 4; g++) mfma_cstep(lok ? ld64(&a[g]) : c64(0, 0), b, cr[g], ci[g]);
+    }
+    if (lo < Q) {
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int row = 16 * g + kq + 4 * e;
+                if (row < T.rows) part[(T.p + row) * Q + lo] = c64(cr[g][e], ci[g][e]);
             }
-        }
     }
 }
 
@@ -2900,11 +2934,9 @@ constexpr int kMaxOps = 8;
 struct OpsArg {
     int32_t pad[kMaxOps];
     const void* F[kMaxOps];                  // near-field storage read
-    const int32_t* tt[kMaxOps];              // phase-1 (block, l0) tasks
-    const int32_t* ut[kMaxOps];              // phase-2 (block, row chunk) tasks
+    const LrT* tt[kMaxOps];                  // phase-1 tasks
+    const LrU* ut[kMaxOps];                  // phase-2 tasks
     int64_t ntt[kMaxOps], nut[kMaxOps];
-    const int32_t* rank[kMaxOps];
-    const int64_t *voff[kMaxOps], *aoff[kMaxOps], *toff[kMaxOps], *uoff[kMaxOps];
     const void *U[kMaxOps], *V[kMaxOps], *A[kMaxOps];
     bem_c64* t[kMaxOps];                     // R columns per operator
     int64_t n, P;                            // rows; partial vector entries per column
@@ -2934,47 +2966,31 @@ __global__ __launch_bounds__(kWG) void k_mvm_dense_ops(const Tile* __restrict__ 
     }
     const S* F = (const S*)O.F[g];
     const bem_c64* x = xg + (int64_t)g * O.n * R;
-    if constexpr (R == 1) mvm_dense_tile<S, 1>(tiles[blockIdx.x], F, x, pg);
-    else mvm_dense_tile_q<S, R, R>(tiles[blockIdx.x], F, x, pg);
+    mvm_dense_tile<S, R>(tiles[blockIdx.x], F, x, pg);
 }
 
 template <class S, int R>
-__global__ __launch_bounds__(kWG) void k_lr_t_ops(OpsArg O, const int64_t* __restrict__ col0,
-                                                  const int64_t* __restrict__ cols, const bem_c64* __restrict__ xg)
+__global__ __launch_bounds__(kWG) void k_lr_t_ops(OpsArg O, const bem_c64* __restrict__ xg)
 {
     const int g = blockIdx.y;
-    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + (threadIdx.x >> 6);
+    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + wave_id();
     if (task >= O.ntt[g]) return;
-    const bem_c64* x = xg + (int64_t)g * O.n * R;
-    if constexpr (R == 1)
-        lr_t_task<S, 1>(task, O.tt[g], col0, cols, O.rank[g], O.voff[g], O.aoff[g], O.toff[g], (const S*)O.V[g],
-                        (const S*)O.A[g], x, O.t[g]);
-    else
-        lr_t_task_q<S, R, R>(task, O.tt[g], col0, cols, O.rank[g], O.voff[g], O.aoff[g], O.toff[g],
-                             (const S*)O.V[g], (const S*)O.A[g], x, O.t[g]);
+    lr_t_task<S, R>(O.tt[g][task], (const S*)O.V[g], (const S*)O.A[g], xg + (int64_t)g * O.n * R, O.t[g]);
 }
 
 template <class S, int R>
-__global__ __launch_bounds__(kWG) void k_lr_u_ops(OpsArg O, const int64_t* __restrict__ rows,
-                                                  const int64_t* __restrict__ poff, bem_c64* __restrict__ part)
+__global__ __launch_bounds__(kWG) void k_lr_u_ops(OpsArg O, bem_c64* __restrict__ part)
 {
-    extern __shared__ bem_c64 st[];
     const int g = blockIdx.y;
-    if ((int64_t)blockIdx.x >= O.nut[g]) return;   // uniform per workgroup
+    const int64_t task = (int64_t)blockIdx.x * (kWG / 64) + wave_id();
+    if (task >= O.nut[g]) return;
     bem_c64* pg = part + (int64_t)g * O.P * R;
+    const LrU T = O.ut[g][task];
     if (O.pad[g]) {
-        const int b = O.ut[g][2 * blockIdx.x], chunk = O.ut[g][2 * blockIdx.x + 1];
-        const int64_t i = (int64_t)chunk * kWG + threadIdx.x;
-        if (i < rows[b])
-            for (int q = 0; q < R; q++) pg[(poff[b] + i) * R + q] = c64(0, 0);
+        for (int o = threadIdx.x & 63; o < T.rows * R; o += 64) pg[T.p * R + o] = c64(0, 0);
         return;
     }
-    if constexpr (R == 1)
-        lr_u_task<S, 1>(blockIdx.x, O.ut[g], rows, O.rank[g], O.uoff[g], O.toff[g], poff, (const S*)O.U[g], O.t[g],
-                        st, pg);
-    else
-        lr_u_task_q<S, R, R>(blockIdx.x, O.ut[g], rows, O.rank[g], O.uoff[g], O.toff[g], poff, (const S*)O.U[g],
-                             O.t[g], pg);
+    lr_u_task<S, R>(T, (const S*)O.U[g], O.t[g], pg);
 }
 
 // y[i Q + g R + r] = sum of operator g's partial vectors covering row i (in
@@ -3431,11 +3447,11 @@ struct bem_hmat {
     int64_t *d_uoff = nullptr, *d_voff = nullptr, *d_aoff = nullptr;
     int32_t* d_rank = nullptr;
     // two-phase low-rank MVM: (block, l) and (block, row chunk) work lists
-    int32_t *d_ttask = nullptr, *d_utask = nullptr;
+    LrT* d_ttask = nullptr;
+    LrU* d_utask = nullptr;
     int64_t nttask = 0, nutask = 0;
     int64_t* d_toff = nullptr;
     bem_c64* d_t = nullptr;
-    int maxrank = 1;
     int64_t t_total = 0;      // sum of the ranks (entries of d_t)
     bem_c64* d_tq = nullptr;  // t vectors of Q right-hand sides (t_total x tq_cap)
     int tq_cap = 0;
@@ -4226,7 +4242,7 @@ int bem_hmat_destroy(bem_hmat_t h)
     (void)hipStreamSynchronize(h->ctx->stream);
     for (hipStream_t t : h->ctx->side) (void)hipStreamSynchronize(t);
     for (void* p : {(void*)h->dense, h->dense64, (void*)h->U, (void*)h->V, (void*)h->A, h->meta, (void*)h->d_t,
-                    (void*)h->d_tq})
+                    (void*)h->d_tq, (void*)h->d_ttask, (void*)h->d_utask})
         pfree(h->ctx, p);
     for (auto* v : {&h->uoff, &h->voff, &h->aoff}) h->ctx->vp.give(*v);
     h->ctx->vp.give(h->rank);
@@ -4758,7 +4774,7 @@ int finish_hmat(bem_ctx* c, bem_hmat* h, bool f32, AcaScratch& S1, AcaScratch& S
     for (int32_t b : c->adm_list) {
         tot += h->rank[b];
         ntt += (h->rank[b] + kLrRows - 1) / kLrRows;
-        nchunks += (c->blocks[b].rows + kWG - 1) / kWG;
+        nchunks += (c->blocks[b].rows + kLrURows - 1) / kLrURows;
     }
     std::vector<int32_t> tt = c->vp.take<int32_t>((size_t)2 * ntt, 0), ut = c->vp.take<int32_t>((size_t)2 * nchunks, 0);
     {
@@ -4767,9 +4783,8 @@ int finish_hmat(bem_ctx* c, bem_hmat* h, bool f32, AcaScratch& S1, AcaScratch& S
             const int r = h->rank[b];
             toff[b] = acc;
             acc += r;
-            h->maxrank = std::max(h->maxrank, r);
             for (int l = 0; l < r; l += kLrRows, pt++) { tt[2 * pt] = b; tt[2 * pt + 1] = l; }
-            const int64_t nq = (c->blocks[b].rows + kWG - 1) / kWG;
+            const int64_t nq = (c->blocks[b].rows + kLrURows - 1) / kLrURows;
             for (int64_t q = 0; q < nq; q++, pu++) { ut[2 * pu] = b; ut[2 * pu + 1] = (int32_t)q; }
         }
     }
@@ -4785,9 +4800,18 @@ int finish_hmat(bem_ctx* c, bem_hmat* h, bool f32, AcaScratch& S1, AcaScratch& S
     if (rc) return rc;
     h->d_uoff = pk.ptr<int64_t>(k_uoff); h->d_voff = pk.ptr<int64_t>(k_voff); h->d_aoff = pk.ptr<int64_t>(k_aoff);
     h->d_rank = pk.ptr<int32_t>(k_rank);
+    if (tot > INT32_MAX) return set_err(c, BEM_ERR_ARG, "bem_assemble: more than 2^31 low-rank terms");
     int32_t* d_srank = pk.ptr<int32_t>(k_srank);
-    h->d_ttask = pk.ptr<int32_t>(k_tt); h->d_utask = pk.ptr<int32_t>(k_ut); h->d_toff = pk.ptr<int64_t>(k_toff);
+    h->d_toff = pk.ptr<int64_t>(k_toff);
     if ((rc = dalloc(c, &h->d_t, tot, nullptr))) return rc;
+    if ((rc = dalloc(c, &h->d_ttask, (size_t)ntt, nullptr))) return rc;
+    if ((rc = dalloc(c, &h->d_utask, (size_t)nchunks, nullptr))) return rc;
+    if (ntt > 0) {
+        hipLaunchKernelGGL(k_lr_tasks, dim3(nblk(std::max(ntt, nchunks), 256)), dim3(256), 0, c->stream,
+                           pk.ptr<int32_t>(k_tt), ntt, pk.ptr<int32_t>(k_ut), nchunks, c->d_rows, c->d_col0, c->d_cols,
+                           h->d_rank, h->d_uoff, h->d_voff, h->d_aoff, h->d_toff, c->d_lr_part, h->d_ttask, h->d_utask);
+        if ((rc = launch_check(c, "k_lr_tasks"))) return rc;
+    }
     auto compact = [&](const std::vector<int32_t>& lst, const int32_t* d_lst, const AcaScratch& Sx) -> int {
         if (lst.empty()) return BEM_OK;
         dim3 g((unsigned)lst.size());
@@ -5782,6 +5806,19 @@ int bem_set_aca_schedule(bem_ctx_t c, int precision, int64_t small_bound, int64_
 
 namespace {
 
+// the low-rank blocks of one H-MVM into the partial vectors
+template <class S>
+int hmvm_lowrank(bem_ctx* c, bem_hmat* h, const bem_c64* xd)
+{
+    if (h->nttask == 0) return BEM_OK;
+    Timer t(c, 4);
+    hipLaunchKernelGGL((k_lr_t<S, 1>), dim3(nblk(h->nttask, kWG / 64)), dim3(kWG), 0, c->stream, h->d_ttask, h->nttask,
+                       (const S*)h->V, (const S*)h->A, xd, h->d_t);
+    hipLaunchKernelGGL((k_lr_u<S, 1>), dim3(nblk(h->nutask, kWG / 64)), dim3(kWG), 0, c->stream, h->d_utask, h->nutask,
+                       (const S*)h->U, h->d_t, c->d_part);
+    return launch_check(c, "k_lr");
+}
+
 // near-field tiles and low-rank blocks of one H-MVM into the partial vectors
 template <class S>
 int hmvm_blocks(bem_ctx* c, bem_hmat* h, const bem_c64* xd)
@@ -5789,21 +5826,11 @@ int hmvm_blocks(bem_ctx* c, bem_hmat* h, const bem_c64* xd)
     int rc;
     if (!c->tiles.empty()) {
         Timer t(c, 3);
-        hipLaunchKernelGGL(k_mvm_dense<S>, dim3((unsigned)c->tiles.size()), dim3(kWG), 0, c->stream, c->d_tiles,
+        hipLaunchKernelGGL((k_mvm_dense<S, 1>), dim3((unsigned)c->tiles.size()), dim3(kWG), 0, c->stream, c->d_tiles,
                            (const S*)h->dense, xd, c->d_part);
         if ((rc = launch_check(c, "k_mvm_dense"))) return rc;
     }
-    if (h->nttask > 0) {
-        Timer t(c, 4);
-        hipLaunchKernelGGL(k_lr_t<S>, dim3(nblk(h->nttask, kWG / 64)), dim3(kWG), 0, c->stream, h->d_ttask,
-                           h->nttask, c->d_col0, c->d_cols, h->d_rank, h->d_voff, h->d_aoff, h->d_toff,
-                           (const S*)h->V, (const S*)h->A, xd, h->d_t);
-        hipLaunchKernelGGL(k_lr_u<S>, dim3((unsigned)h->nutask), dim3(kWG), h->maxrank * sizeof(bem_c64), c->stream,
-                           h->d_utask, c->d_rows, h->d_rank, h->d_uoff, h->d_toff, c->d_lr_part, (const S*)h->U,
-                           h->d_t, c->d_part);
-        if ((rc = launch_check(c, "k_lr"))) return rc;
-    }
-    return BEM_OK;
+    return hmvm_lowrank<S>(c, h, xd);
 }
 
 // The refinement operator of an FP32 H-matrix with a kept FP64 near field:
@@ -5814,21 +5841,11 @@ int hmvm_blocks_near64(bem_ctx* c, bem_hmat* h, const bem_c64* xd)
     int rc;
     if (!c->tiles.empty()) {
         Timer t(c, 3);
-        hipLaunchKernelGGL(k_mvm_dense<bem_c64>, dim3((unsigned)c->tiles.size()), dim3(kWG), 0, c->stream,
+        hipLaunchKernelGGL((k_mvm_dense<bem_c64, 1>), dim3((unsigned)c->tiles.size()), dim3(kWG), 0, c->stream,
                            c->d_tiles, (const bem_c64*)h->dense64, xd, c->d_part);
         if ((rc = launch_check(c, "k_mvm_dense"))) return rc;
     }
-    if (h->nttask > 0) {
-        Timer t(c, 4);
-        hipLaunchKernelGGL(k_lr_t<bem_c32>, dim3(nblk(h->nttask, kWG / 64)), dim3(kWG), 0, c->stream, h->d_ttask,
-                           h->nttask, c->d_col0, c->d_cols, h->d_rank, h->d_voff, h->d_aoff, h->d_toff,
-                           (const bem_c32*)h->V, (const bem_c32*)h->A, xd, h->d_t);
-        hipLaunchKernelGGL(k_lr_u<bem_c32>, dim3((unsigned)h->nutask), dim3(kWG), h->maxrank * sizeof(bem_c64),
-                           c->stream, h->d_utask, c->d_rows, h->d_rank, h->d_uoff, h->d_toff, c->d_lr_part,
-                           (const bem_c32*)h->U, h->d_t, c->d_part);
-        if ((rc = launch_check(c, "k_lr"))) return rc;
-    }
-    return BEM_OK;
+    return hmvm_lowrank<bem_c32>(c, h, xd);
 }
 
 // count complex entries at src (FP64 or FP32 on the device) into FP64 host memory
@@ -6463,34 +6480,26 @@ int hmvm_q(bem_ctx* c, bem_hmat* h, const void* dense, const bem_c64* X, bem_c64
     if (!c->tiles.empty()) {
         Timer t(c, 3);
         const dim3 g((unsigned)c->tiles.size());
-        if (Q == 1)
-            hipLaunchKernelGGL(k_mvm_dense<DS>, g, dim3(kWG), 0, c->stream, c->d_tiles, (const DS*)dense, X, part);
-        else if (mf)
+        if (mf)
             hipLaunchKernelGGL((k_mvm_dense_mfma<DS, Q>), g, dim3(kWG), 0, c->stream, c->d_tiles, (const DS*)dense, X,
                                part);
         else
-            hipLaunchKernelGGL((k_mvm_dense_q<DS, Q>), g, dim3(kWG), 0, c->stream, c->d_tiles, (const DS*)dense, X,
-                               part);
+            hipLaunchKernelGGL((k_mvm_dense<DS, Q>), g, dim3(kWG), 0, c->stream, c->d_tiles, (const DS*)dense, X, part);
         if ((rc = launch_check(c, "k_mvm_dense"))) return rc;
     }
     if (h->nttask > 0) {
         Timer t(c, 4);
-        const dim3 gt(nblk(h->nttask, kWG / 64)), gu((unsigned)h->nutask);
-        if (Q == 1) {
-            hipLaunchKernelGGL(k_lr_t<LS>, gt, dim3(kWG), 0, c->stream, h->d_ttask, h->nttask, c->d_col0, c->d_cols,
-                               h->d_rank, h->d_voff, h->d_aoff, h->d_toff, (const LS*)h->V, (const LS*)h->A, X, tv);
-            hipLaunchKernelGGL(k_lr_u<LS>, gu, dim3(kWG), h->maxrank * sizeof(bem_c64), c->stream, h->d_utask,
-                               c->d_rows, h->d_rank, h->d_uoff, h->d_toff, c->d_lr_part, (const LS*)h->U, tv, part);
+        const dim3 gt(nblk(h->nttask, kWG / 64)), gu(nblk(h->nutask, kWG / 64));
+        if (mf) {
+            hipLaunchKernelGGL((k_lr_t_mfma<LS, Q>), dim3((unsigned)h->nttask), dim3(kWG), 0, c->stream, h->d_ttask,
+                               (const LS*)h->V, (const LS*)h->A, X, tv);
+            hipLaunchKernelGGL((k_lr_u_mfma<LS, Q>), gu, dim3(kWG), 0, c->stream, h->d_utask, h->nutask,
+                               (const LS*)h->U, tv, part);
         } else {
-            hipLaunchKernelGGL((k_lr_t_q<LS, Q>), gt, dim3(kWG), 0, c->stream, h->d_ttask, h->nttask, c->d_col0,
-                               c->d_cols, h->d_rank, h->d_voff, h->d_aoff, h->d_toff, (const LS*)h->V,
+            hipLaunchKernelGGL((k_lr_t<LS, Q>), gt, dim3(kWG), 0, c->stream, h->d_ttask, h->nttask, (const LS*)h->V,
                                (const LS*)h->A, X, tv);
-            if (mf)
-                hipLaunchKernelGGL((k_lr_u_mfma<LS, Q>), gu, dim3(kWG), 0, c->stream, h->d_utask, c->d_rows, h->d_rank,
-                                   h->d_uoff, h->d_toff, c->d_lr_part, (const LS*)h->U, tv, part);
-            else
-                hipLaunchKernelGGL((k_lr_u_q<LS, Q>), gu, dim3(kWG), 0, c->stream, h->d_utask, c->d_rows, h->d_rank,
-                                   h->d_uoff, h->d_toff, c->d_lr_part, (const LS*)h->U, tv, part);
+            hipLaunchKernelGGL((k_lr_u<LS, Q>), gu, dim3(kWG), 0, c->stream, h->d_utask, h->nutask, (const LS*)h->U, tv,
+                               part);
         }
         if ((rc = launch_check(c, "k_lr"))) return rc;
     }
@@ -6543,7 +6552,6 @@ int hmvm_ops(bem_ctx* c, const OpSet& S, const bem_c64* X, bem_c64* Y)
     O.n = c->n;
     O.P = std::max<int64_t>(c->part_total, 1);
     int64_t mtt = 0, mut = 0;
-    int maxrank = 0;
     for (int g = 0; g < G; g++) {
         const bem_hmat* h = S.ops[g];
         O.pad[g] = S.active && (size_t)g >= S.active;
@@ -6552,18 +6560,12 @@ int hmvm_ops(bem_ctx* c, const OpSet& S, const bem_c64* X, bem_c64* Y)
         O.ut[g] = h->d_utask;
         O.ntt[g] = O.pad[g] ? 0 : h->nttask;
         O.nut[g] = h->nutask;
-        O.rank[g] = h->d_rank;
-        O.voff[g] = h->d_voff;
-        O.aoff[g] = h->d_aoff;
-        O.toff[g] = h->d_toff;
-        O.uoff[g] = h->d_uoff;
         O.U[g] = h->U;
         O.V[g] = h->V;
         O.A[g] = h->A;
         O.t[g] = R == 1 ? h->d_t : h->d_tq;
         mtt = std::max(mtt, h->nttask);
         mut = std::max(mut, h->nutask);
-        maxrank = std::max(maxrank, h->maxrank);
     }
     int rc;
     hipLaunchKernelGGL((k_group_cols<R, Q>), dim3(nblk(c->n * Q, 256)), dim3(256), 0, c->stream, c->n, X, c->d_xq);
@@ -6576,10 +6578,8 @@ int hmvm_ops(bem_ctx* c, const OpSet& S, const bem_c64* X, bem_c64* Y)
     if (mut > 0) {
         Timer t(c, 4);
         if (mtt > 0)
-            hipLaunchKernelGGL((k_lr_t_ops<LS, R>), dim3(nblk(mtt, kWG / 64), G), dim3(kWG), 0, c->stream, O,
-                               c->d_col0, c->d_cols, c->d_xq);
-        hipLaunchKernelGGL((k_lr_u_ops<LS, R>), dim3((unsigned)mut, G), dim3(kWG),
-                           R == 1 ? maxrank * sizeof(bem_c64) : 0, c->stream, O, c->d_rows, c->d_lr_part, c->d_partq);
+            hipLaunchKernelGGL((k_lr_t_ops<LS, R>), dim3(nblk(mtt, kWG / 64), G), dim3(kWG), 0, c->stream, O, c->d_xq);
+        hipLaunchKernelGGL((k_lr_u_ops<LS, R>), dim3(nblk(mut, kWG / 64), G), dim3(kWG), 0, c->stream, O, c->d_partq);
         if ((rc = launch_check(c, "k_lr_ops"))) return rc;
     }
     Timer t(c, 5);
