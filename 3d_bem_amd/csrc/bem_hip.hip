@@ -39,9 +39,12 @@ constexpr int kTile = 64;       // dense tile edge
 constexpr int kCapFirst = 48;   // first-pass ACA rank capacity per block
 constexpr int kCapMax = 1016;   // second-pass capacity limit (FP64 LDS: (4 cap + 2) x 16 B <= 64 KiB)
 // ACA workgroup size classes by m + n, per storage precision [FP64, FP32]:
-// up to kSmallBlock one wavefront, up to kHugeBlock kMidThreads, above kHugeThreads
+// up to kSmallBlock one wavefront, up to kHugeBlock kMidThreads, above
+// kHugeThreads; kSmallBlock lower where a launch's blocks total little
+// (aca_bounds)
 constexpr int64_t kSmallBlock[2] = {384, 384};
 constexpr int64_t kHugeBlock[2] = {(int64_t)1 << 40, 2048};
+constexpr int64_t kClassMin = 64, kClassShare = 3200;
 // bounds on the m + n above which a block takes the ACA over several
 // workgroups (wide_bound), and the resident 256-thread workgroups it counts
 constexpr int64_t kWideMin = 1024, kWideMax = 4096, kWideShare = 800;
@@ -3423,9 +3426,10 @@ struct bem_ctx {
     bool use_mfma = true;
     bool use_graphs = true;
     // ACA size classes by m + n per storage precision [FP64, FP32]: up to
-    // cls_small one wavefront, up to cls_huge the middle class, above the
-    // largest; batched assemblies on persistent workgroups (queue counter)
-    int64_t cls_small[2] = {kSmallBlock[0], kSmallBlock[1]};
+    // cls_small (negative: by the launch's total, aca_bounds) one wavefront, up
+    // to cls_huge the middle class, above the largest; batched assemblies on
+    // persistent workgroups (queue counter)
+    int64_t cls_small[2] = {-1, -1};
     int64_t cls_huge[2] = {kHugeBlock[0], kHugeBlock[1]};
     bool aca_queue = false;
     // wide ACA: "a block still works" flags of the last two bursts (pinned
@@ -4375,12 +4379,34 @@ int64_t wide_sum(const std::vector<bemsetup::Block>& blocks, const std::vector<i
     return s;
 }
 
-// ACA class of a block: 0, 1, 2 the workgroup classes (largest first), 3 wide
-int aca_class(const bem_ctx* c, const bemsetup::Block& B, int prec, int64_t wide)
+// The m + n bounds of the size classes for a launch of prec's blocks with
+// total m + n `sum`: one wavefront up to `small`, kMidThreads up to `huge`,
+// kHugeThreads up to `wide`, several workgroups above.  While the chip has
+// blocks for all its wavefronts, one wavefront per block gives the higher
+// rate and `small` is kSmallBlock.  With less in total the longest pivot chain
+// decides, and blocks whose line takes one wavefront more passes than the
+// others' get more threads: `small` falls with sum / kClassShare to kClassMin,
+// where a line is half a pass.  Phi and DPhi assembled with `small` 64 / 128 /
+// 384: 1280-triangle sphere FP64 (sum / 3200 = 21) 0.80 0.94 / 0.84 1.00 / 1.10
+// 1.42 ms; 5120-triangle ellipsoid over a plane, FP32 (86) 2.65 5.02 / 2.62
+// 4.99 / 2.73 5.25 ms; 20480-triangle sphere FP64 (781) 6.3 8.0 / 5.8 7.4 / 5.1
+// 6.6 ms.
+struct AcaBounds {
+    int64_t small, huge, wide;
+};
+AcaBounds aca_bounds(const bem_ctx* c, int prec, int64_t sum)
 {
     const int pi = prec == BEM_PREC_FP32 ? 1 : 0;
+    AcaBounds b{c->cls_small[pi], c->cls_huge[pi], wide_bound(sum)};
+    if (b.small < 0) b.small = std::min(kSmallBlock[pi], std::max(kClassMin, sum / kClassShare));
+    return b;
+}
+
+// ACA class of a block: 0, 1, 2 the workgroup classes (largest first), 3 wide
+int aca_class(const bemsetup::Block& B, const AcaBounds& bd)
+{
     const int64_t s2 = B.rows + B.cols;
-    return s2 > wide ? 3 : s2 > c->cls_huge[pi] ? 0 : s2 > c->cls_small[pi] ? 1 : 2;
+    return s2 > bd.wide ? 3 : s2 > bd.huge ? 0 : s2 > bd.small ? 1 : 2;
 }
 
 // First-pass rank capacities of the listed blocks (largest first): kCapFirst,
@@ -4575,7 +4601,7 @@ size_t aca_shm_bytes(int cap, size_t esz)
 // the results array, and the kernel arguments (blist = the ordered list)
 int aca_prepare(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_t seed,
                 const std::vector<int32_t>& list, const std::vector<int32_t>& cap, const int64_t* d_pivoff,
-                const int32_t* d_piv, int64_t wide, AcaScratch& S, AcaArgs& a, std::vector<int32_t> (&cls)[4],
+                const int32_t* d_piv, const AcaBounds& bd, AcaScratch& S, AcaArgs& a, std::vector<int32_t> (&cls)[4],
                 size_t& shm, const PartView* pv = nullptr)
 {
     const std::vector<bemsetup::Block>& blocks = pv ? *pv->blocks : c->blocks;
@@ -4588,7 +4614,7 @@ int aca_prepare(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uin
         const auto& B = blocks[b];
         S.uoff[b] = tu; S.voff[b] = tv; S.aoff[b] = ta;
         tu += B.rows * cap[b]; tv += B.cols * cap[b]; ta += cap[b];
-        if (B.rows + B.cols <= wide) maxcap = std::max(maxcap, cap[b]);
+        if (B.rows + B.cols <= bd.wide) maxcap = std::max(maxcap, cap[b]);
     }
     int rc;
     const size_t esz = prec == BEM_PREC_FP32 ? sizeof(bem_c32) : sizeof(bem_c64);
@@ -4599,16 +4625,14 @@ int aca_prepare(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uin
     if ((rc = dalloc_bytes(c, &S.A, ta * esz))) return rc;
     S.owned.push_back(S.A);
     S.tu = tu; S.tv = tv; S.ta = ta;
-    // size classes: m + n <= kSmallBlock one wavefront, <= kHugeBlock
-    // kMidThreads, larger kHugeThreads (measured: with several lanes sharing
-    // the chip, smaller workgroups than one block's pivot chain alone would
-    // want give the higher rate), above `wide` ([3]) several workgroups
-    // per block.  The two multi-wavefront classes and the wide blocks run on
-    // streams of their own so that their pivot chains overlap the small
-    // blocks (and the caller's dense tiles); within each class the largest
-    // blocks start first.
+    // size classes (aca_bounds).  The middle class has a stream of its own,
+    // the wide blocks, or without them the largest class, another, so that
+    // their pivot chains overlap the small blocks (and the caller's dense
+    // tiles); within each class the largest blocks start first.  (Both
+    // multi-wavefront classes on one stream, one after the other: Phi and DPhi
+    // of the 20480-triangle sphere in FP32 5.3 and 7.5 ms, now 3.2 and 4.4.)
     for (auto& v : cls) v.clear();
-    for (int32_t b : list) cls[aca_class(c, blocks[b], prec, wide)].push_back(b);
+    for (int32_t b : list) cls[aca_class(blocks[b], bd)].push_back(b);
     std::vector<int32_t> ordered;
     for (int q = 0; q < 3; q++) ordered.insert(ordered.end(), cls[q].begin(), cls[q].end());
     // offsets, capacities and the block list in one upload; ranks, flags and
@@ -4680,8 +4704,8 @@ int run_aca(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_
     std::vector<int32_t> cls[4];
     size_t shm = 0;
     int rc;
-    const int64_t wide = wide_bound(wide_sum(pv ? *pv->blocks : c->blocks, list));
-    if ((rc = aca_prepare(c, kind, prec, tol, maxrank, seed, list, cap, d_pivoff, d_piv, wide, S, a, cls, shm, pv)))
+    const AcaBounds bd = aca_bounds(c, prec, wide_sum(pv ? *pv->blocks : c->blocks, list));
+    if ((rc = aca_prepare(c, kind, prec, tol, maxrank, seed, list, cap, d_pivoff, d_piv, bd, S, a, cls, shm, pv)))
         return rc;
     const bool x = kind == BEM_KIND_DPHI, f32 = prec == BEM_PREC_FP32;
     std::vector<WideSrc> ws;
@@ -4700,7 +4724,7 @@ int run_aca(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_
         off += cls[q].size();
         if (q == 2 && (rc = main_work())) return rc;   // e.g. the dense tiles, overlapping the large classes
         if (cls[q].empty()) continue;
-        hipStream_t st = q < 2 ? c->side[1] : c->stream;
+        hipStream_t st = q == 2 ? c->stream : c->side[q == 1 || R.nrt];
         Timer t(c, 2, st);
         if (f32) launch_aca<bem_c32>(q, x, (unsigned)cls[q].size(), shm, st, aq);
         else launch_aca<bem_c64>(q, x, (unsigned)cls[q].size(), shm, st, aq);
@@ -4887,12 +4911,12 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
     std::vector<int64_t> uoff(nb, 0), voff(nb, 0), aoff(nb, 0);
     int64_t tu = 0, tv = 0, ta = 0;
     int maxcap = 1;
-    const int64_t wide = wide_bound(nf * wide_sum(c->blocks, list));
+    const AcaBounds bd = aca_bounds(c, prec, nf * wide_sum(c->blocks, list));
     for (int32_t b : list) {
         const auto& B = c->blocks[b];
         uoff[b] = tu; voff[b] = tv; aoff[b] = ta;
         tu += B.rows * cap[b]; tv += B.cols * cap[b]; ta += cap[b];
-        if (B.rows + B.cols <= wide) maxcap = std::max(maxcap, cap[b]);
+        if (B.rows + B.cols <= bd.wide) maxcap = std::max(maxcap, cap[b]);
     }
     std::vector<uint64_t> Up(nf), Vp(nf), Ap(nf), Sp(nf);
     std::vector<double> kf(nf);
@@ -4917,7 +4941,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
     }
     const int pi = prec == BEM_PREC_FP32 ? 1 : 0;
     std::vector<int32_t> cls[4];
-    for (int32_t b : list) cls[aca_class(c, c->blocks[b], prec, wide)].push_back(b);
+    for (int32_t b : list) cls[aca_class(c->blocks[b], bd)].push_back(b);
     std::vector<int32_t> items;
     size_t ncls[3];
     for (int q = 0; q < 3; q++) {
@@ -4984,7 +5008,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
         off += ncls[q];
         if (q == 2 && (rc = main_work())) return rc;
         if (!ncls[q]) continue;
-        hipStream_t st = q < 2 ? c->side[1] : c->stream;
+        hipStream_t st = q == 2 ? c->stream : c->side[q == 1 || R.nrt];
         unsigned grid = (unsigned)ncls[q];
         if (useq) {
             aq.queue = d_queue + q;
@@ -5497,9 +5521,9 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
     };
     int rc;
     size_t shm = 0;
-    int64_t wide = 0;
-    for (int64_t q = 0; q < nctx; q++) wide += wide_sum(ctxs[q]->blocks, ctxs[q]->adm_list);
-    wide = wide_bound(wide);
+    int64_t sum = 0;
+    for (int64_t q = 0; q < nctx; q++) sum += wide_sum(ctxs[q]->blocks, ctxs[q]->adm_list);
+    const AcaBounds bd = aca_bounds(lead, precision, sum);   // every context classifies by the lead's schedule
     for (int64_t q = 0; q < nctx; q++) {   // per context: near field, singular table, ACA scratch
         bem_ctx* c = ctxs[q];
         drop_kept(c);
@@ -5554,19 +5578,13 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
         }
         const int64_t nb = (int64_t)c->blocks.size();
         caps[q].assign(nb, 0);
-        first_caps(c->blocks, c->adm_list, wide, maxrank, caps[q]);
-        // every context classifies its blocks by the lead's schedule
-        const int64_t keep_s = c->cls_small[pi], keep_h = c->cls_huge[pi];
-        c->cls_small[pi] = lead->cls_small[pi];
-        c->cls_huge[pi] = lead->cls_huge[pi];
+        first_caps(c->blocks, c->adm_list, bd.wide, maxrank, caps[q]);
         size_t shm_q = 0;
         std::vector<int32_t> cq[4];
         c->sing_cur = c->d_sing;
-        rc = aca_prepare(c, kind, precision, tol, maxrank, seed, c->adm_list, caps[q], d_pivoff, d_piv, wide, S1[q], A[q],
+        rc = aca_prepare(c, kind, precision, tol, maxrank, seed, c->adm_list, caps[q], d_pivoff, d_piv, bd, S1[q], A[q],
                          cq, shm_q);
         c->sing_cur = nullptr;
-        c->cls_small[pi] = keep_s;
-        c->cls_huge[pi] = keep_h;
         if (rc) return fail(rc);
         for (int k = 0; k < 4; k++) cls[q][k] = std::move(cq[k]);
         shm = std::max(shm, shm_q);
@@ -5627,7 +5645,7 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
         aq.blist = d_items + off;
         off += ncls[k];
         if (!ncls[k]) continue;
-        hipStream_t st = k < 2 ? lead->side[1] : lead->stream;
+        hipStream_t st = k == 2 ? lead->stream : lead->side[k == 1 || R.nrt];
         unsigned grid = (unsigned)ncls[k];
         if (lead->aca_queue) {
             aq.queue = d_queue + k;

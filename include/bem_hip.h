@@ -159,7 +159,8 @@ int bem_hmat_destroy(bem_hmat_t h);
    precision (one wavefront up to small_bound, the middle workgroup shape
    up to huge_bound, the largest above; the few blocks, above 1024 to 4096
    depending on the launch's total, that would outlast all others run over
-   several workgroups whatever the bounds) and, for queue >= 0, whether batched
+   several workgroups whatever the bounds; until it is called, small_bound
+   depends on the launch's total too) and, for queue >= 0, whether batched
    ACA launches run as persistent workgroups that take items from a device
    counter (1) or one workgroup per item (0).  Results do not depend on it. */
 int bem_assemble_batch(bem_ctx_t ctx, int kind, int64_t nf, const double* kcc3, double aca_tol, int64_t max_rank,

@@ -5,7 +5,7 @@ bit-identical to each other in both precisions."""
 import numpy as np
 import pytest
 
-from helpers import upload_problem
+from helpers import sphere_problem, upload_problem
 
 pytestmark = pytest.mark.gpu
 WIDE = 1024
@@ -85,3 +85,26 @@ def test_wide_launch_forms_agree(bem, O, meshes):
                 single.close()
     ctx.close()
     ctx2.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("level", [1, 2, 3])
+def test_class_bounds_keep_factors(bem, O, meshes, level, prec):
+    """The bounds that depend on the launch's total (no schedule set) give the
+    factors of the fixed schedules, to the bit: small bound at, below and
+    above the blocks' extents, the largest class empty and not."""
+    P = sphere_problem(O, meshes, level=level, leaf=12, eta=2.0, freq=400.0)
+    adm = [b for b in range(len(P.blocks)) if P.blocks[b][4]]
+    ctx = upload_problem(bem, P)
+    for kind in (0, 1):
+        ref = ctx.assemble(kind, 1e-6, 0, precision=prec, seed=5)
+        other = upload_problem(bem, P)
+        for small, huge in ((0, 0), (64, 96), (384, 2048)):
+            other.set_aca_schedule(prec, small, huge)
+            G = other.assemble(kind, 1e-6, 0, precision=prec, seed=5)
+            for b in adm:
+                assert all(same(x, y) for x, y in zip(G.block(b), ref.block(b))), (kind, small, huge, b)
+            G.close()
+        ref.close()
+        other.close()
+    ctx.close()
