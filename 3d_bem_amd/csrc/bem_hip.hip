@@ -3308,7 +3308,7 @@ struct bem_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     hipStream_t side[2] = {nullptr, nullptr};   // concurrent ACA launches (default priority)
-    hipEvent_t ev_fork = nullptr, ev_join[2] = {nullptr, nullptr};
+    hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
     std::string err;
     // mesh
     int64_t n = 0;
@@ -3432,10 +3432,13 @@ struct bem_ctx {
     int64_t cls_small[2] = {-1, -1};
     int64_t cls_huge[2] = {kHugeBlock[0], kHugeBlock[1]};
     bool aca_queue = false;
-    // wide ACA: "a block still works" flags of the last two bursts (pinned
-    // host memory; [2] takes the other steps' stores) and their events
+    // wide ACA, per operator run at the same time: "a block still works" flags
+    // of the last two bursts (pinned host memory; [2] of four takes the other
+    // steps' stores) and their events; the second operator's stream (created
+    // by the first call that needs it)
     int32_t* wide_active = nullptr;
-    hipEvent_t wide_ev[2] = {nullptr, nullptr};
+    hipEvent_t wide_ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    hipStream_t wide2 = nullptr;
     bool capturing = false;   // Timer records no events while a graph is captured
     hipEvent_t gm_ev[2] = {nullptr, nullptr};
 };
@@ -3520,6 +3523,7 @@ void resolve_pending(bem_ctx* c)
     if (c->pending.empty()) return;
     (void)hipStreamSynchronize(c->stream);
     for (hipStream_t t : c->side) (void)hipStreamSynchronize(t);
+    if (c->wide2) (void)hipStreamSynchronize(c->wide2);
     for (auto& p : c->pending) {
         float ms = 0;
         if (hipEventElapsedTime(&ms, p.e0, p.e1) == hipSuccess) {
@@ -3823,11 +3827,14 @@ int bem_create(bem_ctx_t* out, int device)
         hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_join[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_join[1], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->ev_join[2], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->stage_done, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->gm_ev[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->wide_ev[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->wide_ev[1], hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc((void**)&c->wide_active, 4 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&c->wide_ev[2], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->wide_ev[3], hipEventDisableTiming) != hipSuccess ||
+        hipHostMalloc((void**)&c->wide_active, 8 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->gm_ev[1], hipEventDisableTiming) != hipSuccess ||
         hipHostMalloc((void**)&c->gm_res, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&c->gm_resq, 2 * kArnMax * sizeof(double), hipHostMallocDefault) != hipSuccess ||
@@ -3859,6 +3866,7 @@ int bem_destroy(bem_ctx_t c)
     resolve_pending(c);
     for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
     for (hipStream_t t : c->side) { (void)hipStreamSynchronize(t); (void)hipStreamDestroy(t); }
+    if (c->wide2) { (void)hipStreamSynchronize(c->wide2); (void)hipStreamDestroy(c->wide2); }
     (void)hipEventDestroy(c->ev_fork);
     for (hipEvent_t e : c->ev_join) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->gm_ev) (void)hipEventDestroy(e);
@@ -4553,40 +4561,61 @@ void wide_step_any(const WideRun& R, const AcaArgs& a, bool extra, int odd, int3
     }
 }
 
-// The wide ACA on stream st, the whole loop: bursts of kWideBurst steps, one
-// burst in flight ahead of the check whether a block still worked at the last
-// step of the one before (launches past the end return at once).
+// The wide ACA of one or two operators, each on its stream, the whole loop:
+// bursts of kWideBurst steps, one burst in flight ahead of the check whether a
+// block still worked at the last step of the one before (launches past the end
+// return at once).
 constexpr int kWideBurst = 4;
-int wide_run(bem_ctx* c, const WideRun& R, const AcaArgs& a, bool extra, bool f32, hipStream_t st)
+struct WideLoop {
+    const WideRun* R;
+    const AcaArgs* a;
+    bool extra;
+    hipStream_t st;
+};
+int wide_run(bem_ctx* c, const WideLoop* L, int nl, bool f32)
 {
-    if (!R.nrt) return BEM_OK;
-    Timer t(c, 2, st);
     auto run = [&]() -> int {
-        auto burst = [&](int64_t q) -> int {
-            c->wide_active[q & 1] = 0;
+        bool live[2] = {false, false};
+        for (int o = 0; o < nl; o++) live[o] = L[o].R->nrt > 0;
+        auto burst = [&](int o, int64_t q) -> int {
+            int32_t* flags = c->wide_active + 4 * o;
+            flags[q & 1] = 0;
             for (int u = 0; u < kWideBurst; u++) {
-                int32_t* act = c->wide_active + (u == kWideBurst - 1 ? q & 1 : 2);
-                if (f32) wide_step_any<bem_c32>(R, a, extra, u & 1, act, st);
-                else wide_step_any<bem_c64>(R, a, extra, u & 1, act, st);
+                int32_t* act = flags + (u == kWideBurst - 1 ? q & 1 : 2);
+                if (f32) wide_step_any<bem_c32>(*L[o].R, *L[o].a, L[o].extra, u & 1, act, L[o].st);
+                else wide_step_any<bem_c64>(*L[o].R, *L[o].a, L[o].extra, u & 1, act, L[o].st);
             }
             int rc = launch_check(c, "k_wide_row / k_wide_col");
             if (rc) return rc;
-            HIPC(c, hipEventRecord(c->wide_ev[q & 1], st));
+            HIPC(c, hipEventRecord(c->wide_ev[2 * o + (q & 1)], L[o].st));
             return BEM_OK;
         };
         static_assert(kWideBurst % 2 == 0, "the step parity runs on across bursts");
         int rc;
-        if ((rc = burst(0))) return rc;
-        for (int64_t q = 1;; q++) {
-            if ((rc = burst(q))) return rc;
-            HIPC(c, hipEventSynchronize(c->wide_ev[(q - 1) & 1]));
-            if (!((volatile int32_t*)c->wide_active)[(q - 1) & 1]) return BEM_OK;
-            if (q * kWideBurst > R.max_steps) return set_err(c, BEM_ERR_STATE, "wide ACA: no end");
+        for (int64_t q = 0; live[0] || live[1]; q++) {
+            for (int o = 0; o < nl; o++)
+                if (live[o] && (rc = burst(o, q))) return rc;
+            if (q == 0) continue;
+            for (int o = 0; o < nl; o++) {
+                if (!live[o]) continue;
+                HIPC(c, hipEventSynchronize(c->wide_ev[2 * o + ((q - 1) & 1)]));
+                live[o] = ((volatile int32_t*)c->wide_active)[4 * o + ((q - 1) & 1)] != 0;
+                if (q * kWideBurst > L[o].R->max_steps) return set_err(c, BEM_ERR_STATE, "wide ACA: no end");
+            }
         }
+        return BEM_OK;
     };
+    if (!L[0].R->nrt && (nl < 2 || !L[1].R->nrt)) return BEM_OK;
+    Timer t(c, 2, L[0].st);
     const int rc = run();
-    if (rc) (void)hipStreamSynchronize(st);   // nothing runs on when the caller gives the buffers back
+    if (rc)
+        for (int o = 0; o < nl; o++) (void)hipStreamSynchronize(L[o].st);   // nothing runs on when the caller gives the buffers back
     return rc;
+}
+int wide_run(bem_ctx* c, const WideRun& R, const AcaArgs& a, bool extra, bool f32, hipStream_t st)
+{
+    const WideLoop l{&R, &a, extra, st};
+    return wide_run(c, &l, 1, f32);
 }
 
 // dynamic LDS of aca_block for rank capacity cap and storage size esz
@@ -4693,49 +4722,87 @@ int aca_collect(bem_ctx* c, const AcaScratch& S, int64_t nb, std::vector<int32_t
     return BEM_OK;
 }
 
+// One operator of a run_aca: its kind and pivot lists, and where the results go
+struct AcaOp {
+    int kind;
+    const int64_t* d_pivoff;
+    const int32_t* d_piv;
+    AcaScratch* S;
+    std::vector<int32_t> *rank, *flag;
+    std::vector<int64_t>* ev;
+};
+
+// ACA of the listed blocks for one operator, or for Phi and DPhi of the same
+// blocks at once: their launches share the class streams, and the wide blocks
+// of the second have a stream of their own, so that the two chains of
+// dependent launches run side by side (field of 20011 points through the
+// H-matrix of 5120 triangles, 48 steps each: 12.0 ms one after the other, 11.5 so).
+int run_aca_ops(bem_ctx* c, const AcaOp* ops, int nop, int prec, double tol, int64_t maxrank, uint64_t seed,
+                const std::vector<int32_t>& list, const std::vector<int32_t>& cap,
+                const std::function<int()>& main_work, const PartView* pv)
+{
+    const int64_t nb = (int64_t)(pv ? pv->blocks->size() : c->blocks.size());
+    AcaArgs a[2];
+    std::vector<int32_t> cls[2][4];
+    size_t shm[2] = {0, 0};
+    WideRun R[2];
+    const bool f32 = prec == BEM_PREC_FP32;
+    int rc;
+    const AcaBounds bd = aca_bounds(c, prec, wide_sum(pv ? *pv->blocks : c->blocks, list));
+    for (int o = 0; o < nop; o++) {
+        AcaScratch& S = *ops[o].S;
+        if ((rc = aca_prepare(c, ops[o].kind, prec, tol, maxrank, seed, list, cap, ops[o].d_pivoff, ops[o].d_piv, bd, S,
+                              a[o], cls[o], shm[o], pv)))
+            return rc;
+        std::vector<WideSrc> ws;
+        for (int32_t b : cls[o][3]) {
+            const auto& B = pv ? (*pv->blocks)[b] : c->blocks[b];
+            ws.push_back(WideSrc{b, cap[b], B, S.uoff[b], S.voff[b], S.aoff[b], !pv && c->h_bnear[b] != 0});
+        }
+        if ((rc = wide_prepare(c, ws, f32 ? sizeof(bem_c32) : sizeof(bem_c64), &S.owned, R[o]))) return rc;
+    }
+    const bool second = nop > 1 && R[1].nrt;
+    if (second && !c->wide2) HIPC(c, hipStreamCreateWithFlags(&c->wide2, hipStreamNonBlocking));
+    HIPC(c, hipEventRecord(c->ev_fork, c->stream));
+    for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
+    if (second) HIPC(c, hipStreamWaitEvent(c->wide2, c->ev_fork, 0));
+    size_t off = 0;
+    for (int q = 0; q < 3; q++) {
+        const size_t count = cls[0][q].size();   // the same blocks for both operators
+        if (q == 2 && (rc = main_work())) return rc;   // e.g. the dense tiles, overlapping the large classes
+        for (int o = 0; o < nop && count; o++) {
+            AcaArgs aq = a[o];
+            aq.blist = ops[o].S->d_list + off;
+            hipStream_t st = q == 2 ? c->stream : c->side[q == 1 || R[0].nrt];
+            const bool x = ops[o].kind == BEM_KIND_DPHI;
+            Timer t(c, 2, st);
+            if (f32) launch_aca<bem_c32>(q, x, (unsigned)count, shm[o], st, aq);
+            else launch_aca<bem_c64>(q, x, (unsigned)count, shm[o], st, aq);
+            if ((rc = launch_check(c, "k_aca"))) return rc;
+        }
+        off += count;
+    }
+    const WideLoop L[2] = {{&R[0], &a[0], ops[0].kind == BEM_KIND_DPHI, c->side[0]},
+                           {&R[1], &a[1], nop > 1 && ops[1].kind == BEM_KIND_DPHI, c->wide2}};
+    if ((rc = wide_run(c, L, nop, f32))) return rc;
+    for (int q = 0; q < 2 + second; q++) {
+        hipStream_t st = q < 2 ? c->side[q] : c->wide2;
+        HIPC(c, hipEventRecord(c->ev_join[q], st));
+        HIPC(c, hipStreamWaitEvent(c->stream, c->ev_join[q], 0));
+    }
+    for (int o = 0; o < nop; o++)
+        if ((rc = aca_collect(c, *ops[o].S, nb, *ops[o].rank, *ops[o].flag, *ops[o].ev))) return rc;
+    return BEM_OK;
+}
+
 int run_aca(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, uint64_t seed, const std::vector<int32_t>& list,
             const std::vector<int32_t>& cap, const int64_t* d_pivoff, const int32_t* d_piv,
             const std::function<int()>& main_work, AcaScratch& S,
             std::vector<int32_t>& rank, std::vector<int32_t>& flag, std::vector<int64_t>& ev,
             const PartView* pv = nullptr)
 {
-    const int64_t nb = (int64_t)(pv ? pv->blocks->size() : c->blocks.size());
-    AcaArgs a;
-    std::vector<int32_t> cls[4];
-    size_t shm = 0;
-    int rc;
-    const AcaBounds bd = aca_bounds(c, prec, wide_sum(pv ? *pv->blocks : c->blocks, list));
-    if ((rc = aca_prepare(c, kind, prec, tol, maxrank, seed, list, cap, d_pivoff, d_piv, bd, S, a, cls, shm, pv)))
-        return rc;
-    const bool x = kind == BEM_KIND_DPHI, f32 = prec == BEM_PREC_FP32;
-    std::vector<WideSrc> ws;
-    for (int32_t b : cls[3]) {
-        const auto& B = pv ? (*pv->blocks)[b] : c->blocks[b];
-        ws.push_back(WideSrc{b, cap[b], B, S.uoff[b], S.voff[b], S.aoff[b], !pv && c->h_bnear[b] != 0});
-    }
-    WideRun R;
-    if ((rc = wide_prepare(c, ws, f32 ? sizeof(bem_c32) : sizeof(bem_c64), &S.owned, R))) return rc;
-    HIPC(c, hipEventRecord(c->ev_fork, c->stream));
-    for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
-    size_t off = 0;
-    for (int q = 0; q < 3; q++) {
-        AcaArgs aq = a;
-        aq.blist = S.d_list + off;
-        off += cls[q].size();
-        if (q == 2 && (rc = main_work())) return rc;   // e.g. the dense tiles, overlapping the large classes
-        if (cls[q].empty()) continue;
-        hipStream_t st = q == 2 ? c->stream : c->side[q == 1 || R.nrt];
-        Timer t(c, 2, st);
-        if (f32) launch_aca<bem_c32>(q, x, (unsigned)cls[q].size(), shm, st, aq);
-        else launch_aca<bem_c64>(q, x, (unsigned)cls[q].size(), shm, st, aq);
-        if ((rc = launch_check(c, "k_aca"))) return rc;
-    }
-    if ((rc = wide_run(c, R, a, x, f32, c->side[0]))) return rc;
-    for (int q = 0; q < 2; q++) {
-        HIPC(c, hipEventRecord(c->ev_join[q], c->side[q]));
-        HIPC(c, hipStreamWaitEvent(c->stream, c->ev_join[q], 0));
-    }
-    return aca_collect(c, S, nb, rank, flag, ev);
+    const AcaOp op{kind, d_pivoff, d_piv, &S, &rank, &flag, &ev};
+    return run_aca_ops(c, &op, 1, prec, tol, maxrank, seed, list, cap, main_work, pv);
 }
 
 // Packs the ACA results of h's assembly (first pass S1, re-run of the
@@ -7425,15 +7492,20 @@ int bem_field_hmat(bem_ctx_t c, int64_t nobs, const double* obs3, int64_t nblock
     std::vector<int64_t> evs[2];
     int64_t evaluated = 0;
     int maxr = 0;
-    for (int kind = 0; kind < 2; kind++) {
-        std::vector<int32_t> cap((size_t)nblocks, 0), flag, rank2, flag2;
-        std::vector<int64_t> evs2;
+    std::vector<int32_t> flags[2];
+    if (!adm.empty()) {
+        std::vector<int32_t> cap((size_t)nblocks, 0);
         first_caps(blocks, adm, wide_bound(wide_sum(blocks, adm)), maxrank, cap);
-        if (adm.empty()) break;
-        if ((rc = run_aca(c, kind, BEM_PREC_FP64, tol, maxrank, seed, adm, cap, kind ? d_pivoff : nullptr,
-                          kind ? d_piv : nullptr, [] { return BEM_OK; }, S[kind][0], rank[kind], flag, evs[kind],
-                          &pv)))
+        const AcaOp ops[2] = {{0, nullptr, nullptr, &S[0][0], &rank[0], &flags[0], &evs[0]},
+                              {1, d_pivoff, d_piv, &S[1][0], &rank[1], &flags[1], &evs[1]}};
+        if ((rc = run_aca_ops(c, ops, 2, BEM_PREC_FP64, tol, maxrank, seed, adm, cap, [] { return BEM_OK; }, &pv)))
             return fail(rc);
+    }
+    for (int kind = 0; kind < 2; kind++) {
+        std::vector<int32_t> rank2, flag2;
+        std::vector<int64_t> evs2;
+        if (adm.empty()) break;
+        const std::vector<int32_t>& flag = flags[kind];
         std::vector<int32_t> over;
         for (int32_t b : adm) {
             if (flag[b] == 2) return fail(set_err(c, BEM_ERR_NAN, "bem_field_hmat: non-finite ACA value"));
@@ -7465,7 +7537,11 @@ int bem_field_hmat(bem_ctx_t c, int64_t nobs, const double* obs3, int64_t nblock
     // per 64 x 64 tile; each row sums its partials in partition order
     std::vector<FieldLR> lr;
     std::vector<FieldTile> tiles;
-    std::vector<std::vector<int64_t>> cover((size_t)nobs);
+    // rows of a block or tile and their first partial (the rows' lists are
+    // counted and filled from these: 11.5 -> 7.5 ms of a call at 20011 points,
+    // against a growing vector per point)
+    struct Piece { int64_t row0, rows, part; };
+    std::vector<Piece> cover;
     int64_t ptot = 0, maxr2 = 1;
     for (int64_t b = 0; b < nblocks; b++) {
         const auto& B = blocks[b];
@@ -7490,7 +7566,7 @@ int bem_field_hmat(bem_ctx_t c, int64_t nobs, const double* obs3, int64_t nblock
             L.part = ptot;
             maxr2 = std::max<int64_t>(maxr2, (int64_t)r[0] + r[1]);
             lr.push_back(L);
-            for (int64_t i = 0; i < B.rows; i++) cover[B.row0 + i].push_back(ptot + i);
+            cover.push_back(Piece{B.row0, B.rows, ptot});
             ptot += B.rows;
             continue;
         }
@@ -7499,16 +7575,19 @@ int bem_field_hmat(bem_ctx_t c, int64_t nobs, const double* obs3, int64_t nblock
             for (int64_t c0 = 0; c0 < B.cols; c0 += kTile) {
                 const int32_t cc = (int32_t)std::min<int64_t>(kTile, B.cols - c0);
                 tiles.push_back(FieldTile{B.row0 + r0, B.col0 + c0, ptot, rr, cc});
-                for (int64_t i = 0; i < rr; i++) cover[B.row0 + r0 + i].push_back(ptot + i);
+                cover.push_back(Piece{B.row0 + r0, rr, ptot});
                 ptot += rr;
             }
         }
     }
     // (a row's partials: tiles of one dense block in column order, blocks in partition order)
-    std::vector<int64_t> gptr((size_t)nobs + 1, 0), gidx;
-    for (int64_t i = 0; i < nobs; i++) gptr[i + 1] = gptr[i] + (int64_t)cover[i].size();
-    gidx.reserve(gptr[nobs]);
-    for (auto& v : cover) gidx.insert(gidx.end(), v.begin(), v.end());
+    std::vector<int64_t> gptr((size_t)nobs + 1, 0), gidx((size_t)ptot);
+    for (const Piece& q : cover)
+        for (int64_t i = 0; i < q.rows; i++) gptr[q.row0 + i + 1]++;
+    for (int64_t i = 0; i < nobs; i++) gptr[i + 1] += gptr[i];
+    std::vector<int64_t> at(gptr.begin(), gptr.end() - 1);
+    for (const Piece& q : cover)
+        for (int64_t i = 0; i < q.rows; i++) gidx[at[q.row0 + i]++] = q.part + i;
     FieldLR* d_lr = nullptr;
     FieldTile* d_tiles = nullptr;
     int64_t *d_gptr, *d_gidx;

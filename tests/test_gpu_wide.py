@@ -108,3 +108,32 @@ def test_class_bounds_keep_factors(bem, O, meshes, level, prec):
         ref.close()
         other.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("far,near,tol,maxrank", [(1500, 500, 1e-5, 0), (4000, 300, 1e-8, 0), (1500, 500, 1e-5, 3),
+                                                  (300, 900, 1e-5, 0)])
+def test_field_chains_side_by_side(bem, O, meshes, far, near, tol, maxrank):
+    """Both field operators' wide blocks at once, against the restatement (its
+    ranks and counts; 1e-12 for products summed in another order) and, to the
+    bit, against a repeated call."""
+    P = sphere_problem(O, meshes, level=4, leaf=32, eta=2.0, freq=700.0)
+    ctx = upload_problem(bem, P)
+    rng = np.random.default_rng(3)
+    phi, dphi = (rng.standard_normal(P.n) + 1j * rng.standard_normal(P.n) for _ in range(2))
+    d = rng.standard_normal((near, 3))
+    obs = np.concatenate([rng.uniform(0.9, 2.0, near)[:, None] * d / np.linalg.norm(d, axis=1)[:, None],
+                          rng.uniform(-1, 1, (far, 3)) + [0, 0, 6.0]])   # a far cluster: a large admissible block
+    perm, b5 = P.field_partition(obs, leaf=50, eta=3.0)
+    mn = (b5[:, 1] + b5[:, 3])[b5[:, 4] != 0]
+    print("field points", len(obs), "largest", mn.max(), flush=True)
+    assert mn.max() > WIDE and mn.sum() < 800 * WIDE
+    runs = [ctx.field_hmat(obs[perm], b5, ctx.array(phi), ctx.array(dphi), tol, maxrank=maxrank, seed=7)
+            for _ in range(2)]
+    got = np.empty_like(runs[0][0])
+    got[perm] = runs[0][0]
+    ref, (nadm, maxr, ev) = P.field_hmat(obs, phi, dphi, tol, maxrank=maxrank, seed=7, leaf=50, eta=3.0)
+    st = runs[0][1]
+    assert int(st[1]) == nadm and int(st[2]) == maxr and int(st[3]) == ev, (st, nadm, maxr, ev)
+    assert np.linalg.norm(got - ref) < 1e-12 * np.linalg.norm(ref)
+    assert same(runs[0][0], runs[1][0])
+    ctx.close()
