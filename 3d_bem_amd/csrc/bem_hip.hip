@@ -849,56 +849,65 @@ __device__ __forceinline__ double wave_sum_spread(const double (&x)[NV], int lan
     return cur[0];
 }
 
-// tasks over vector v (length len) against basis W (stride len): k = 0 is
-// |v|^2 into out[base], k >= 1 is v^H W_{k-1} into out[base + 2k].  The
-// group's loads of one element are issued together, unconditionally: a task
-// without a basis vector (k = 0, or k >= ntask) reads v itself and discards
-// the value, so that no load sits behind a branch and the group pays one
-// memory latency per element instead of one per task.
+// G tasks, from kb on, over vector v (length len) against basis W (stride
+// len): task k = 0 is |v|^2 into out[base], k >= 1 is v^H W_{k-1} into
+// out[base + 2k].  One wavefront, the canonical order of every task: lane l
+// takes the elements l, l + 64, ... in ascending order, then the pairwise tree
+// over the lanes.  The group's loads of one element are issued together,
+// unconditionally: a task without a basis vector (k = 0, or k >= ntask) reads v
+// itself and discards the value, so that no load sits behind a branch and the
+// group pays one memory latency per element instead of one per task.
+template <int G, class C>
+__device__ __forceinline__ void dot_group(const C* __restrict__ v, const C* __restrict__ W, int64_t len, int ntask,
+                                          int kb, bem_c64* out, int base)
+{
+    const int lane = threadIdx.x & 63;
+    const C* src[G];
+    bem_c64 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const int k = kb + g;
+        src[g] = (k >= 1 && k < ntask) ? W + (int64_t)(k - 1) * len : v;
+        acc[g] = c64(0, 0);
+    }
+    // branch-free: every task accumulates (the products of tasks without
+    // a basis vector are never written out) and |v|^2 is accumulated
+    // beside them, taking task 0's place in the first group
+    double nrm = 0.0;
+    for (int64_t t = lane; t < len; t += 64) {
+        const bem_c64 cv = ldg64(v + t);
+        C wv[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) wv[g] = ldg(src[g] + t);
+        nrm = nrm + c64_abs2(cv);
+#pragma unroll
+        for (int g = 0; g < G; g++) acc[g] = c64_fma(c64_conj(cv), ld64(&wv[g]), acc[g]);
+    }
+    if (kb == 0) acc[0] = c64(nrm, 0.0);
+    double x[2 * G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        x[2 * g] = acc[g].re;
+        x[2 * g + 1] = acc[g].im;
+    }
+    const double tot = wave_sum_spread<2 * G>(x, lane);
+    constexpr int kStride = 64 / (2 * G);
+    if ((lane & (kStride - 1)) == 0) {
+        const int q = lane / kStride, k = kb + (q >> 1);
+        if (k < ntask) {
+            double* o = (double*)(out + (k == 0 ? base : base + 2 * k));
+            o[q & 1] = tot;
+        }
+    }
+}
+
+// all ntask tasks, dealt to the workgroup's wavefronts
 template <int NT, class C>
 __device__ __forceinline__ void dot_group_pass(const C* __restrict__ v, const C* __restrict__ W, int64_t len,
                                                int ntask, bem_c64* out, int base)
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int kb = w * kDotGroup; kb < ntask; kb += (NT / 64) * kDotGroup) {
-        const C* src[kDotGroup];
-        bem_c64 acc[kDotGroup];
-#pragma unroll
-        for (int g = 0; g < kDotGroup; g++) {
-            const int k = kb + g;
-            src[g] = (k >= 1 && k < ntask) ? W + (int64_t)(k - 1) * len : v;
-            acc[g] = c64(0, 0);
-        }
-        // branch-free: every task accumulates (the products of tasks without
-        // a basis vector are never written out) and |v|^2 is accumulated
-        // beside them, taking task 0's place in the first group
-        double nrm = 0.0;
-        for (int64_t t = lane; t < len; t += 64) {
-            const bem_c64 cv = ldg64(v + t);
-            C wv[kDotGroup];
-#pragma unroll
-            for (int g = 0; g < kDotGroup; g++) wv[g] = ldg(src[g] + t);
-            nrm = nrm + c64_abs2(cv);
-#pragma unroll
-            for (int g = 0; g < kDotGroup; g++) acc[g] = c64_fma(c64_conj(cv), ld64(&wv[g]), acc[g]);
-        }
-        if (kb == 0) acc[0] = c64(nrm, 0.0);
-        double x[2 * kDotGroup];
-#pragma unroll
-        for (int g = 0; g < kDotGroup; g++) {
-            x[2 * g] = acc[g].re;
-            x[2 * g + 1] = acc[g].im;
-        }
-        const double tot = wave_sum_spread<2 * kDotGroup>(x, lane);
-        constexpr int kStride = 64 / (2 * kDotGroup);
-        if ((lane & (kStride - 1)) == 0) {
-            const int v = lane / kStride, k = kb + (v >> 1);
-            if (k < ntask) {
-                double* o = (double*)(out + (k == 0 ? base : base + 2 * k));
-                o[v & 1] = tot;
-            }
-        }
-    }
+    for (int kb = (threadIdx.x >> 6) * kDotGroup; kb < ntask; kb += (NT / 64) * kDotGroup)
+        dot_group<kDotGroup>(v, W, len, ntask, kb, out, base);
 }
 
 // sdots[0] |row|^2, [1] |col|^2, [2 + 2l] row^H V_l, [3 + 2l] col^H U_l (l < r)
@@ -1365,16 +1374,17 @@ __global__ __launch_bounds__(NT, (PLANE && kAcaWaves<NT, C> > 3 ? 3 : kAcaWaves<
 // step evaluates (m + n) / NT entries per thread one after the other while
 // the rest of the chip is idle (the 76440-triangle capsule's ten largest
 // blocks, m + n up to 39000: 287 ms per pass, and a second pass for those
-// above the first rank capacity).  Here a step is two launches over all large
-// blocks at once, a workgroup per kWideChunk entries of a row (k_wide_row)
-// or column (k_wide_col): the entries, the chunk's part of the argmax and of
-// the norm-estimate dot products.  The next launch's workgroups combine the
-// parts, each for itself and in one fixed order, and take the decisions of
-// aca_block (the same pivots, factors, ranks and counts); the kernel
-// boundary is the only barrier.  States are double buffered: a launch reads
-// one copy and its first workgroup of the block writes the other.
+// above the first rank capacity).  Here a step is three launches over all large
+// blocks at once: a workgroup per kWideChunk entries of a row (k_wide_row) and
+// of a column (k_wide_col), the entries and the chunk's part of the argmax,
+// then a wavefront per dot product of the norm estimate (k_wide_dots).  The
+// dot products are whole and in the order of aca_block, so that a block has
+// the same pivots, factors, rank and count whichever of the two forms a launch
+// gives it (the bound between them depends on the launch's total).  The next
+// row launch's workgroups take the decisions of aca_block, each for itself; the
+// kernel boundary is the only barrier.  States are double buffered: a launch
+// reads one copy and its first workgroup of the block writes the other.
 constexpr int kWideChunk = 256;   // entries (and threads) per workgroup
-constexpr int kWideDots = 4;      // dot products per wavefront at a time
 enum WidePhase : int32_t {
     kWideStart,      // nothing computed yet
     kWideProbe,      // EXTRA: the inner loop ended, the next listed pivot comes
@@ -1396,7 +1406,7 @@ struct WideBlk {
     int64_t row0, rows, col0, cols, uoff, voff, aoff;   // the block's, so that one load has them
     int64_t nearb;         // 0: no self or near-singular pair in the block
     int64_t am_col, am_row;   // the chunks' argmax parts
-    int64_t d_col, d_row[2];  // the chunks' dot-product parts, cap + 1 each (rows: of even and odd steps)
+    int64_t dots;             // the step's 2 (cap + 1) dot products, in the places of aca_dots
 };
 struct WideTask { int32_t w, chunk; };
 struct WideArgs {
@@ -1407,7 +1417,6 @@ struct WideArgs {
     ArgMax* am;
     bem_c64* dots;
     int32_t* active;       // host memory: set when a block still works
-    int odd;               // step parity: a row launch writes d_row[odd] and reads the other
 };
 
 // the best of `cnt` argmax parts (every thread gets it); better() keeps the
@@ -1421,124 +1430,38 @@ __device__ __forceinline__ ArgMax wide_best(const ArgMax* part, int cnt, ArgMax*
 
 // One chunk of a residual row (ROW: entries (gi, c0 + t), basis V of stride
 // n) or column: the entries minus the cross approximation with the weights
-// sw[0 .. r), into dst, the chunk's argmax (index excl counts as 0) into *am
-// and, with DOTS, |v|^2 and v^H W_l (l < r) into dots[0 .. r].
+// sw[0 .. r), into dst, and the chunk's argmax (index excl counts as 0) into
+// *am.
 template <bool ROW, class C, bool PLANE, bool FIELD>
 __device__ __forceinline__ void wide_line(const AcaArgs& a, int64_t r0, int64_t c0, int64_t len, int r, int64_t fixed,
                                           const C* W, C* dst, const C* sw, bool nearb, int64_t t0, int64_t excl,
-                                          bool want_dots, C* sv, ArgMax* sred, ArgMax* am, bem_c64* dots)
+                                          ArgMax* sred, ArgMax* am)
 {
-    const int tid = threadIdx.x;
-    const int64_t t = t0 + tid;
-    const int cnt = (int)(len - t0 < kWideChunk ? len - t0 : kWideChunk);
+    const int64_t t = t0 + threadIdx.x;
     const int64_t gf = (ROW ? r0 : c0) + fixed;
-    C v = cx_zero<C>();
-    if (tid < cnt) {
-        const int64_t gi = ROW ? gf : r0 + t, gj = ROW ? c0 + t : gf;
-        const C e = entry_any<PLANE, C, FIELD>(a, gi, gj, nearb);
-        v = cx_sub(e, cross_sum<ROW>(sw, W, len, t, r));
-        dst[t] = v;
-    }
-    sv[tid] = v;
     double best = -1.0;
     int at = kNoIndex;
-    if (tid < cnt) {
+    if (t < len) {
+        const int64_t gi = ROW ? gf : r0 + t, gj = ROW ? c0 + t : gf;
+        const C e = entry_any<PLANE, C, FIELD>(a, gi, gj, nearb);
+        const C v = cx_sub(e, cross_sum<ROW>(sw, W, len, t, r));
+        dst[t] = v;
         const double x = t == excl ? 0.0 : cx_abs2(v);
         if (x > best) { best = x; at = (int)t; }
     }
-    const ArgMax q = group_best<kWideChunk>(best, at, sred);   // (its barriers also publish sv)
-    if (tid == 0) *am = q;
-    if (!want_dots) return;
-    const int lane = tid & 63;
-    for (int kb = (tid >> 6) * kWideDots; kb <= r; kb += (kWideChunk / 64) * kWideDots) {
-        const C* src[kWideDots];
-        bem_c64 acc[kWideDots];
-#pragma unroll
-        for (int g = 0; g < kWideDots; g++) {
-            const int k = kb + g;
-            src[g] = (k >= 1 && k <= r) ? W + (int64_t)(k - 1) * len + t0 : dst + t0;
-            acc[g] = c64(0, 0);
-        }
-        double nrm = 0.0;
-#pragma unroll
-        for (int q = 0; q < kWideChunk / 64; q++) {
-            const int u = lane + 64 * q;
-            if (u >= cnt) break;
-            const bem_c64 cv = ld64(&sv[u]);
-            C wv[kWideDots];
-#pragma unroll
-            for (int g = 0; g < kWideDots; g++) wv[g] = ldg(src[g] + u);
-            nrm = nrm + c64_abs2(cv);
-#pragma unroll
-            for (int g = 0; g < kWideDots; g++) acc[g] = c64_fma(c64_conj(cv), ld64(&wv[g]), acc[g]);
-        }
-        if (kb == 0) acc[0] = c64(nrm, 0.0);
-        double x[2 * kWideDots];
-#pragma unroll
-        for (int g = 0; g < kWideDots; g++) {
-            x[2 * g] = acc[g].re;
-            x[2 * g + 1] = acc[g].im;
-        }
-        const double tot = wave_sum_spread<2 * kWideDots>(x, lane);
-        constexpr int kStride = 64 / (2 * kWideDots);
-        if ((lane & (kStride - 1)) == 0) {
-            const int q = lane / kStride, k = kb + (q >> 1);
-            if (k <= r) ((double*)(dots + k))[q & 1] = tot;
-        }
-    }
-}
-
-// Totals of the chunks' dot-product parts (chunks of stride cap + 1), r + 1
-// values of the column's and the row's into `col` and `row` (LDS).  The
-// chunks are dealt to groups of threads, a thread per value in each, so that
-// the loads run side by side (one thread per value took 8 us of a step at 35
-// chunks); the groups' sums are added in group order.  `red`: two doubles per
-// thread.  A barrier is left to the caller.
-__device__ __forceinline__ void wide_totals(const bem_c64* pc, int nc, const bem_c64* pr, int nr, int cap, int r,
-                                            double* red, bem_c64* col, bem_c64* row)
-{
-    const int nv = 2 * (r + 1), tid = threadIdx.x;
-    const int64_t ld = 2 * (int64_t)(cap + 1);
-    if (nv > kWideChunk) {
-        for (int k = tid; k < nv; k += kWideChunk) {
-            double x = 0.0, y = 0.0;
-            for (int q = 0; q < nc; q++) x = x + ((const double*)pc)[q * ld + k];
-            for (int q = 0; q < nr; q++) y = y + ((const double*)pr)[q * ld + k];
-            ((double*)col)[k] = x;
-            ((double*)row)[k] = y;
-        }
-        return;
-    }
-    const int lg = 32 - __builtin_clz(nv - 1);   // values rounded up to a power of two
-    const int k = tid & ((1 << lg) - 1), g = tid >> lg, ng = kWideChunk >> lg;
-    double x = 0.0, y = 0.0;
-    if (k < nv) {
-#pragma unroll 4
-        for (int q = g; q < nc; q += ng) x = x + ((const double*)pc)[q * ld + k];
-#pragma unroll 4
-        for (int q = g; q < nr; q += ng) y = y + ((const double*)pr)[q * ld + k];
-    }
-    red[tid] = x;
-    red[kWideChunk + tid] = y;
-    __syncthreads();
-    for (int t = tid; t < 2 * nv; t += kWideChunk) {
-        const int side = t >= nv, v = side ? t - nv : t;
-        double z = red[side * kWideChunk + v];
-        for (int q = 1; q < ng; q++) z = z + red[side * kWideChunk + (q << lg) + v];
-        ((double*)(side ? row : col))[v] = z;
-    }
+    const ArgMax q = group_best<kWideChunk>(best, at, sred);
+    if (threadIdx.x == 0) *am = q;
 }
 
 // The decisions between a step's column and the next row (norm update,
 // stopping rules, the next row pivot or, EXTRA, the next listed pivot), then
-// a chunk of that row.  Dynamic LDS: sw[cap] (C), then 2 (cap + 1) totals.
+// a chunk of that row.  Dynamic LDS: sw[cap] (C), then 2 (cap + 1) dot
+// products.
 template <bool EXTRA, class C, bool PLANE, int MODE, bool FIELD>
 __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
 {
     extern __shared__ __attribute__((aligned(16))) char dyn[];
     __shared__ ArgMax sred[kWideChunk / 64];
-    __shared__ C sv[kWideChunk];
-    __shared__ double red[2 * kWideChunk];
     const WideTask T = w.task[blockIdx.x];
     const WideBlk B = w.blk[T.w];
     WideState s = w.in[T.w];
@@ -1559,24 +1482,16 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
     C* V = (C*)a.V + B.voff;
     const C* A = (const C*)a.A + B.aoff;
     C* sw = (C*)dyn;
-    bem_c64* tot = (bem_c64*)(dyn + (((size_t)cap * sizeof(C) + 15) & ~(size_t)15));
+    bem_c64* sdots = (bem_c64*)(dyn + (((size_t)cap * sizeof(C) + 15) & ~(size_t)15));
     const double tiny2 = kTiny * kTiny, tol2 = a.tol * a.tol;
     bool probe = false;
     if (s.phase == kWideStep) {
         const int r = s.r;
-        bem_c64 *dc = tot, *dr = tot + cap + 1;
         const C alpha = ldg(A + r);
-        wide_totals(w.dots + B.d_col, B.nmc, w.dots + (w.odd ? B.d_row[0] : B.d_row[1]), B.nnc, cap, r, red, dc, dr);
-        __syncthreads();
-        // aca_update_norm: the terms in parallel, added in rank order
-        const double gain = (cx_abs2(alpha) * dr[0].re) * dc[0].re;
-        const bem_c64 ca2 = c64_scale(c64_conj(ld64(&alpha)), 2.0);
-        for (int l = tid; l < r; l += kWideChunk)
-            dr[1 + l] = c64_mul(c64_mul(c64_mul(ca2, ldg64(A + l)), dc[1 + l]), dr[1 + l]);
+        for (int k = tid; k < 2 * (r + 1); k += kWideChunk) sdots[k] = ldg64(w.dots + B.dots + k);
         __syncthreads();
         const bem_c64 oldS = s.S;
-        s.S.re = s.S.re + gain;
-        for (int l = 0; l < r; l++) s.S = c64_add(s.S, dr[1 + l]);
+        const double gain = aca_update_norm<kWideChunk>(alpha, A, r, sdots, s.S);
         s.r++;
         if (!isfinite(gain)) {
             s.flag = 2;
@@ -1658,18 +1573,16 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_row(AcaArgs a0, WideArgs w)
     for (int l = tid; l < s.r; l += kWideChunk) sw[l] = cx_mul(ldg(U + (int64_t)l * m + s.i), ldg(A + l));
     __syncthreads();
     wide_line<true, C, PLANE, FIELD>(a, r0, c0, n, s.r, s.i, V, V + (int64_t)s.r * n, sw, nearb,
-                                     (int64_t)T.chunk * kWideChunk, -1, true, sv, sred, w.am + B.am_row + T.chunk,
-                                     w.dots + (w.odd ? B.d_row[1] : B.d_row[0]) + (int64_t)T.chunk * (cap + 1));
+                                     (int64_t)T.chunk * kWideChunk, -1, sred, w.am + B.am_row + T.chunk);
 }
 
 // The column pivot from the row's parts, then a chunk of that column (or of
-// a first column).  Dynamic LDS as k_wide_row.
+// a first column).  Dynamic LDS: sw[cap].
 template <bool EXTRA, class C, bool PLANE, int MODE, bool FIELD>
 __global__ __launch_bounds__(kWideChunk) void k_wide_col(AcaArgs a0, WideArgs w)
 {
     extern __shared__ __attribute__((aligned(16))) char dyn[];
     __shared__ ArgMax sred[kWideChunk / 64];
-    __shared__ C sv[kWideChunk];
     const WideTask T = w.task[blockIdx.x];
     const WideBlk B = w.blk[T.w];
     WideState s = w.in[T.w];
@@ -1720,8 +1633,65 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_col(AcaArgs a0, WideArgs w)
     for (int l = tid; l < r; l += kWideChunk) sw[l] = cx_mul(ldg(A + l), ldg(V + (int64_t)l * n + s.j));
     __syncthreads();
     wide_line<false, C, PLANE, FIELD>(a, r0, c0, m, r, s.j, U, U + (int64_t)r * m, sw, nearb,
-                                      (int64_t)T.chunk * kWideChunk, step ? s.i : -1, step, sv, sred,
-                                      w.am + B.am_col + T.chunk, w.dots + B.d_col + (int64_t)T.chunk * (cap + 1));
+                                      (int64_t)T.chunk * kWideChunk, step ? s.i : -1, sred, w.am + B.am_col + T.chunk);
+}
+
+// The dot products of a step's row and column for the norm estimate, a
+// wavefront each (workgroup (x, y): block x, product y), in the order of
+// dot_group.  A lane's sum is one chain over its elements: kWideAhead of them
+// are loaded together, and a workgroup is one wavefront so that the few long
+// products of the late steps have a compute unit each.  Steps of the
+// 76440-triangle capsule: 50 us while its 204 wide blocks are at work (the
+// factors read once at 5 TB/s), 20 us at the end (590 elements a lane; 47 us
+// with four products in a workgroup and the two kinds of product selected per
+// element).  Solves 27.2 and 115.9 ms at 17892 and 76440 triangles; 27.9 and
+// 114.4 ms when the row and column launches added them in 256-entry parts,
+// another order than aca_block's.
+constexpr int kWideAhead = 16;
+template <bool NORM, class C>
+__device__ __forceinline__ bem_c64 wide_dot(const C* v, const C* x, int len)
+{
+    const int lane = threadIdx.x;
+    bem_c64 acc = c64(0, 0);
+    auto batch = [&](int t0, auto full) {   // elements t0, t0 + 64, ... of the lane
+        constexpr bool FULL = decltype(full)::value;
+        C cv[kWideAhead], xv[kWideAhead];
+#pragma unroll
+        for (int u = 0; u < kWideAhead; u++) {
+            const int t = FULL ? t0 + 64 * u : min(t0 + 64 * u, len - 1);
+            cv[u] = ldg(v + t);
+            if (!NORM) xv[u] = ldg(x + t);
+        }
+#pragma unroll
+        for (int u = 0; u < kWideAhead; u++) {
+            if (!FULL && t0 + 64 * u >= len) continue;
+            if (NORM) acc.re = acc.re + c64_abs2(ld64(&cv[u]));
+            else acc = c64_fma(c64_conj(ld64(&cv[u])), ld64(&xv[u]), acc);
+        }
+    };
+    int t0 = 0;
+    for (; t0 + 64 * kWideAhead <= len; t0 += 64 * kWideAhead) batch(t0 + lane, std::true_type());
+    if (t0 < len) batch(t0 + lane, std::false_type());
+    return acc;
+}
+template <class C, int MODE>
+__global__ __launch_bounds__(64) void k_wide_dots(AcaArgs a0, WideArgs w)
+{
+    const WideState& s = w.in[blockIdx.x];
+    const int k = blockIdx.y, r = s.r;
+    if (s.phase != kWideStep || k >= 2 * (r + 1)) return;
+    const WideBlk B = w.blk[blockIdx.x];
+    AcaArgs a = a0;
+    aca_resolve<MODE>(a, a0, B.item);
+    // [0] |row|^2, [1] |col|^2, [2 + 2l] row^H V_l, [3 + 2l] col^H U_l
+    const bool col = k & 1;
+    const int len = (int)(col ? B.rows : B.cols), lane = threadIdx.x;
+    const C* W = col ? (const C*)a.U + B.uoff : (const C*)a.V + B.voff;
+    const C* v = W + (int64_t)r * len;
+    const bem_c64 acc = k < 2 ? wide_dot<true>(v, v, len) : wide_dot<false>(v, W + (int64_t)((k >> 1) - 1) * len, len);
+    const double sums[2] = {acc.re, acc.im};
+    const double tot = wave_sum_spread<2>(sums, lane);
+    if ((lane & 31) == 0) ((double*)(w.dots + B.dots + k))[lane >> 5] = tot;
 }
 
 // copy the first rank columns/rows of the ACA scratch into the packed
@@ -4371,7 +4341,7 @@ struct PartView {
 // workgroups of 256 threads are resident) is still at work, alone on its
 // compute unit, when the others have ended; a smaller one is better in one
 // workgroup, which keeps its place while the chip is full (a wide step's
-// workgroups wait for one every time).  Between kWideMin, where a step of two
+// workgroups wait for one every time).  Between kWideMin, where a step of three
 // launches takes as long as one workgroup does, and kWideMax.  Solves with
 // the bound at 1024 / 2048 / 4096: 5120-triangle ellipsoid over a plane (share
 // 345) 18.6 / 25.4 / 38.4 ms, 17892-triangle capsule (2491) 31.0 / 31.6 /
@@ -4460,8 +4430,9 @@ struct WideRun {
     WideArgs w{};
     const WideTask *rtask = nullptr, *ctask = nullptr;
     WideState* state[2] = {nullptr, nullptr};
-    unsigned nrt = 0, nct = 0;
-    size_t shm = 0;
+    unsigned nblk = 0, nrt = 0, nct = 0;
+    int maxcap = 1;
+    size_t shm_row = 0, shm_col = 0;
     int64_t max_steps = 0;
 };
 
@@ -4486,11 +4457,8 @@ int wide_prepare(bem_ctx* c, const std::vector<WideSrc>& src, size_t esz, std::v
         B.am_col = am;
         B.am_row = am + B.nmc;
         am += B.nmc + B.nnc;
-        const int64_t ld = B.cap + 1;
-        B.d_col = d;
-        B.d_row[0] = d + B.nmc * ld;
-        B.d_row[1] = B.d_row[0] + B.nnc * ld;
-        d = B.d_row[1] + B.nnc * ld;
+        B.dots = d;
+        d += 2 * (B.cap + 1);
         for (int32_t k = 0; k < B.nnc; k++) rt.push_back(WideTask{(int32_t)q, k});
         for (int32_t k = 0; k < B.nmc; k++) ct.push_back(WideTask{(int32_t)q, k});
         st[q] = WideState{};
@@ -4508,56 +4476,63 @@ int wide_prepare(bem_ctx* c, const std::vector<WideSrc>& src, size_t esz, std::v
     R.state[1] = pk.ptr<WideState>(k_st2);
     if ((rc = dalloc(c, &R.w.am, (size_t)am, owned))) return rc;
     if ((rc = dalloc(c, &R.w.dots, (size_t)d, owned))) return rc;
+    R.nblk = (unsigned)src.size();
     R.nrt = (unsigned)rt.size();
     R.nct = (unsigned)ct.size();
-    R.shm = (((size_t)maxcap * esz + 15) & ~(size_t)15) + 2 * (size_t)(maxcap + 1) * sizeof(bem_c64);
+    R.maxcap = maxcap;
+    R.shm_col = ((size_t)maxcap * esz + 15) & ~(size_t)15;
+    R.shm_row = R.shm_col + 2 * (size_t)(maxcap + 1) * sizeof(bem_c64);
     // every step adds a rank or moves on in a pivot list (20 groups of pivots
     // at most); the loop ends long before this bound
     R.max_steps = 4 * (int64_t)maxcap + 4096;
     return BEM_OK;
 }
 
-// a row and a column launch of one step
+// the row, column and dot-product launches of step `step` (whose row and
+// column are those of at most `step` + 1 terms)
 template <bool EXTRA, class C, bool PLANE, int MODE, bool FIELD>
-void wide_step(const WideRun& R, const AcaArgs& a, int odd, int32_t* active, hipStream_t st)
+void wide_step(const WideRun& R, const AcaArgs& a, int64_t step, int32_t* active, hipStream_t st)
 {
     WideArgs w = R.w;
-    w.odd = odd;
     w.active = active;
     w.task = R.rtask;
     w.in = R.state[0];
     w.out = R.state[1];
-    hipLaunchKernelGGL((k_wide_row<EXTRA, C, PLANE, MODE, FIELD>), dim3(R.nrt), dim3(kWideChunk), R.shm, st, a, w);
+    hipLaunchKernelGGL((k_wide_row<EXTRA, C, PLANE, MODE, FIELD>), dim3(R.nrt), dim3(kWideChunk), R.shm_row, st, a, w);
     w.task = R.ctask;
     w.in = R.state[1];
     w.out = R.state[0];
-    hipLaunchKernelGGL((k_wide_col<EXTRA, C, PLANE, MODE, FIELD>), dim3(R.nct), dim3(kWideChunk), R.shm, st, a, w);
+    hipLaunchKernelGGL((k_wide_col<EXTRA, C, PLANE, MODE, FIELD>), dim3(R.nct), dim3(kWideChunk), R.shm_col, st, a, w);
+    w.in = R.state[0];
+    w.out = nullptr;
+    const unsigned terms = (unsigned)std::min<int64_t>(step + 1, R.maxcap);
+    hipLaunchKernelGGL((k_wide_dots<C, MODE>), dim3(R.nblk, 2 * terms), dim3(64), 0, st, a, w);
 }
 
 template <class C>
-void wide_step_any(const WideRun& R, const AcaArgs& a, bool extra, int odd, int32_t* active, hipStream_t st)
+void wide_step_any(const WideRun& R, const AcaArgs& a, bool extra, int64_t step, int32_t* active, hipStream_t st)
 {
     if constexpr (sizeof(C) == sizeof(bem_c64)) {
         if (a.obs) {
-            if (extra) wide_step<true, C, false, 0, true>(R, a, odd, active, st);
-            else wide_step<false, C, false, 0, true>(R, a, odd, active, st);
+            if (extra) wide_step<true, C, false, 0, true>(R, a, step, active, st);
+            else wide_step<false, C, false, 0, true>(R, a, step, active, st);
             return;
         }
     }
     const bool plane = a.M.rvtx != nullptr;
     if (a.jobs) {
-        if (extra) wide_step<true, C, false, 3, false>(R, a, odd, active, st);
-        else wide_step<false, C, false, 3, false>(R, a, odd, active, st);
+        if (extra) wide_step<true, C, false, 3, false>(R, a, step, active, st);
+        else wide_step<false, C, false, 3, false>(R, a, step, active, st);
     } else if (a.nf > 0) {
-        if (extra && plane) wide_step<true, C, true, 1, false>(R, a, odd, active, st);
-        else if (extra) wide_step<true, C, false, 1, false>(R, a, odd, active, st);
-        else if (plane) wide_step<false, C, true, 1, false>(R, a, odd, active, st);
-        else wide_step<false, C, false, 1, false>(R, a, odd, active, st);
+        if (extra && plane) wide_step<true, C, true, 1, false>(R, a, step, active, st);
+        else if (extra) wide_step<true, C, false, 1, false>(R, a, step, active, st);
+        else if (plane) wide_step<false, C, true, 1, false>(R, a, step, active, st);
+        else wide_step<false, C, false, 1, false>(R, a, step, active, st);
     } else {
-        if (extra && plane) wide_step<true, C, true, 0, false>(R, a, odd, active, st);
-        else if (extra) wide_step<true, C, false, 0, false>(R, a, odd, active, st);
-        else if (plane) wide_step<false, C, true, 0, false>(R, a, odd, active, st);
-        else wide_step<false, C, false, 0, false>(R, a, odd, active, st);
+        if (extra && plane) wide_step<true, C, true, 0, false>(R, a, step, active, st);
+        else if (extra) wide_step<true, C, false, 0, false>(R, a, step, active, st);
+        else if (plane) wide_step<false, C, true, 0, false>(R, a, step, active, st);
+        else wide_step<false, C, false, 0, false>(R, a, step, active, st);
     }
 }
 
@@ -4582,15 +4557,14 @@ int wide_run(bem_ctx* c, const WideLoop* L, int nl, bool f32)
             flags[q & 1] = 0;
             for (int u = 0; u < kWideBurst; u++) {
                 int32_t* act = flags + (u == kWideBurst - 1 ? q & 1 : 2);
-                if (f32) wide_step_any<bem_c32>(*L[o].R, *L[o].a, L[o].extra, u & 1, act, L[o].st);
-                else wide_step_any<bem_c64>(*L[o].R, *L[o].a, L[o].extra, u & 1, act, L[o].st);
+                if (f32) wide_step_any<bem_c32>(*L[o].R, *L[o].a, L[o].extra, q * kWideBurst + u, act, L[o].st);
+                else wide_step_any<bem_c64>(*L[o].R, *L[o].a, L[o].extra, q * kWideBurst + u, act, L[o].st);
             }
-            int rc = launch_check(c, "k_wide_row / k_wide_col");
+            int rc = launch_check(c, "k_wide_row / k_wide_col / k_wide_dots");
             if (rc) return rc;
             HIPC(c, hipEventRecord(c->wide_ev[2 * o + (q & 1)], L[o].st));
             return BEM_OK;
         };
-        static_assert(kWideBurst % 2 == 0, "the step parity runs on across bursts");
         int rc;
         for (int64_t q = 0; live[0] || live[1]; q++) {
             for (int o = 0; o < nl; o++)

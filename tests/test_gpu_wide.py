@@ -137,3 +137,67 @@ def test_field_chains_side_by_side(bem, O, meshes, far, near, tol, maxrank):
     assert np.linalg.norm(got - ref) < 1e-12 * np.linalg.norm(ref)
     assert same(runs[0][0], runs[1][0])
     ctx.close()
+
+
+def ulps(x):
+    return int(np.float64(x).view(np.int64))
+
+
+def flip_tolerance(rank, lo, hi):
+    """adjacent tolerances t0 < t1 with rank(t0) = rank(lo) > rank(t1), by bisection"""
+    r0, a, b = rank(lo), ulps(lo), ulps(hi)
+    assert rank(hi) < r0
+    while b - a > 1:
+        mid = (a + b) // 2
+        if rank(np.int64(mid).view(np.float64)) < r0:
+            b = mid
+        else:
+            a = mid
+    return float(np.int64(a).view(np.float64)), float(np.int64(b).view(np.float64))
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_stopping_rule_in_every_launch_form(bem, O, meshes, kind):
+    """The bound above which a block runs over several workgroups depends on
+    the launch's total: blocks of m + n from 1024 to 3500 run so in a single
+    assembly and in one workgroup in a batch of 16.  At tolerances where the stopping
+    rule of such a block turns from one representable number to the next, so
+    that the last bit of its norm estimate decides, both forms give the same
+    ranks and evaluation counts, and the restatement's."""
+    P, wide = capsule_problem(O, meshes, 0.055, 800.0, impedance=0.0)
+    nf = 16
+    mn = P.blocks[:, 1] + P.blocks[:, 3]
+    total = int(mn[P.blocks[:, 4] != 0].sum())
+    assert total < 800 * WIDE < nf * total   # one bound at its least, the other above it
+    both = [b for b in wide if mn[b] <= min(4096, nf * total // 800)]
+    ctx = upload_problem(bem, P)
+    prm = P.params()
+    kcc = np.array([[prm["k"], prm["cc"].real, prm["cc"].imag]] * nf)
+
+    def single(tol, b):
+        G = ctx.assemble(kind, tol, seed=5)
+        r = G.rank(b)
+        G.close()
+        return r
+
+    tested = 0
+    for lo in (1e-6, 2e-5):
+        for b in both:
+            if single(1e-3, b) >= single(lo, b):
+                continue
+            for t in flip_tolerance(lambda x: single(x, b), lo, 1e-3):
+                G = ctx.assemble(kind, t, seed=5)
+                batch = ctx.assemble_batch(kind, kcc, t, seed=5)
+                rs = [G.rank(w) for w in wide]
+                rb = [[H.rank(w) for w in wide] for H in batch]
+                ev = [H.stats()["evaluated"] for H in (G, *batch)]
+                for H in (G, *batch):
+                    H.close()
+                print("kind", kind, "block", b, "m+n", mn[b], "tol", t, "ranks", rs, rb[0], ev[:2], flush=True)
+                assert all(r == rs for r in rb) and len(set(ev)) == 1, (b, t)
+                if tested < 2:
+                    H = P.assemble(kind, t, 0, 5)
+                    assert [H.rank(w) for w in wide] == rs and H.evaluated == ev[0], (b, t)
+            tested += 1
+    assert tested >= 8, tested
+    ctx.close()
