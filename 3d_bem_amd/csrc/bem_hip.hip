@@ -40,8 +40,8 @@ constexpr int kCapFirst = 48;   // first-pass ACA rank capacity per block
 constexpr int kCapMax = 1016;   // second-pass capacity limit (FP64 LDS: (4 cap + 2) x 16 B <= 64 KiB)
 // ACA workgroup size classes by m + n, per storage precision [FP64, FP32]:
 // up to kSmallBlock one wavefront, up to kHugeBlock kMidThreads, above
-// kHugeThreads; kSmallBlock lower where a launch's blocks total little
-// (aca_bounds)
+// kHugeThreads.  A one-wavefront bound of kSmallBlock stands for the built-in
+// rule: lower where a launch's blocks total little (aca_bounds)
 constexpr int64_t kSmallBlock[2] = {384, 384};
 constexpr int64_t kHugeBlock[2] = {(int64_t)1 << 40, 2048};
 constexpr int64_t kClassMin = 64, kClassShare = 3200;
@@ -3396,10 +3396,10 @@ struct bem_ctx {
     bool use_mfma = true;
     bool use_graphs = true;
     // ACA size classes by m + n per storage precision [FP64, FP32]: up to
-    // cls_small (negative: by the launch's total, aca_bounds) one wavefront, up
-    // to cls_huge the middle class, above the largest; batched assemblies on
+    // cls_small (kSmallBlock: by the launch's total, aca_bounds) one wavefront,
+    // up to cls_huge the middle class, above the largest; batched assemblies on
     // persistent workgroups (queue counter)
-    int64_t cls_small[2] = {-1, -1};
+    int64_t cls_small[2] = {kSmallBlock[0], kSmallBlock[1]};
     int64_t cls_huge[2] = {kHugeBlock[0], kHugeBlock[1]};
     bool aca_queue = false;
     // wide ACA, per operator run at the same time: "a block still works" flags
@@ -4368,7 +4368,8 @@ int64_t wide_sum(const std::vector<bemsetup::Block>& blocks, const std::vector<i
 // 384: 1280-triangle sphere FP64 (sum / 3200 = 21) 0.80 0.94 / 0.84 1.00 / 1.10
 // 1.42 ms; 5120-triangle ellipsoid over a plane, FP32 (86) 2.65 5.02 / 2.62
 // 4.99 / 2.73 5.25 ms; 20480-triangle sphere FP64 (781) 6.3 8.0 / 5.8 7.4 / 5.1
-// 6.6 ms.
+// 6.6 ms.  The rule is the built-in schedule's, and setting the bound to
+// kSmallBlock returns to it; any other bound set or tuned is taken as it is.
 struct AcaBounds {
     int64_t small, huge, wide;
 };
@@ -4376,7 +4377,7 @@ AcaBounds aca_bounds(const bem_ctx* c, int prec, int64_t sum)
 {
     const int pi = prec == BEM_PREC_FP32 ? 1 : 0;
     AcaBounds b{c->cls_small[pi], c->cls_huge[pi], wide_bound(sum)};
-    if (b.small < 0) b.small = std::min(kSmallBlock[pi], std::max(kClassMin, sum / kClassShare));
+    if (b.small == kSmallBlock[pi]) b.small = std::min(b.small, std::max(kClassMin, sum / kClassShare));
     return b;
 }
 

@@ -159,10 +159,12 @@ int bem_hmat_destroy(bem_hmat_t h);
    precision (one wavefront up to small_bound, the middle workgroup shape
    up to huge_bound, the largest above; the few blocks, above 1024 to 4096
    depending on the launch's total, that would outlast all others run over
-   several workgroups whatever the bounds; until it is called, small_bound
-   depends on the launch's total too) and, for queue >= 0, whether batched
+   several workgroups whatever the bounds) and, for queue >= 0, whether batched
    ACA launches run as persistent workgroups that take items from a device
-   counter (1) or one workgroup per item (0).  Results do not depend on it. */
+   counter (1) or one workgroup per item (0).  The built-in schedule is
+   small_bound 384, huge_bound 2048 (FP32) or 1 << 40 (FP64), queue 0; its
+   small_bound 384 is lowered, to 64 at the least, in launches whose blocks
+   total little, any other is taken as it is.  Results do not depend on it. */
 int bem_assemble_batch(bem_ctx_t ctx, int kind, int64_t nf, const double* kcc3, double aca_tol, int64_t max_rank,
                        int precision, uint64_t seed, bem_hmat_t* outs);
 /* Several meshes at once (no counterpart in the reference, which solves
@@ -181,9 +183,9 @@ int bem_set_aca_schedule(bem_ctx_t ctx, int precision, int64_t small_bound, int6
    tasks go to a thread pool, hmatrix.cpp:793-846): times the assembly of
    `kind` at the nf frequencies kcc3 (bem_assemble for nf = 1,
    bem_assemble_batch otherwise; the fastest of two runs each) under
-   candidate schedules by coordinate descent -- the one-wavefront bound
-   (128, 256, 384, 512), then for FP32 the huge bound (1024, 2048, 4096,
-   none), then for nf > 1 the work queue, a candidate taking over only when
+   candidate schedules by coordinate descent from the built-in one -- the
+   one-wavefront bound (128, 256, 384 as built in, 512), then for FP32 the huge
+   bound (1024, 2048, 4096, none), then for nf > 1 the work queue, a candidate taking over only when
    3 % faster than the current choice -- and keeps the choice on the
    context.  choice3: small bound, huge bound, queue; best_ms: its time.
    Operators kept for near-field pairing are dropped. */

@@ -268,6 +268,42 @@ def test_autotune_keeps_results(bem, O, meshes):
     S.close()
 
 
+def aca_launches(ctx, run):
+    """ACA launches of run() on ctx"""
+    ctx.profile(1)
+    run()
+    return int(ctx.profile(0)[7 + 2])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_builtin_schedule_comes_back(bem, O, meshes, prec):
+    """The built-in schedule lowers the one-wavefront bound 384 in launches
+    whose blocks total little.  Setting it after another schedule returns to
+    that rule: as many ACA launches (one per size class with blocks) as a
+    context that was never set, one more than with every block in the
+    one-wavefront class; and a tuned context whose tuner kept 384 has it too."""
+    P = sphere_problem(O, meshes, level=3, leaf=32, eta=2.0, freq=500.0)
+    mn = P.blocks[P.blocks[:, 4] != 0][:, [1, 3]].sum(axis=1)
+    assert mn.min() <= 64 < mn.max() <= 384   # two classes by the rule, one below 384
+    ctx = upload_problem(bem, P)
+    prm = P.params()
+    kcc = [[prm["k"], prm["cc"].real, prm["cc"].imag]]
+    huge = 2048 if prec == bem.FP32 else 1 << 40
+
+    def count():
+        return aca_launches(ctx, lambda: ctx.assemble(0, 1e-6, precision=prec, seed=3).close())
+
+    assert count() == 2
+    ctx.set_aca_schedule(prec, 512, huge, 0)
+    assert count() == 1
+    ctx.set_aca_schedule(prec, 384, huge, 0)
+    assert count() == 2
+    (small, _, _), _ = ctx.autotune_aca(0, kcc, 1e-6, precision=prec, seed=3)
+    print("tuned small bound", small, flush=True)
+    assert count() == (2 if small in (128, 384) else 1 + int(mn.max() > small))
+    ctx.close()
+
+
 def test_batched_sweep_impedance_ellipsoid(bem, O, meshes):
     """Batched sweep on a non-spherical body with mixed boundary conditions:
     ellipsoid (0.5, 0.3, 0.2) m, 1280 triangles, Z = rho c (1.5 + 0.5i) on a

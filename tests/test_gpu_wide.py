@@ -99,7 +99,7 @@ def test_class_bounds_keep_factors(bem, O, meshes, level, prec):
     for kind in (0, 1):
         ref = ctx.assemble(kind, 1e-6, 0, precision=prec, seed=5)
         other = upload_problem(bem, P)
-        for small, huge in ((0, 0), (64, 96), (384, 2048)):
+        for small, huge in ((0, 0), (64, 96), (384, 2048), (385, 2048)):
             other.set_aca_schedule(prec, small, huge)
             G = other.assemble(kind, 1e-6, 0, precision=prec, seed=5)
             for b in adm:
