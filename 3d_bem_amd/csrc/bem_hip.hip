@@ -42,8 +42,8 @@ constexpr int kCapMax = 1016;   // second-pass capacity limit (FP64 LDS: (4 cap 
 // up to kSmallBlock one wavefront, up to kHugeBlock kMidThreads, above
 // kHugeThreads.  A one-wavefront bound of kSmallBlock stands for the built-in
 // rule: lower where a launch's blocks total little (aca_bounds)
-constexpr int64_t kSmallBlock[2] = {384, 384};
-constexpr int64_t kHugeBlock[2] = {(int64_t)1 << 40, 2048};
+using bemsetup::kHugeBlock;
+using bemsetup::kSmallBlock;
 constexpr int64_t kClassMin = 64, kClassShare = 3200;
 // bounds on the m + n above which a block takes the ACA over several
 // workgroups (wide_bound), and the resident 256-thread workgroups it counts

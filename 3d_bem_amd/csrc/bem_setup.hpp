@@ -9,6 +9,11 @@
 
 namespace bemsetup {
 
+// The built-in ACA schedule's bounds on m + n per storage precision [FP64,
+// FP32] (bem_set_aca_schedule), without its work queue
+constexpr int64_t kSmallBlock[2] = {384, 384};
+constexpr int64_t kHugeBlock[2] = {(int64_t)1 << 40, 2048};
+
 struct Vec3 { double x, y, z; };
 
 // Per-element geometry in one order (cluster order after reordering).

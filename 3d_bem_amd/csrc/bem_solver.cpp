@@ -1008,6 +1008,7 @@ struct bem_solver {
     // the first batched chunk of the first sweep and then used on every lane
     bool autotune = false;
     bool tuned[2] = {false, false};
+    bool scheduled[2] = {false, false};   // the contexts hold a tuned or given schedule
     int64_t schedule[2][3] = {};
     double tunedMs[2] = {0, 0};
 };
@@ -1234,7 +1235,19 @@ int bem_solver_set_autotune(bem_solver_t s, int on)
 {
     if (!s || !s->s) return BEM_ERR_ARG;
     s->autotune = on != 0;
-    if (!on) s->tuned[0] = s->tuned[1] = false;
+    if (on) return BEM_OK;
+    for (int pi = 0; pi < 2; pi++) {   // the contexts back to the built-in schedule
+        s->tuned[pi] = false;
+        if (!s->scheduled[pi]) continue;
+        std::vector<bem_ctx_t> cs{s->s->context()};
+        for (auto& l : s->lanes) cs.push_back(l->context());
+        for (bem_ctx_t c : cs) {
+            const int rc = bem_set_aca_schedule(c, pi ? BEM_PREC_FP32 : BEM_PREC_FP64, bemsetup::kSmallBlock[pi],
+                                                bemsetup::kHugeBlock[pi], 0);
+            if (rc != BEM_OK) return rc;
+        }
+        s->scheduled[pi] = false;
+    }
     return BEM_OK;
 }
 
@@ -1432,13 +1445,14 @@ int bem_solver_sweep(bem_solver_t s, int64_t nf, const double* freqs, double c, 
             P.refine = s->refine;
             std::vector<double> fr(freqs, freqs + std::min(nf, chunk));
             S.tuneAca(fr, s->schedule[pi], &s->tunedMs[pi]);
-            s->tuned[pi] = true;
+            s->tuned[pi] = s->scheduled[pi] = true;
         }
         while ((int)s->lanes.size() < L - 1)
             s->lanes.push_back(std::make_unique<bem::BoundaryElementSolver>(s->device, s->input, s->leaf, s->eta));
         std::vector<bem::BoundaryElementSolver*> solver(L);
         solver[0] = s->s.get();
         for (int q = 1; q < L; q++) solver[q] = s->lanes[q - 1].get();
+        if (s->tuned[pi]) s->scheduled[pi] = true;
         if (s->tuned[pi])
             for (int q = 0; q < L; q++)
                 bem::check(solver[q]->context(),

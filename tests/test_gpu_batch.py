@@ -3,6 +3,8 @@ frequencies from one ACA launch per size class over the flattened
 (frequency, block) list equal the per-frequency assemblies bit for bit, in
 FP64 and FP32, with one workgroup per item and with persistent workgroups on
 a work queue, and under another size-class schedule."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -302,6 +304,34 @@ def test_builtin_schedule_comes_back(bem, O, meshes, prec):
     print("tuned small bound", small, flush=True)
     assert count() == (2 if small in (128, 384) else 1 + int(mn.max() > small))
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_forgotten_schedule_leaves_the_contexts(bem, O, meshes, prec):
+    """set_autotune(False) forgets a schedule: the next sweep on every lane
+    has the ACA launches of a solver that was never given one (two size
+    classes per assembly by the built-in rule, fewer with every block in the
+    one-wavefront class)."""
+    tri = meshes.icosphere(3, 0.5)
+    S = bem.Solver(tri, meshes.robin_bc(len(tri), 0, 1, 1), leaf=32, eta=2.0)
+    S.set_sweep_batch(2)
+
+    def count():
+        prof = np.zeros(14)
+        ptr = prof.ctypes.data_as(ctypes.c_void_p)
+        assert bem.lib().bem_solver_profile(S.h, 1, ptr) == bem.BEM_OK
+        S.sweep(np.array(FREQS), aca_tol=1e-6, gmres_tol=1e-8, precision=prec, lanes=2)
+        assert bem.lib().bem_solver_profile(S.h, 0, ptr) == bem.BEM_OK
+        return int(prof[7 + 2])
+
+    S.sweep(np.array(FREQS), aca_tol=1e-6, gmres_tol=1e-8, precision=prec, lanes=2)   # makes the lanes
+    fresh = count()
+    S.set_aca_schedule(prec, 512, 1 << 40, 0)
+    assert count() < fresh
+    S.set_autotune(False)
+    assert S.aca_schedule(prec) is None
+    assert count() == fresh
+    S.close()
 
 
 def test_batched_sweep_impedance_ellipsoid(bem, O, meshes):
