@@ -3002,6 +3002,9 @@ __global__ void k_mvm_gather_ops(int64_t n, int64_t P, const int64_t* __restrict
 // graph that is captured once and replayed for every j.
 
 constexpr int kArnMax = 8;   // right-hand sides of one lockstep solve
+// a context's pinned host memory (bem_ctx::pinned)
+constexpr size_t kPinnedBytes = 256;
+static_assert((2 + 2 * kArnMax) * sizeof(double) <= kPinnedBytes - 64, "residual estimates before the wide ACA's flags");
 
 // X = column *jp of the bases (the product's input)
 template <int Q>
@@ -3402,10 +3405,14 @@ struct bem_ctx {
     int64_t cls_small[2] = {kSmallBlock[0], kSmallBlock[1]};
     int64_t cls_huge[2] = {kHugeBlock[0], kHugeBlock[1]};
     bool aca_queue = false;
+    // pinned host memory: gm_res, gm_resq and, on a cache line of their own,
+    // the flags of the wide ACA (one allocation: each costs a context 0.2 ms)
+    void* pinned = nullptr;
     // wide ACA, per operator run at the same time: "a block still works" flags
-    // of the last two bursts (pinned host memory; [2] of four takes the other
-    // steps' stores) and their events; the second operator's stream (created
-    // by the first call that needs it)
+    // of the last two bursts ([2] of four takes the other steps' stores) and
+    // their events; the second operator's stream and its join event
+    // (ev_join[2]).  Events and stream are created by the first call that needs
+    // them.
     int32_t* wide_active = nullptr;
     hipEvent_t wide_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     hipStream_t wide2 = nullptr;
@@ -3797,21 +3804,17 @@ int bem_create(bem_ctx_t* out, int device)
         hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_join[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_join[1], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_join[2], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->stage_done, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->gm_ev[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->wide_ev[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->wide_ev[1], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->wide_ev[2], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->wide_ev[3], hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc((void**)&c->wide_active, 8 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->gm_ev[1], hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc((void**)&c->gm_res, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&c->gm_resq, 2 * kArnMax * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&c->pinned, kPinnedBytes, hipHostMallocDefault) != hipSuccess ||
         scratch_address(device, &c->scratch_dev) != hipSuccess) {
         delete c;
         return BEM_ERR_HIP;
     }
+    c->gm_res = (double*)c->pinned;
+    c->gm_resq = c->gm_res + 2;
+    c->wide_active = (int32_t*)((char*)c->pinned + kPinnedBytes - 64);
     *out = c;
     return BEM_OK;
 }
@@ -3838,14 +3841,14 @@ int bem_destroy(bem_ctx_t c)
     for (hipStream_t t : c->side) { (void)hipStreamSynchronize(t); (void)hipStreamDestroy(t); }
     if (c->wide2) { (void)hipStreamSynchronize(c->wide2); (void)hipStreamDestroy(c->wide2); }
     (void)hipEventDestroy(c->ev_fork);
-    for (hipEvent_t e : c->ev_join) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->ev_join)
+        if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->gm_ev) (void)hipEventDestroy(e);
-    for (hipEvent_t e : c->wide_ev) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->wide_ev)
+        if (e) (void)hipEventDestroy(e);
     (void)hipEventDestroy(c->stage_done);
     if (c->stage) (void)hipHostFree(c->stage);
-    if (c->wide_active) (void)hipHostFree(c->wide_active);
-    if (c->gm_res) (void)hipHostFree(c->gm_res);
-    if (c->gm_resq) (void)hipHostFree(c->gm_resq);
+    if (c->pinned) (void)hipHostFree(c->pinned);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return BEM_OK;
@@ -4551,6 +4554,8 @@ struct WideLoop {
 int wide_run(bem_ctx* c, const WideLoop* L, int nl, bool f32)
 {
     auto run = [&]() -> int {
+        for (int e = 0; e < 2 * nl; e++)
+            if (!c->wide_ev[e]) HIPC(c, hipEventCreateWithFlags(&c->wide_ev[e], hipEventDisableTiming));
         bool live[2] = {false, false};
         for (int o = 0; o < nl; o++) live[o] = L[o].R->nrt > 0;
         auto burst = [&](int o, int64_t q) -> int {
@@ -4738,6 +4743,7 @@ int run_aca_ops(bem_ctx* c, const AcaOp* ops, int nop, int prec, double tol, int
     }
     const bool second = nop > 1 && R[1].nrt;
     if (second && !c->wide2) HIPC(c, hipStreamCreateWithFlags(&c->wide2, hipStreamNonBlocking));
+    if (second && !c->ev_join[2]) HIPC(c, hipEventCreateWithFlags(&c->ev_join[2], hipEventDisableTiming));
     HIPC(c, hipEventRecord(c->ev_fork, c->stream));
     for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
     if (second) HIPC(c, hipStreamWaitEvent(c->wide2, c->ev_fork, 0));
