@@ -21,6 +21,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -4586,7 +4587,9 @@ int wide_run(bem_ctx* c, const WideLoop* L, int nl, bool f32)
         return BEM_OK;
     };
     if (!L[0].R->nrt && (nl < 2 || !L[1].R->nrt)) return BEM_OK;
-    Timer t(c, 2, L[0].st);
+    std::optional<Timer> t[2];   // a window per chain
+    for (int o = 0; o < nl; o++)
+        if (L[o].R->nrt) t[o].emplace(c, 2, L[o].st);
     const int rc = run();
     if (rc)
         for (int o = 0; o < nl; o++) (void)hipStreamSynchronize(L[o].st);   // nothing runs on when the caller gives the buffers back

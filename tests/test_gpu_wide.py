@@ -127,8 +127,17 @@ def test_field_chains_side_by_side(bem, O, meshes, far, near, tol, maxrank):
     mn = (b5[:, 1] + b5[:, 3])[b5[:, 4] != 0]
     print("field points", len(obs), "largest", mn.max(), flush=True)
     assert mn.max() > WIDE and mn.sum() < 800 * WIDE
-    runs = [ctx.field_hmat(obs[perm], b5, ctx.array(phi), ctx.array(dphi), tol, maxrank=maxrank, seed=7)
-            for _ in range(2)]
+    x = ctx.array(phi), ctx.array(dphi)
+    ctx.profile(1)
+    runs = [ctx.field_hmat(obs[perm], b5, *x, tol, maxrank=maxrank, seed=7)]
+    # launches of the profile: both operators' size classes (the bounds of an
+    # FP64 launch with this total) and both wide chains, in each pass
+    small = max(64, min(384, mn.sum() // 3200))
+    classes = int((mn <= small).any()) + int(((mn > small) & (mn <= WIDE)).any()) + 1
+    launches = int(ctx.profile(0)[7 + 2])
+    print("size classes", classes, "launches", launches, flush=True)
+    assert launches == 2 * classes or (maxrank == 0 and launches > 2 * classes)
+    runs.append(ctx.field_hmat(obs[perm], b5, *x, tol, maxrank=maxrank, seed=7))
     got = np.empty_like(runs[0][0])
     got[perm] = runs[0][0]
     ref, (nadm, maxr, ev) = P.field_hmat(obs, phi, dphi, tol, maxrank=maxrank, seed=7, leaf=50, eta=3.0)
