@@ -4590,16 +4590,29 @@ int wide_run(bem_ctx* c, const WideLoop* L, int nl, bool f32)
     std::optional<Timer> t[2];   // a window per chain
     for (int o = 0; o < nl; o++)
         if (L[o].R->nrt) t[o].emplace(c, 2, L[o].st);
-    const int rc = run();
-    if (rc)
-        for (int o = 0; o < nl; o++) (void)hipStreamSynchronize(L[o].st);   // nothing runs on when the caller gives the buffers back
-    return rc;
+    return run();
 }
 int wide_run(bem_ctx* c, const WideRun& R, const AcaArgs& a, bool extra, bool f32, hipStream_t st)
 {
     const WideLoop l{&R, &a, extra, st};
     return wide_run(c, &l, 1, f32);
 }
+
+// From the fork of an ACA's streams to their join: a return in between (a failed
+// launch, the caller's work, the step limit) waits for all of them, so that
+// nothing runs on when the caller gives the buffers back to the pool, which
+// hands them to the next call without a wait
+struct AcaStreams {
+    bem_ctx* c;
+    bool joined = false;
+    ~AcaStreams()
+    {
+        if (joined) return;
+        (void)hipStreamSynchronize(c->stream);
+        for (hipStream_t s : c->side) (void)hipStreamSynchronize(s);
+        if (c->wide2) (void)hipStreamSynchronize(c->wide2);
+    }
+};
 
 // dynamic LDS of aca_block for rank capacity cap and storage size esz
 size_t aca_shm_bytes(int cap, size_t esz)
@@ -4747,6 +4760,7 @@ int run_aca_ops(bem_ctx* c, const AcaOp* ops, int nop, int prec, double tol, int
     const bool second = nop > 1 && R[1].nrt;
     if (second && !c->wide2) HIPC(c, hipStreamCreateWithFlags(&c->wide2, hipStreamNonBlocking));
     if (second && !c->ev_join[2]) HIPC(c, hipEventCreateWithFlags(&c->ev_join[2], hipEventDisableTiming));
+    AcaStreams streams{c};
     HIPC(c, hipEventRecord(c->ev_fork, c->stream));
     for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
     if (second) HIPC(c, hipStreamWaitEvent(c->wide2, c->ev_fork, 0));
@@ -4774,6 +4788,7 @@ int run_aca_ops(bem_ctx* c, const AcaOp* ops, int nop, int prec, double tol, int
         HIPC(c, hipEventRecord(c->ev_join[q], st));
         HIPC(c, hipStreamWaitEvent(c->stream, c->ev_join[q], 0));
     }
+    streams.joined = true;
     for (int o = 0; o < nop; o++)
         if ((rc = aca_collect(c, *ops[o].S, nb, *ops[o].rank, *ops[o].flag, *ops[o].ev))) return rc;
     return BEM_OK;
@@ -5046,6 +5061,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
     a.Uf = pk.ptr<void*>(k_up); a.Vf = pk.ptr<void*>(k_vp); a.Af = pk.ptr<void*>(k_ap);
     a.queue = nullptr; a.nitems = 0;
     size_t shm = aca_shm_bytes(maxcap, esz);
+    AcaStreams streams{c};
     HIPC(c, hipEventRecord(c->ev_fork, c->stream));
     for (hipStream_t st : c->side) HIPC(c, hipStreamWaitEvent(st, c->ev_fork, 0));
     size_t off = 0;
@@ -5077,6 +5093,7 @@ int run_aca_batch(bem_ctx* c, int kind, int prec, double tol, int64_t maxrank, u
         HIPC(c, hipEventRecord(c->ev_join[q], c->side[q]));
         HIPC(c, hipStreamWaitEvent(c->stream, c->ev_join[q], 0));
     }
+    streams.joined = true;
     std::vector<char> h((size_t)nf * nb * 16);
     HIPC(c, hipMemcpyAsync(h.data(), res, h.size(), hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
@@ -5686,6 +5703,7 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
                                  S1[q].voff[b], S1[q].aoff[b], ctxs[q]->h_bnear[b] != 0});
     WideRun R;
     if ((rc = wide_prepare(lead, ws, esz, &lead_own, R))) return fail(rc);
+    AcaStreams streams{lead};
     HIPC(lead, hipEventRecord(lead->ev_fork, lead->stream));
     for (hipStream_t st : lead->side) HIPC(lead, hipStreamWaitEvent(st, lead->ev_fork, 0));
     const int nt[3] = {pi ? kHugeThreads<bem_c32> : kHugeThreads<bem_c64>,
@@ -5714,6 +5732,7 @@ int bem_assemble_multi(const bem_ctx_t* ctxs, int64_t nctx, int kind, double tol
         HIPC(lead, hipEventRecord(lead->ev_join[k], lead->side[k]));
         HIPC(lead, hipStreamWaitEvent(lead->stream, lead->ev_join[k], 0));
     }
+    streams.joined = true;
     HIPC(lead, hipStreamSynchronize(lead->stream));
     const double t1 = now_ms();
     // per context: results, re-run of the overflowing blocks, packing
