@@ -8,9 +8,31 @@ meshes are returned as an (n, 9) float64 array of triangle nodes
 (b - a) x (c - a) points into the exterior domain as the reference expects
 (vectortriangle.h:90, global.cpp:903-908).
 """
+import math
+
 import numpy as np
 
 _PHI = (1.0 + 5.0 ** 0.5) / 2.0
+
+
+def _fma(a, b, c):
+    """a b + c rounded once: Dekker's exact product by Veltkamp's splitting,
+    then the correctly rounded sum of its two parts and c"""
+    def split(x):
+        t = 134217729.0 * x
+        hi = t - (t - x)
+        return hi, x - hi
+    p = a * b
+    (ah, al), (bh, bl) = split(a), split(b)
+    return math.fsum((p, ((ah * bh - p) + ah * bl + al * bh) + al * bl, c))
+
+
+def _norm3(p):
+    """|p| with one order of operations on every CPU (numpy's norm takes its
+    dot product from BLAS, whose kernel, and with it the last bit, follows
+    the CPU)"""
+    x, y, z = (float(q) for q in p)
+    return math.sqrt(_fma(z, z, _fma(y, y, x * x)))
 
 
 def _icosahedron():
@@ -37,7 +59,7 @@ def icosphere_vf(level):
             key = (i, j) if i < j else (j, i)
             if key not in cache:
                 p = np.array(vl[i]) + np.array(vl[j])
-                p /= np.linalg.norm(p)
+                p /= _norm3(p)
                 cache[key] = len(vl)
                 vl.append(tuple(p))
             return cache[key]
@@ -163,7 +185,7 @@ def impedance_bc(n, k, fraction, seed, rho_c_ratio=1.5 + 0.5j):
 def unit_direction(seed):
     """Direction uniform on the unit sphere (normalised N(0, I3))."""
     d = np.random.default_rng(seed).standard_normal(3)
-    return d / np.linalg.norm(d)
+    return d / _norm3(d)
 
 
 def write_msh(path, tri, groups=None, names=None, version="4.1"):
