@@ -74,11 +74,10 @@ __global__ void k_quadpoints(int64_t n, const double* __restrict__ nodes, double
     if (j >= n) return;
     const double* v = nodes + 9 * j;
     for (int q = 0; q < 16; q++) {
-        double x1 = kTriX[q][0], x2 = kTriX[q][1];
-        double x3 = (1.0 - x2) - x1;
-        qx[q * n + j] = (x1 * v[0] + x2 * v[3]) + x3 * v[6];
-        qy[q * n + j] = (x1 * v[1] + x2 * v[4]) + x3 * v[7];
-        qz[q * n + j] = (x1 * v[2] + x2 * v[5]) + x3 * v[8];
+        const TriPoint T = kTri16[q];
+        qx[q * n + j] = (T.x1 * v[0] + T.x2 * v[3]) + T.x3 * v[6];
+        qy[q * n + j] = (T.x1 * v[1] + T.x2 * v[4]) + T.x3 * v[7];
+        qz[q * n + j] = (T.x1 * v[2] + T.x2 * v[5]) + T.x3 * v[8];
     }
 }
 
@@ -993,18 +992,9 @@ __device__ __forceinline__ bem_c32f4 ops_of_f32(int need, const DevFreq32& F, co
                                                 const double* edg, const double* qnx, const double* qny,
                                                 const double* qnz)
 {
-    const int64_t n = M.n;
-    const double* g = edg + j;
-    const double dx = M.px[i] - g[0], dy = M.py[i] - g[n], dz = M.pz[i] - g[2 * n];
-    const double ax = g[3 * n], ay = g[4 * n], az = g[5 * n], bx = g[6 * n], by = g[7 * n], bz = g[8 * n];
-    const float npx = (float)M.nx[i], npy = (float)M.ny[i], npz = (float)M.nz[i];
-    const float nqx = (float)qnx[j], nqy = (float)qny[j], nqz = (float)qnz[j];
-    const float area = (float)M.area[j];
-    if (need == 1)
-        return regular_ops_f32_need<1, kQuadUnroll>(F, dx, dy, dz, ax, ay, az, bx, by, bz, npx, npy, npz, nqx, nqy, nqz, area);
-    if (need == 2)
-        return regular_ops_f32_need<2, kQuadUnroll>(F, dx, dy, dz, ax, ay, az, bx, by, bz, npx, npy, npz, nqx, nqy, nqz, area);
-    return regular_ops_f32_need<3, kQuadUnroll>(F, dx, dy, dz, ax, ay, az, bx, by, bz, npx, npy, npz, nqx, nqy, nqz, area);
+    if (need == 1) return pair_ops_f32<1, kQuadUnroll>(F, M, i, j, edg, qnx, qny, qnz);
+    if (need == 2) return pair_ops_f32<2, kQuadUnroll>(F, M, i, j, edg, qnx, qny, qnz);
+    return pair_ops_f32<3, kQuadUnroll>(F, M, i, j, edg, qnx, qny, qnz);
 }
 template <bool PLANE>
 __device__ __forceinline__ bool regular_entry(const AcaArgs& a, int64_t i, int64_t j, bem_c64* e, bool nearb = true)
@@ -4487,8 +4477,10 @@ int wide_prepare(bem_ctx* c, const std::vector<WideSrc>& src, size_t esz, std::v
     R.maxcap = maxcap;
     R.shm_col = ((size_t)maxcap * esz + 15) & ~(size_t)15;
     R.shm_row = R.shm_col + 2 * (size_t)(maxcap + 1) * sizeof(bem_c64);
-    // every step adds a rank or moves on in a pivot list (20 groups of pivots
-    // at most); the loop ends long before this bound
+    // a step adds a rank that stays, or it is one of at most three of a listed
+    // pivot (its first column, a row without a pivot, a rank taken back); a
+    // block has at most 400 listed pivots (20 x 20 orientation groups), so the
+    // loop ends within cap + 1200 steps
     R.max_steps = 4 * (int64_t)maxcap + 4096;
     return BEM_OK;
 }

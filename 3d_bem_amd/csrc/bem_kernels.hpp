@@ -11,19 +11,7 @@ typedef struct { float re, im; } bem_c32;
 
 namespace bemdev {
 
-// order-8 16-point triangle rule weights (trianglequadraturerules.cpp:91-108)
-__constant__ static const double kTriW[16] = {
-    0.14431560767779, 0.09509163426728, 0.09509163426728, 0.09509163426728, 0.10321737053472, 0.10321737053472,
-    0.10321737053472, 0.03245849762320, 0.03245849762320, 0.03245849762320, 0.02723031417443, 0.02723031417443,
-    0.02723031417443, 0.02723031417443, 0.02723031417443, 0.02723031417443};
-// barycentric (xi1, xi2) of the same rule
-__constant__ static const double kTriX[16][2] = {
-    {0.33333333333333, 0.33333333333333}, {0.45929258829272, 0.45929258829272}, {0.45929258829272, 0.08141482341455},
-    {0.08141482341455, 0.45929258829272}, {0.17056930775176, 0.17056930775176}, {0.17056930775176, 0.65886138449648},
-    {0.65886138449648, 0.17056930775176}, {0.05054722831703, 0.05054722831703}, {0.05054722831703, 0.89890554336594},
-    {0.89890554336594, 0.05054722831703}, {0.26311282963464, 0.72849239295540}, {0.72849239295540, 0.00839477740996},
-    {0.00839477740996, 0.26311282963464}, {0.72849239295540, 0.26311282963464}, {0.26311282963464, 0.00839477740996},
-    {0.00839477740996, 0.72849239295540}};
+// order-8 16-point triangle rule (trianglequadraturerules.cpp:91-108):
 // (xi1, xi2, xi3, w) with xi3 = (1 - xi2) - xi1 as the points are formed, and
 // the weight in FP32
 struct TriPoint { double x1, x2, x3, w; float wf, pad; };
@@ -557,12 +545,6 @@ __device__ __forceinline__ void point_accumulate_f32_r(bem_c32f4* acc, const Dev
     }
 }
 
-// order-8 16-point rule weights in FP32
-__constant__ static const float kTriWf[16] = {
-    0.14431560767779f, 0.09509163426728f, 0.09509163426728f, 0.09509163426728f, 0.10321737053472f, 0.10321737053472f,
-    0.10321737053472f, 0.03245849762320f, 0.03245849762320f, 0.03245849762320f, 0.02723031417443f, 0.02723031417443f,
-    0.02723031417443f, 0.02723031417443f, 0.02723031417443f, 0.02723031417443f};
-
 template <int UNROLL = 2>
 __device__ __forceinline__ bem_c32f4 regular_ops_f32(const DevFreq32& F, double px, double py, double pz, float npx,
                                                      float npy, float npz, float nqx, float nqy, float nqz, float area,
@@ -574,40 +556,7 @@ __device__ __forceinline__ bem_c32f4 regular_ops_f32(const DevFreq32& F, double 
 #pragma unroll UNROLL
     for (int q = 0; q < 16; q++)
         point_accumulate_f32(&o, F, px, py, pz, npx, npy, npz, nqx, nqy, nqz, upnq, qx[q * qs], qy[q * qs],
-                             qz[q * qs], kTriWf[q]);
-    o.L = c32(o.L.re * area, o.L.im * area);
-    o.M = c32(o.M.re * area, o.M.im * area);
-    o.Mt = c32(o.Mt.re * area, o.Mt.im * area);
-    o.N = c32(o.N.re * area, o.N.im * area);
-    return o;
-}
-
-// regular_ops_f32 with R = d - xi1 (a - c) - xi2 (b - c), d = p - c: the
-// point q = c + xi1 (a - c) + xi2 (b - c) (the rule's point, rounded
-// differently from the FP64 path's form) at two FP64 fma per coordinate
-template <int UNROLL = 1>
-__device__ __forceinline__ bem_c32f4 regular_ops_f32_edge_of(const DevFreq32& F, const DevMesh& M, int64_t i,
-                                                             int64_t j, const double* edg, const double* qnx,
-                                                             const double* qny, const double* qnz,
-                                                             bool needX = true, bool needY = true)
-{
-    const int64_t n = M.n;
-    const double* g = edg + j;
-    const double dx = M.px[i] - g[0], dy = M.py[i] - g[n], dz = M.pz[i] - g[2 * n];
-    const double ax = g[3 * n], ay = g[4 * n], az = g[5 * n], bx = g[6 * n], by = g[7 * n], bz = g[8 * n];
-    const float npx = (float)M.nx[i], npy = (float)M.ny[i], npz = (float)M.nz[i];
-    const float nqx = (float)qnx[j], nqy = (float)qny[j], nqz = (float)qnz[j];
-    const float upnq = fmaf(npz, nqz, fmaf(npy, nqy, npx * nqx));
-    bem_c32f4 o;
-    o.L = o.M = o.Mt = o.N = c32(0.0f, 0.0f);
-#pragma unroll UNROLL
-    for (int q = 0; q < 16; q++) {
-        const double x1 = kTriX[q][0], x2 = kTriX[q][1];
-        point_accumulate_f32_r(&o, F, fma(-x1, ax, fma(-x2, bx, dx)), fma(-x1, ay, fma(-x2, by, dy)),
-                               fma(-x1, az, fma(-x2, bz, dz)), npx, npy, npz, nqx, nqy, nqz, upnq, kTriWf[q], needX,
-                               needY);
-    }
-    const float area = (float)M.area[j];
+                             qz[q * qs], kTri16[q].wf);
     o.L = c32(o.L.re * area, o.L.im * area);
     o.M = c32(o.M.re * area, o.M.im * area);
     o.Mt = c32(o.Mt.re * area, o.Mt.im * area);
@@ -631,8 +580,10 @@ __device__ __forceinline__ int bc_needs(const int32_t* subst, const C* cd, int k
     return (__any(need & 1) ? 1 : 0) | (__any(need & 2) ? 2 : 0);
 }
 
-// regular_ops_f32_edge_of with the operators that NEED names, for a row point
-// p (normal np) and the column's edge form
+// regular_ops_f32 with only the operators that NEED names and R = d -
+// xi1 (a - c) - xi2 (b - c), d = p - c: the point q = c + xi1 (a - c) +
+// xi2 (b - c) (the rule's point, rounded differently from the FP64 path's
+// form) at two FP64 fma per coordinate
 template <int NEED, int UNROLL>
 __device__ __forceinline__ bem_c32f4 regular_ops_f32_need(const DevFreq32& F, double dx, double dy, double dz,
                                                           double ax, double ay, double az, double bx, double by,
@@ -656,10 +607,26 @@ __device__ __forceinline__ bem_c32f4 regular_ops_f32_need(const DevFreq32& F, do
     return o;
 }
 
+// regular_ops_f32_need of the pair (i, j) with the column's edge form edg and
+// normal qn: the element's (M.edg, M.nx ..) or its mirror image's (M.redg, M.rnx ..)
+template <int NEED, int UNROLL>
+__device__ __forceinline__ bem_c32f4 pair_ops_f32(const DevFreq32& F, const DevMesh& M, int64_t i, int64_t j,
+                                                  const double* edg, const double* qnx, const double* qny,
+                                                  const double* qnz)
+{
+    const int64_t n = M.n;
+    const double* g = edg + j;
+    const double dx = M.px[i] - g[0], dy = M.py[i] - g[n], dz = M.pz[i] - g[2 * n];
+    const double ax = g[3 * n], ay = g[4 * n], az = g[5 * n], bx = g[6 * n], by = g[7 * n], bz = g[8 * n];
+    return regular_ops_f32_need<NEED, UNROLL>(F, dx, dy, dz, ax, ay, az, bx, by, bz, (float)M.nx[i], (float)M.ny[i],
+                                              (float)M.nz[i], (float)qnx[j], (float)qny[j], (float)qnz[j],
+                                              (float)M.area[j]);
+}
+
 // the FP32 form of refl_ops (mirror image of element j, edge form)
 __device__ __forceinline__ bem_c32f4 refl_ops_f32(const DevFreq32& F, const DevMesh& M, int64_t i, int64_t j)
 {
-    return regular_ops_f32_edge_of<1>(F, M, i, j, M.redg, M.rnx, M.rny, M.rnz);
+    return pair_ops_f32<3, 1>(F, M, i, j, M.redg, M.rnx, M.rny, M.rnz);
 }
 
 // off-diagonal Phi / DPhi entry from the FP32 operators (bem_phi_entry,
