@@ -18,20 +18,20 @@ _PHI = (1.0 + 5.0 ** 0.5) / 2.0
 def _fma(a, b, c):
     """a b + c rounded once: Dekker's exact product by Veltkamp's splitting,
     then the correctly rounded sum of its two parts and c"""
-    def split(x):
-        t = 134217729.0 * x
-        hi = t - (t - x)
-        return hi, x - hi
     p = a * b
-    (ah, al), (bh, bl) = split(a), split(b)
+    t = 134217729.0 * a
+    ah = t - (t - a)
+    al = a - ah
+    t = 134217729.0 * b
+    bh = t - (t - b)
+    bl = b - bh
     return math.fsum((p, ((ah * bh - p) + ah * bl + al * bh) + al * bl, c))
 
 
-def _norm3(p):
-    """|p| with one order of operations on every CPU (numpy's norm takes its
-    dot product from BLAS, whose kernel, and with it the last bit, follows
-    the CPU)"""
-    x, y, z = (float(q) for q in p)
+def _norm3(x, y, z):
+    """|(x, y, z)| with one order of operations on every CPU (numpy's norm
+    takes its dot product from BLAS, whose kernel, and with it the last bit,
+    follows the CPU)"""
     return math.sqrt(_fma(z, z, _fma(y, y, x * x)))
 
 
@@ -50,7 +50,7 @@ def _icosahedron():
 def icosphere_vf(level):
     """Unit icosphere vertices/faces after `level` midpoint subdivisions."""
     v, f = _icosahedron()
-    verts = [tuple(x) for x in v]
+    verts = v.tolist()
     for _ in range(level):
         cache = {}
         vl = verts
@@ -58,10 +58,11 @@ def icosphere_vf(level):
         def mid(i, j):
             key = (i, j) if i < j else (j, i)
             if key not in cache:
-                p = np.array(vl[i]) + np.array(vl[j])
-                p /= _norm3(p)
+                (ax, ay, az), (bx, by, bz) = vl[i], vl[j]
+                x, y, z = ax + bx, ay + by, az + bz
+                r = _norm3(x, y, z)
                 cache[key] = len(vl)
-                vl.append(tuple(p))
+                vl.append((x / r, y / r, z / r))
             return cache[key]
 
         nf = []
@@ -185,7 +186,7 @@ def impedance_bc(n, k, fraction, seed, rho_c_ratio=1.5 + 0.5j):
 def unit_direction(seed):
     """Direction uniform on the unit sphere (normalised N(0, I3))."""
     d = np.random.default_rng(seed).standard_normal(3)
-    return d / _norm3(d)
+    return d / _norm3(*d.tolist())
 
 
 def write_msh(path, tri, groups=None, names=None, version="4.1"):
