@@ -324,7 +324,7 @@ def roofline(avg_ms, cnt, st, blocks, n, prec_name, points0, traffic_sched, quad
 
 def measured_traffic(family, prec_name, sched):
     """HBM bytes per launch of a kernel family under one scheduling (sched:
-    e.g. "batch4 s384 h2048 q0") from the committed rocprofv3 FETCH_SIZE /
+    e.g. "batch2 s384 h2048 q0") from the committed rocprofv3 FETCH_SIZE /
     WRITE_SIZE summary (scaled by the copy calibration), or None"""
     key = f"traffic_bytes_per_launch {family} {prec_name} {sched} ="
     path = os.path.join(ROOT, "profiles", f"{family}_{prec_name}_sphere20480_traffic.md")
