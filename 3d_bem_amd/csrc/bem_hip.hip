@@ -4337,9 +4337,11 @@ struct PartView {
 // workgroup, which keeps its place while the chip is full (a wide step's
 // workgroups wait for one every time).  Between kWideMin, where a step of three
 // launches takes as long as one workgroup does, and kWideMax.  Solves with
-// the bound at 1024 / 2048 / 4096: 5120-triangle ellipsoid over a plane (share
-// 345) 18.6 / 25.4 / 38.4 ms, 17892-triangle capsule (2491) 31.0 / 31.6 /
-// 53.9 ms, 20480-triangle sphere in FP64 (3126) 23.0 / 22.4 / 20.7 ms.
+// the bound at 1024 / 2048 / 4096: 17892-triangle capsule (share 2491) 27.7 /
+// 27.4 / 50.2 ms, 20480-triangle sphere in FP64 (3126) 23.2 / 21.7 / 20.3 ms,
+// 76440-triangle capsule (above 4096) 143.6 / 119.4 / 117.0 ms; 5120-triangle
+// ellipsoid over a plane (345; with the dot products in the other two
+// launches) 18.6 / 25.4 / 38.4 ms.
 int64_t wide_bound(int64_t sum)
 {
     return std::min(kWideMax, std::max(kWideMin, sum / kWideShare));
