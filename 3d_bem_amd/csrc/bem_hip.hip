@@ -1630,48 +1630,50 @@ __global__ __launch_bounds__(kWideChunk) void k_wide_col(AcaArgs a0, WideArgs w)
 // The dot products of a step's row and column for the norm estimate, a
 // wavefront each (workgroup (x, y): block x, product y), in the order of
 // dot_group.  A lane's sum is one chain over its elements: kWideAhead of them
-// are loaded together, and a workgroup is one wavefront so that the few long
-// products of the late steps have a compute unit each.  Steps of the
+// (128 bytes; with 256 or 512 the FP64 form needs 160 or 298 registers and
+// waits for room beside the one-workgroup classes) are loaded together, and a
+// workgroup is one wavefront so that the few long products of the late steps
+// have a compute unit each.  Steps of the
 // 76440-triangle capsule: 50 us while its 204 wide blocks are at work (the
 // factors read once at 5 TB/s), 20 us at the end (590 elements a lane; 47 us
 // with four products in a workgroup and the two kinds of product selected per
-// element).  Solves 27.2 and 115.9 ms at 17892 and 76440 triangles; 27.9 and
-// 114.4 ms when the row and column launches added them in 256-entry parts,
+// element).  Solves 27.4 and 116.8 ms at 17892 and 76440 triangles; 28.0 and
+// 114.5 ms when the row and column launches added them in 256-entry parts,
 // another order than aca_block's.
-constexpr int kWideAhead = 16;
+template <class C> constexpr int kWideAhead = 128 / sizeof(C);
 template <bool NORM, class C>
 __device__ __forceinline__ bem_c64 wide_dot(const C* v, const C* x, int len)
 {
+    constexpr int kAhead = kWideAhead<C>;
     const int lane = threadIdx.x;
     bem_c64 acc = c64(0, 0);
     auto batch = [&](int t0, auto full) {   // elements t0, t0 + 64, ... of the lane
         constexpr bool FULL = decltype(full)::value;
-        C cv[kWideAhead], xv[kWideAhead];
+        C cv[kAhead], xv[kAhead];
 #pragma unroll
-        for (int u = 0; u < kWideAhead; u++) {
+        for (int u = 0; u < kAhead; u++) {
             const int t = FULL ? t0 + 64 * u : min(t0 + 64 * u, len - 1);
             cv[u] = ldg(v + t);
             if (!NORM) xv[u] = ldg(x + t);
         }
 #pragma unroll
-        for (int u = 0; u < kWideAhead; u++) {
+        for (int u = 0; u < kAhead; u++) {
             if (!FULL && t0 + 64 * u >= len) continue;
             if (NORM) acc.re = acc.re + c64_abs2(ld64(&cv[u]));
             else acc = c64_fma(c64_conj(ld64(&cv[u])), ld64(&xv[u]), acc);
         }
     };
     int t0 = 0;
-    for (; t0 + 64 * kWideAhead <= len; t0 += 64 * kWideAhead) batch(t0 + lane, std::true_type());
+    for (; t0 + 64 * kAhead <= len; t0 += 64 * kAhead) batch(t0 + lane, std::true_type());
     if (t0 < len) batch(t0 + lane, std::false_type());
     return acc;
 }
 template <class C, int MODE>
 __global__ __launch_bounds__(64) void k_wide_dots(AcaArgs a0, WideArgs w)
 {
-    const WideState& s = w.in[blockIdx.x];
-    const int k = blockIdx.y, r = s.r;
-    if (s.phase != kWideStep || k >= 2 * (r + 1)) return;
     const WideBlk B = w.blk[blockIdx.x];
+    const int k = blockIdx.y, r = w.in[blockIdx.x].r, phase = w.in[blockIdx.x].phase;
+    if (phase != kWideStep || k >= 2 * (r + 1)) return;
     AcaArgs a = a0;
     aca_resolve<MODE>(a, a0, B.item);
     // [0] |row|^2, [1] |col|^2, [2 + 2l] row^H V_l, [3 + 2l] col^H U_l
